@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "forward.hpp"
+#include "gmres.hpp"
 #include "kernels.hpp"
 #include "plan.hpp"
 #include "persample.hpp"
@@ -1148,6 +1149,134 @@ __global__ void k_grhs_full(int m, int n, int64_t Bp, const int32_t* __restrict_
   }
 }
 
+// ---------------------------------------------------------------------------
+// sample-major operands of the per-sample GMRES cycles (gmres.hpp)
+// ---------------------------------------------------------------------------
+
+// A 64 x 64 tile through LDS: rows k0 .. k0 + 63 of a batch-minor array (get(k, b),
+// lanes over samples) to put(k, b, value) with lanes over k.
+template <typename T, typename Get, typename Put>
+__device__ __forceinline__ void minor_to_major_tile(int64_t K, int64_t batch, Get get, Put put) {
+  __shared__ T tile[64][65];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int64_t k0 = (int64_t)blockIdx.x * 64, b0 = (int64_t)blockIdx.y * 64;
+#pragma unroll 4
+  for (int r = ty; r < 64; r += kBlock / 64)
+    tile[r][tx] = k0 + r < K && b0 + tx < batch ? get(k0 + r, b0 + tx) : T(0);
+  __syncthreads();
+#pragma unroll 4
+  for (int r = ty; r < 64; r += kBlock / 64)
+    if (b0 + r < batch && k0 + tx < K) put(k0 + tx, b0 + r, tile[tx][r]);
+}
+
+// The masks and, with steps per element, a, delta and sigma, in position order.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gmr_stage(Adj<T> S, const int32_t* __restrict__ cperm,
+                                                      const int32_t* __restrict__ rperm,
+                                                      int64_t batch, T* mask, T* av, T* dv, T* sv) {
+  const int64_t n = S.n, m = S.m;
+  const int64_t K = S.dg ? 3 * n + 2 * m : n + m;
+  minor_to_major_tile<T>(
+      K, batch,
+      [&](int64_t k, int64_t b) -> T {
+        if (k < n) return S.Cm[(size_t)cperm[k] * S.Bp + b];
+        if (k < n + m) return S.Dm[(size_t)rperm[k - n] * S.Bp + b];
+        if (k < 2 * n + m) return adj_a(S, cperm[k - n - m], b);
+        if (k < 3 * n + m) return adj_d(S, cperm[k - 2 * n - m], b);
+        return adj_sig(S, rperm[k - 3 * n - m], b);
+      },
+      [&](int64_t k, int64_t b, T v) {
+        if (k < n + m)
+          mask[b * (n + m) + k] = v;
+        else if (k < 2 * n + m)
+          av[b * n + k - n - m] = v;
+        else if (k < 3 * n + m)
+          dv[b * n + k - 2 * n - m] = v;
+        else
+          sv[b * m + k - 3 * n - m] = v;
+      });
+}
+
+// dst[b][k] = src[map[k]][b], 0 where map[k] < 0: the entries of the slices
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gmr_entries(const T* __restrict__ src, int64_t Bp,
+                                                        const int32_t* __restrict__ map, int64_t K,
+                                                        int64_t batch, T* __restrict__ dst) {
+  minor_to_major_tile<T>(
+      K, batch,
+      [&](int64_t k, int64_t b) -> T { return map[k] < 0 ? T(0) : src[(size_t)map[k] * Bp + b]; },
+      [&](int64_t k, int64_t b, T v) { dst[b * K + k] = v; });
+}
+
+// The right-hand side g = [cot * eligible, cotd * eligible, 0] of every sample (see
+// k_gm_rhs), x = 0, r = g, and the threshold max(atol, tol * max |g|).  One
+// workgroup per sample; cot is the caller's, divided by ``metric`` where there is one.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gmr_init(Gmr<T> A, T* G, const T* __restrict__ cot,
+                                                     const T* __restrict__ metric,
+                                                     const T* __restrict__ cotd, int64_t Bp,
+                                                     const int32_t* __restrict__ cperm,
+                                                     const int32_t* __restrict__ rperm,
+                                                     const int32_t* __restrict__ conv, int force,
+                                                     T tol, T atol) {
+  const int64_t b = blockIdx.x;
+  const int n = A.n, m = A.m;
+  const bool elig = force || conv[b] != 0;
+  T big = T(0);
+  for (int e = threadIdx.x; e < A.W; e += kBlock) {
+    T v = T(0);
+    if (e < n) {
+      const int j = cperm[e];
+      v = cot[b * n + j];
+      if (metric) v = v / metric[j];
+    } else if (cotd && e < n + m) {
+      v = cotd[(size_t)rperm[e - n] * Bp + b];
+    }
+    v = elig ? v : T(0);
+    G[b * A.Wp + e] = v;
+    A.R[b * A.Wp + e] = v;
+    A.X[b * A.Wp + e] = T(0);
+    big = maxp(big, absv(v));
+  }
+  __shared__ T part[kBlock];
+  part[threadIdx.x] = big;
+  __syncthreads();
+  for (int h = kBlock / 2; h > 0; h >>= 1) {
+    if ((int)threadIdx.x < h) part[threadIdx.x] = maxp(part[threadIdx.x], part[threadIdx.x + h]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    A.thr[b] = maxp(atol, tol * part[0]);
+    A.rinf[b] = part[0];  // x0 = 0: rhs - matvec(0) = rhs
+    A.xfin[b] = T(1);
+    A.total[b] = 0;
+  }
+}
+
+// The solution back to batch-minor rows in the variables' and rows' own order.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_gmr_solution(const T* __restrict__ X, int64_t Wp, int n,
+                                                         int m, const int32_t* __restrict__ cperm,
+                                                         const int32_t* __restrict__ rperm,
+                                                         int64_t batch, int64_t Bp,
+                                                         T* __restrict__ dst) {
+  __shared__ T tile[64][65];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int64_t k0 = (int64_t)blockIdx.x * 64, b0 = (int64_t)blockIdx.y * 64;
+  const int64_t W = 2 * (int64_t)n + m;
+#pragma unroll 4
+  for (int r = ty; r < 64; r += kBlock / 64)
+    tile[r][tx] = b0 + r < batch && k0 + tx < W ? X[(b0 + r) * Wp + k0 + tx] : T(0);
+  __syncthreads();
+#pragma unroll 4
+  for (int r = ty; r < 64; r += kBlock / 64) {
+    const int64_t k = k0 + r;
+    if (k >= W) continue;
+    const int64_t row = k < n ? cperm[k] : (k < n + m ? n + rperm[k - n] : n + m + cperm[k - n - m]);
+    dst[row * Bp + b0 + tx] = tile[tx][r];
+  }
+}
+
 template <typename T>
 __global__ void k_copy_i32(int64_t count, const int32_t* __restrict__ src, int32_t* dst) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1295,8 +1424,12 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
                           ? 5
                           : (int)std::min<int64_t>({(int64_t)o.restart, (int64_t)o.max_iterations, W});
   if (restart > kMaxRestart) return set_error(PURIN_CP_ERR_UNSUPPORTED, "restart above 128");
-  static_assert((kMaxRestart + 2) * 4 <= kPinnedBytes, "per-step counts must fit the pinned buffer");
   const bool dense = qa && qa->dense;
+  static_assert((kMaxRestart + 2) * 4 <= kPinnedBytes, "per-step counts must fit the pinned buffer");
+  // GMRES runs one workgroup per sample where its vectors u and w fit LDS and the
+  // restart length its one-lane-per-vector algebra; otherwise on batch-minor passes
+  // (very large problems, long restarts)
+  const bool wg = !dense && gmr_fits(p, restart);
   // workspace
   const int nchunk = (int)((W + kChunk - 1) / kChunk);
   // Gram--Schmidt passes: about 1024 blocks of 4 wavefronts over the batch tiles
@@ -1312,24 +1445,38 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   const size_t vec = (size_t)W * Bp * es;
   size_t o_ = 0;
   auto take = [&](size_t bytes) { size_t r = o_; o_ = al(o_ + bytes); return r; };
-  const size_t oV = take(vec * (restart + 1)), oX = take(vec), oG = take(vec), oRr = take(vec),
-               oT1 = take(vec), oCm = take(n * Bp * es), oClo = take(n * Bp * es),
+  const size_t oX = take(vec), oCm = take(n * Bp * es), oClo = take(n * Bp * es),
                oChi = take(n * Bp * es), oDm = take(m * Bp * es), oDp = take(m * Bp * es),
-               oU = take(n * Bp * es), oWv = take(m * Bp * es),
-               oPart = take((size_t)(restart + 1) * std::max(nchunk, nchunk2) * Bp * es),
-               oS1 = take(Bp * es), oS2 = take(Bp * es), oThr = take(Bp * es), oRinf = take(Bp * es),
-               oCyc = take(Bp * 4), oAct = take(Bp * 4), oSteps = take(Bp * 4),
-               oScale = take(Bp * es), oHess = take((size_t)Bp * (restart + 1) * restart * es),
-               oCs = take((size_t)restart * Bp * es), oSn = take((size_t)restart * Bp * es),
-               oGv = take((size_t)(restart + 1) * Bp * es), oCoef = take((size_t)restart * Bp * es),
-               oCnt = take(256), oStepCnt = take((size_t)(restart + 2) * 4), oLw = take(Bp * es), oGt = take(n * Bp * es),
+               oU = take(n * Bp * es), oThr = take(Bp * es), oRinf = take(Bp * es),
+               oS2 = take(Bp * es), oLw = take(Bp * es), oGt = take(n * Bp * es),
                oGlo = take(n * Bp * es), oGhi = take(n * Bp * es), oGr = take(m * Bp * es),
-               oGF = take((size_t)M * Bp * es),
-               oTm = take((size_t)(restart + 1) * (restart + 1) * Bp * es),
-               oHu = take((size_t)(restart + 1) * restart * Bp * es),
-               oU2 = take((size_t)(restart + 1) * Bp * es), oG1 = take((size_t)(restart + 1) * Bp * es),
-               oQ1 = take((size_t)(restart + 1) * Bp * es), oCg = take((size_t)(restart + 1) * Bp * es),
-               oWc = take((size_t)restart * Bp * es), oTot = take(Bp * 4);
+               oGF = take((size_t)M * Bp * es), oTot = take(Bp * 4), oCnt = take(256);
+  // the batch-minor passes' vectors and scalars
+  const size_t old = wg ? 0 : 1;
+  const size_t oV = take(old * vec * (restart + 1)), oG = take(old * vec), oRr = take(old * vec),
+               oT1 = take(old * vec), oWv = take(old * m * Bp * es),
+               oPart = take(old * (restart + 1) * std::max(nchunk, nchunk2) * Bp * es),
+               oS1 = take(old * Bp * es), oCyc = take(old * Bp * 4), oAct = take(old * Bp * 4),
+               oSteps = take(old * Bp * 4), oScale = take(old * Bp * es),
+               oHess = take(old * Bp * (restart + 1) * restart * es),
+               oCs = take(old * restart * Bp * es), oSn = take(old * restart * Bp * es),
+               oGv = take(old * (restart + 1) * Bp * es), oCoef = take(old * restart * Bp * es),
+               oStepCnt = take(old * (restart + 2) * 4),
+               oTm = take(old * (restart + 1) * (restart + 1) * Bp * es),
+               oHu = take(old * (restart + 1) * restart * Bp * es),
+               oU2 = take(old * (restart + 1) * Bp * es), oG1 = take(old * (restart + 1) * Bp * es),
+               oQ1 = take(old * (restart + 1) * Bp * es), oCg = take(old * (restart + 1) * Bp * es),
+               oWc = take(old * restart * Bp * es);
+  // the per-sample cycles' sample-major vectors: basis, solution, residual, rhs,
+  // masks, steps per element, the samples' matrix entries in slice order
+  const int64_t Wp = round_up(W, 16);
+  const bool dg = per_sample || p->diag;
+  const size_t smp = wg ? (size_t)batch * es : 0;
+  const size_t zZ = take(smp * (restart + 1) * Wp), zX = take(smp * Wp), zR = take(smp * Wp),
+               zG = take(smp * Wp), zM = take(smp * (n + m)), zA = take(dg ? smp * n : 0),
+               zD = take(dg ? smp * n : 0), zS = take(dg ? smp * m : 0),
+               zRv = take(per_sample ? smp * p->sl_rn : 0),
+               zCv = take(per_sample ? smp * p->sl_cn : 0);
   // per-sample coefficients: the forward's per-sample arrays are rebuilt from
   // values in a region laid out like the forward workspace, plus sigma . w and
   // the coefficient gradient in entry order
@@ -1597,7 +1744,7 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   };
 
   // rhs g = [cot * eligible, 0, 0] (cotangent divided by sqrt(D) for a metric)
-  to_minor<T>(st, cot_y, batch, n, n, T1, Bp, metric, metric ? 2 : 0);
+  if (!wg) to_minor<T>(st, cot_y, batch, n, n, T1, Bp, metric, metric ? 2 : 0);
   // the QP's dual cotangent w.r.t. the scaled dual: cot_dual * scale (the
   // returned multipliers are dual * scale, diagonal_qp.py:274)
   T* cotd = nullptr;
@@ -1608,8 +1755,9 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
     k_prep_rows<T><<<2048, 256, 0, st>>>((int)m, Bp, p->dkept, (const T*)p->dscale, PS.SC, CD,
                                          nullptr, cotd, nullptr);
   }
-  k_gm_rhs<T><<<eb, 256, 0, st>>>(n, m, W, Bp, batch, T1, cotd, conv,
-                                  dense ? 1 : o.force_eligible, Gr);
+  if (!wg)
+    k_gm_rhs<T><<<eb, 256, 0, st>>>(n, m, W, Bp, batch, T1, cotd, conv,
+                                    dense ? 1 : o.force_eligible, Gr);
   T* lam_w = (T*)(ws + oLw);
   purin_cp_adjoint_stats stats{};
   if (dense) {
@@ -1663,6 +1811,81 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
     k_fill_weights<T><<<sb, 256, 0, st>>>(batch, Bp, lam_w);
     if (o.arnoldi_iterations)
       k_fill<int32_t><<<sb, 256, 0, st>>>(o.arnoldi_iterations, batch, (int32_t)iters);
+  } else if (wg) {
+    Gmr<T> Q{};
+    Q.n = (int)n;
+    Q.m = (int)m;
+    Q.W = (int)W;
+    Q.restart = restart;
+    Q.Wp = Wp;
+    Q.nsr = p->sl_nsr;
+    Q.nsc = p->sl_nsc;
+    Q.roff = p->sl_roff;
+    Q.coff = p->sl_coff;
+    Q.ridx = p->sl_ridx;
+    Q.cidx = p->sl_cidx;
+    Q.rval = (const T*)p->sl_rval;
+    Q.cval = (const T*)p->sl_cval;
+    Q.a = S.a;
+    Q.delta = S.delta;
+    Q.sigma = S.sigma;
+    Q.mask = (const T*)(ws + zM);
+    Q.G = (const T*)(ws + zG);
+    Q.X = (T*)(ws + zX);
+    Q.R = (T*)(ws + zR);
+    Q.Z = (T*)(ws + zZ);
+    Q.thr = G.thr;
+    Q.rinf = G.rinf;
+    Q.xfin = S2;
+    Q.total = G.total;
+    Q.ctrl = G.counter;
+    const unsigned by = (unsigned)((batch + 63) / 64);
+    if (S.dg) {
+      Q.av = (const T*)(ws + zA);
+      Q.dv = (const T*)(ws + zD);
+      Q.sv = (const T*)(ws + zS);
+    }
+    const int64_t stage = S.dg ? 3 * n + 2 * m : n + m;
+    k_gmr_stage<T><<<dim3((unsigned)((stage + 63) / 64), by), kBlock, 0, st>>>(
+        S, p->sl_cperm, p->sl_rperm, batch, (T*)(ws + zM), (T*)(ws + zA), (T*)(ws + zD),
+        (T*)(ws + zS));
+    if (per_sample) {  // the samples' entries, or one copy of a shared set (S.K.rval)
+      const bool each = S.K.rvb != nullptr;
+      const int64_t copies = each ? batch : 1, ld = each ? Bp : 1;
+      const unsigned cy = (unsigned)((copies + 63) / 64);
+      if (p->sl_rn)
+        k_gmr_entries<T><<<dim3((unsigned)((p->sl_rn + 63) / 64), cy), kBlock, 0, st>>>(
+            each ? S.K.rvb : S.K.rval, ld, p->sl_rsrc, p->sl_rn, copies, (T*)(ws + zRv));
+      if (p->sl_cn)
+        k_gmr_entries<T><<<dim3((unsigned)((p->sl_cn + 63) / 64), cy), kBlock, 0, st>>>(
+            each ? S.K.cvb : S.K.cval, ld, p->sl_csrc, p->sl_cn, copies, (T*)(ws + zCv));
+      Q.rval = (const T*)(ws + zRv);
+      Q.cval = (const T*)(ws + zCv);
+      Q.rstride = each ? p->sl_rn : 0;
+      Q.cstride = each ? p->sl_cn : 0;
+    }
+    k_gmr_init<T><<<(unsigned)batch, kBlock, 0, st>>>(
+        Q, (T*)(ws + zG), cot_y, metric, cotd, Bp, p->sl_cperm, p->sl_rperm, conv,
+        o.force_eligible, (T)o.tolerance, (T)o.atol);
+    // cycles, a few per host read: a cycle that no sample runs ends the solve
+    int64_t completed = 0;
+    for (bool more = true; more && completed < o.max_iterations;) {
+      k_fill<int32_t><<<1, 64, 0, st>>>(G.counter, kGmrGroup, 0);
+      for (int c = 0; c < kGmrGroup; ++c)
+        if (int rc = gmr_cycle<T>(st, Q, batch, S.dg != 0, c, completed, o.max_iterations)) return rc;
+      PURIN_HIP(hipMemcpyAsync(hw.get(), G.counter, kGmrGroup * sizeof(int32_t),
+                               hipMemcpyDeviceToHost, st));
+      PURIN_HIP(hipStreamSynchronize(st));
+      for (int c = 0; c < kGmrGroup && more; ++c) {
+        const int32_t steps = hw.get()[c];
+        more = steps > 0;
+        completed += steps;
+        stats.arnoldi_steps += steps;
+        stats.cycles += steps > 0;
+      }
+    }
+    k_gmr_solution<T><<<dim3((unsigned)((W + 63) / 64), by), kBlock, 0, st>>>(
+        Q.X, Wp, (int)n, (int)m, p->sl_cperm, p->sl_rperm, batch, Bp, X);
   } else {
   // threshold = max(atol, tol * max|g|) and residual_inf = max|g - A 0| = max|g|
   k_gs<T, 4><<<ggs, kBlock, 0, st>>>(nullptr, 0, 0, Gr, nullptr, W, Bp, part, nchunk, Bp);
@@ -1748,19 +1971,22 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
     completed += it;
     stats.arnoldi_steps += it;
   }
-  if (o.arnoldi_iterations)
-    PURIN_HIP(hipMemcpyAsync(o.arnoldi_iterations, G.total, (size_t)batch * sizeof(int32_t),
-                             hipMemcpyDeviceToDevice, st));
-  if (own_ws) {  // read by purin_cp_last_adjoint_iterations until the next such call
-    std::lock_guard<std::mutex> lock(p->mu);
-    p->adj_steps = G.total;
-    p->adj_steps_batch = batch;
-  }
-  // finiteness of the solution, info, valid (operators.py:1119-1122, bounds.py:148-153)
+  // finiteness of the solution
   k_gs<T, 2><<<ggs, kBlock, 0, st>>>(nullptr, 0, 0, X, nullptr, W, Bp, part, nchunk, Bp);
   k_reduce<T><<<sb, 256, 0, st>>>(part + (size_t)nchunk * Bp, 1, nchunk, Bp, S2, 2);
-  k_gm_finish<T><<<sb, 256, 0, st>>>(G, S2, conv, (T)o.adjoint_tolerance, o.force_eligible,
-                                     lam_w, valid, info, gres);
+  }
+  if (!dense) {
+    if (o.arnoldi_iterations)
+      PURIN_HIP(hipMemcpyAsync(o.arnoldi_iterations, G.total, (size_t)batch * sizeof(int32_t),
+                               hipMemcpyDeviceToDevice, st));
+    if (own_ws) {  // read by purin_cp_last_adjoint_iterations until the next such call
+      std::lock_guard<std::mutex> lock(p->mu);
+      p->adj_steps = G.total;
+      p->adj_steps_batch = batch;
+    }
+    // info, valid (operators.py:1119-1122, bounds.py:148-153)
+    k_gm_finish<T><<<sb, 256, 0, st>>>(G, S2, conv, (T)o.adjoint_tolerance, o.force_eligible,
+                                       lam_w, valid, info, gres);
   }
   // final pullback of the masked lambda
   T* gt = (T*)(ws + oGt);

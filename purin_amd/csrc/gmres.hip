@@ -1,0 +1,585 @@
+// Restarted GMRES of the implicit VJP, one workgroup per sample.
+//
+// Reference: _batched_restarted_gmres
+// (src/purin/solvers/primal_dual_interior_point/operators.py:792-1125).  The
+// samples are independent within a restart cycle, so a workgroup runs a whole
+// cycle of one sample: operator, both projections, the Givens step and the stop
+// test of every Arnoldi step, then the correction and the candidate's residual.
+// The batch meets only between cycles, where the reference bounds a cycle by the
+// iterations left (the longest sample's steps count, Gmr::ctrl).
+//
+// The batch-minor passes this replaces took about a dozen dependent launches per
+// Arnoldi step, each over the whole batch: ~110 us a step for a small problem
+// whatever its bytes, and with a large one every sample's basis was streamed until
+// the slowest sample stopped.  Here a step costs its own sample's work.
+//
+// The basis is raw, as in adjoint.hip (k_gm_tri): slot i holds Z_i, the image of
+// step i - 1 after one projection, v_j = sum_{i <= j} Z_i Tm[i][j], so a step reads
+// the prefix twice.  The dot pass walks the elements last to first and the update
+// pass first to last, so the update begins on rows the caches still hold.
+#include <type_traits>
+
+#include "common.hpp"
+#include "gmres.hpp"
+
+namespace purin {
+
+namespace {
+
+constexpr int kLd = kGmrRestart + 1;  // row stride of the per-sample triangular matrices
+
+// --- reductions over a wavefront ------------------------------------------------
+
+template <typename T>
+struct Words;
+template <>
+struct Words<double> {
+  static constexpr int N = 2;
+};
+template <>
+struct Words<float> {
+  static constexpr int N = 1;
+};
+
+// a', b' = [a's lower half, b's lower half], [a's upper half, b's upper half] of
+// the wavefront (BIT = 32) or of each half wavefront's pair of rows (BIT = 16): the
+// sum a' + b' leaves a's total over the pair in the lower and b's in the upper half.
+template <int BIT, typename T>
+__device__ __forceinline__ T swap_add(T a, T b) {
+  constexpr int N = Words<T>::N;
+  typedef uint32_t U __attribute__((ext_vector_type(N)));
+  U x = __builtin_bit_cast(U, a), y = __builtin_bit_cast(U, b);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if constexpr (BIT == 32) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false);
+      x[i] = r[0];
+      y[i] = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+      x[i] = r[0];
+      y[i] = r[1];
+    }
+  }
+  return __builtin_bit_cast(T, x) + __builtin_bit_cast(T, y);
+}
+
+// v of the lane that DPP control CTRL pairs with this one
+template <int CTRL, typename T>
+__device__ __forceinline__ T dpp(T v) {
+  constexpr int N = Words<T>::N;
+  typedef int U __attribute__((ext_vector_type(N)));
+  U x = __builtin_bit_cast(U, v);
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_update_dpp(0, x[i], CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(T, x);
+}
+constexpr int kMirror16 = 0x140;  // lane i of a row of 16 with lane 15 - i
+constexpr int kMirror8 = 0x141;   // lane i of a half row with lane 7 - i
+constexpr int kMirror4 = 0x1b;    // lane i of a quad with lane 3 - i
+constexpr int kMirror2 = 0xb1;    // lane i of a pair with lane 1 - i
+
+// one halving step on lane bit BIT: lanes with the bit keep the upper half of v
+template <int BIT, int N, typename T>
+__device__ __forceinline__ void halve(T (&v)[kGmrRestart], int lane) {
+  constexpr int H = N / 2;
+#pragma unroll
+  for (int i = 0; i < H; ++i) {
+    if constexpr (BIT >= 16) {
+      v[i] = swap_add<BIT>(v[i], v[i + H]);
+    } else {
+      constexpr int C = BIT == 8 ? kMirror16 : (BIT == 4 ? kMirror8 : kMirror4);
+      const bool up = (lane & BIT) != 0;
+      const T send = up ? v[i] : v[i + H];
+      const T keep = up ? v[i + H] : v[i];
+      v[i] = keep + dpp<C>(send);
+    }
+  }
+}
+
+// plain sums over the remaining lane bits below and including BIT
+template <int BIT, typename T>
+__device__ __forceinline__ T fold(T v) {
+  if constexpr (BIT >= 32) v = swap_add<32>(v, v);
+  if constexpr (BIT >= 16) v = swap_add<16>(v, v);
+  if constexpr (BIT >= 8) v = v + dpp<kMirror16>(v);
+  if constexpr (BIT >= 4) v = v + dpp<kMirror8>(v);
+  if constexpr (BIT >= 2) v = v + dpp<kMirror4>(v);
+  return v + dpp<kMirror2>(v);
+}
+
+// Sums of v[0..N) over the wavefront (N = 4, 8, 16 or 32): lane l returns the sum
+// of v[l * N / 64].  A butterfly that halves the values held at each step: 31
+// exchanges for 32 sums in place of 6 each.
+template <int N, typename T>
+__device__ __forceinline__ T wave_sums(T (&v)[kGmrRestart], int lane) {
+  if constexpr (N == 32) {
+    halve<32, 32>(v, lane);
+    halve<16, 16>(v, lane);
+    halve<8, 8>(v, lane);
+    halve<4, 4>(v, lane);
+    halve<2, 2>(v, lane);
+    return v[0] + dpp<kMirror2>(v[0]);
+  } else if constexpr (N == 16) {
+    halve<32, 16>(v, lane);
+    halve<16, 8>(v, lane);
+    halve<8, 4>(v, lane);
+    halve<4, 2>(v, lane);
+    return fold<2>(v[0]);
+  } else if constexpr (N == 8) {
+    halve<32, 8>(v, lane);
+    halve<16, 4>(v, lane);
+    halve<8, 2>(v, lane);
+    return fold<4>(v[0]);
+  } else {
+    halve<32, 4>(v, lane);
+    halve<16, 2>(v, lane);
+    return fold<8>(v[0]);
+  }
+}
+
+// the value every lane holds, as a scalar
+template <typename T>
+__device__ __forceinline__ T uniform(T v) {
+  constexpr int N = Words<T>::N;
+  typedef int U __attribute__((ext_vector_type(N)));
+  U x = __builtin_bit_cast(U, v);
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_readfirstlane(x[i]);
+  return __builtin_bit_cast(T, x);
+}
+
+// LDS written by one lane of a wavefront is read by another after this
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// --- LDS of one workgroup ---------------------------------------------------------
+
+// Elements: u [n + 1], w [m + 1], the wavefronts' partial sums [BS / 64][33], then
+// per-sample algebra (below), then the basis where it fits.
+constexpr int kAlg = 3 * kLd * kLd + 10 * kLd;
+
+template <typename T>
+struct Alg {  // pointers into the algebra block
+  T *Tm, *Hu, *H, *P, *Gv, *Q, *U2, *G1, *Cs, *Sn, *g, *Col, *Wc;
+  __device__ explicit Alg(T* p) {
+    Tm = p;                 // [i][j], upper triangular
+    Hu = Tm + kLd * kLd;    // unrotated Hessenberg matrix
+    H = Hu + kLd * kLd;     // rotated
+    P = H + kLd * kLd;
+    Gv = P + kLd;
+    Q = Gv + kLd;
+    U2 = Q + kLd;
+    G1 = U2 + kLd;
+    Cs = G1 + kLd;
+    Sn = Cs + kLd;
+    g = Sn + kLd;
+    Col = g + kLd;
+    Wc = Col + kLd;
+  }
+};
+
+inline size_t lds_elems(int64_t n, int64_t m, int64_t W, int restart, int bs, bool basis) {
+  return (size_t)(n + 1 + m + 1 + (bs / 64) * kLd + kAlg + (basis ? (restart + 1) * W : 0));
+}
+
+// --- the operator -----------------------------------------------------------------
+
+// out = v sc - pullback(v sc) (adjoint.hip's k_op_*): u = C (gy + 2 gb),
+// w = D (gd - delta K u), out = (gy - (a u - gb), gd - w, gb - sigma K^T w).  One
+// thread per row / column of a slice; u and w meet in LDS.
+template <typename T, int BS, bool DG>
+__device__ __forceinline__ void apply(const Gmr<T>& A, int64_t b, const T* __restrict__ v, T sc,
+                                      T* __restrict__ out, T* u, T* w) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = A.n, m = A.m;
+  const T* __restrict__ mask = A.mask + (size_t)b * (n + m);
+  const T* __restrict__ av = DG ? A.av + (size_t)b * n : nullptr;
+  const T* __restrict__ dv = DG ? A.dv + (size_t)b * n : nullptr;
+  const T* __restrict__ sv = DG ? A.sv + (size_t)b * m : nullptr;
+  for (int j = tid; j < n; j += BS) {
+    const T gy = v[j] * sc, gb = v[n + m + j] * sc;
+    const T uj = mask[j] * (gy + T(2) * gb);
+    u[j] = DG ? dv[j] * uj : uj;
+    out[j] = gy - ((DG ? av[j] : A.a) * uj - gb);
+  }
+  __syncthreads();
+  const T* __restrict__ rval = A.rval + (size_t)b * A.rstride;
+  for (int s = wave; s < A.nsr; s += BS / 64) {
+    const int o0 = A.roff[s], o1 = A.roff[s + 1];
+    T acc = T(0);
+#pragma unroll 4
+    for (int o = o0 + lane; o < o1; o += 64) acc += rval[o] * u[A.ridx[o]];
+    const int i = s * 64 + lane;
+    if (i < m) {
+      const T gd = v[n + i] * sc;
+      const T wi = mask[n + i] * (DG ? gd - acc : gd - A.delta * acc);
+      w[i] = DG ? sv[i] * wi : wi;
+      out[n + i] = gd - wi;
+    }
+  }
+  __syncthreads();
+  const T* __restrict__ cval = A.cval + (size_t)b * A.cstride;
+  for (int s = wave; s < A.nsc; s += BS / 64) {
+    const int o0 = A.coff[s], o1 = A.coff[s + 1];
+    T acc = T(0);
+#pragma unroll 4
+    for (int o = o0 + lane; o < o1; o += 64) acc += cval[o] * w[A.cidx[o]];
+    const int j = s * 64 + lane;
+    if (j < n) {
+      const T gb = v[n + m + j] * sc;
+      out[n + m + j] = DG ? gb - acc : gb - A.sigma * acc;
+    }
+  }
+  __syncthreads();
+}
+
+// --- the two passes over the prefix -------------------------------------------------
+
+// Element e of the first nv vectors of Z into z (the last one again for i >= nv).
+// One 32-bit byte offset walks the vectors from Z's scalar base, so the prefix costs
+// no address registers; NV - 4 < nv <= NV.
+template <typename T, int NV>
+__device__ __forceinline__ void load_prefix(const T* Z, uint32_t ldb, int nv, int e, T (&z)[NV]) {
+  uint32_t off = (uint32_t)e * (uint32_t)sizeof(T);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (i > 0) off += (i <= NV - 4 || i < nv) ? ldb : 0u;
+    z[i] = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(Z) + off);
+  }
+}
+
+// red[wave][i] = the wavefront's part of Z_i . y, i < nv
+template <typename T, int BS, int NV>
+__device__ __forceinline__ void pass_dots(const T* Z, uint32_t ldb, int nv, const T* y, int W,
+                                          T* red) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  T acc[kGmrRestart];
+#pragma unroll
+  for (int i = 0; i < kGmrRestart; ++i) acc[i] = T(0);
+  for (int e = tid + (W - 1 - tid) / BS * BS; e >= 0 && tid < W; e -= BS) {
+    const T ye = y[e];
+    T z[NV];
+    load_prefix<T, NV>(Z, ldb, nv, e, z);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] += z[i] * ye;
+  }
+  constexpr int N = NV <= 4 ? 4 : (NV <= 8 ? 8 : (NV <= 16 ? 16 : 32));
+  const T s = wave_sums<N>(acc, lane);
+  constexpr int per = 64 / N;
+  if (lane % per == 0) red[wave * kLd + lane / per] = s;
+}
+
+// y <- y - sum_i q_i Z_i; red[wave][i] = the wavefront's part of Z_i . y for
+// i < nv, red[wave][kLd - 1] its part of y . y
+template <typename T, int BS, int NV>
+__device__ __forceinline__ void pass_update(const T* Z, uint32_t ldb, int nv, T* y, int W,
+                                            const T* Q, T* red) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  T acc[kGmrRestart], q[NV], nrm = T(0);
+#pragma unroll
+  for (int i = 0; i < kGmrRestart; ++i) acc[i] = T(0);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) q[i] = i < nv ? uniform(Q[i]) : T(0);
+  for (int e = tid; e < W; e += BS) {
+    T ye = y[e];
+    T z[NV];
+    load_prefix<T, NV>(Z, ldb, nv, e, z);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) ye -= q[i] * z[i];
+    y[e] = ye;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) acc[i] += z[i] * ye;
+    nrm += ye * ye;
+  }
+  constexpr int N = NV <= 4 ? 4 : (NV <= 8 ? 8 : (NV <= 16 ? 16 : 32));
+  const T s = wave_sums<N>(acc, lane);
+  nrm = fold<32>(nrm);
+  constexpr int per = 64 / N;
+  if (lane % per == 0) red[wave * kLd + lane / per] = s;
+  if (lane == 0) red[wave * kLd + kLd - 1] = nrm;
+}
+
+template <typename T, int BS, bool UPDATE>
+__device__ __forceinline__ void pass(const T* Z, uint32_t ldb, int nv, T* y, int W, const T* Q,
+                                     T* red) {
+  // the bucket sets the registers a thread holds and the loads it has in flight
+  auto go = [&](auto k) {
+    constexpr int NV = decltype(k)::value;
+    if constexpr (UPDATE)
+      pass_update<T, BS, NV>(Z, ldb, nv, y, W, Q, red);
+    else
+      pass_dots<T, BS, NV>(Z, ldb, nv, y, W, red);
+  };
+  switch ((nv - 1) >> 2) {
+    case 0: go(std::integral_constant<int, 4>{}); break;
+    case 1: go(std::integral_constant<int, 8>{}); break;
+    case 2: go(std::integral_constant<int, 12>{}); break;
+    case 3: go(std::integral_constant<int, 16>{}); break;
+    case 4: go(std::integral_constant<int, 20>{}); break;
+    case 5: go(std::integral_constant<int, 24>{}); break;
+    case 6: go(std::integral_constant<int, 28>{}); break;
+    default: go(std::integral_constant<int, 32>{}); break;
+  }
+}
+
+// --- one restart cycle --------------------------------------------------------------
+
+template <typename T, int BS, bool DG, bool ZL>
+__global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base, int64_t max_it) {
+  extern __shared__ __align__(16) unsigned char gmr_raw[];
+  constexpr int NW = BS / 64;
+  const int64_t b = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = A.n, m = A.m, W = A.W, R = A.restart;
+  int64_t done = base;
+  for (int k = 0; k < c; ++k) done += A.ctrl[k];
+  const int limit = (int)(max_it - done < R ? max_it - done : R);
+  const T thr = A.thr[b];
+  if (limit <= 0 || !(A.rinf[b] > thr)) return;  // the same for the whole workgroup
+  T* u = reinterpret_cast<T*>(gmr_raw);
+  T* w = u + n + 1;
+  T* red = w + m + 1;
+  const Alg<T> S(red + NW * kLd);
+  T* zl = S.Wc + kLd;
+  __shared__ T s_inv;
+  __shared__ int s_on;
+  T* __restrict__ X = A.X + (size_t)b * A.Wp;
+  T* __restrict__ Rr = A.R + (size_t)b * A.Wp;
+  const T* __restrict__ G = A.G + (size_t)b * A.Wp;
+  T* Z = ZL ? zl : A.Z + (size_t)b * (R + 1) * A.Wp;
+  const int64_t ld = ZL ? W : A.Wp;
+  const uint32_t ldb = (uint32_t)(ld * sizeof(T));
+  const T eps = T(1e-30), brk = T(1e-14);
+
+  // beta = ||r||, Z_0 = r / max(beta, eps)
+  T acc = T(0);
+  for (int e = tid; e < W; e += BS) acc += Rr[e] * Rr[e];
+  acc = fold<32>(acc);
+  if (lane == 0) red[wave * kLd] = acc;
+  if (tid == 0) {
+    u[n] = T(0);
+    w[m] = T(0);
+  }
+  __syncthreads();
+  T beta = T(0);
+#pragma unroll
+  for (int k = 0; k < NW; ++k) beta += red[k * kLd];
+  beta = __builtin_sqrt(beta);
+  const T scale = T(1) / maxp(beta, eps);
+  for (int e = tid; e < W; e += BS) Z[e] = Rr[e] * scale;
+  if (tid < kLd) {
+    S.g[tid] = tid == 0 ? beta : T(0);
+    S.U2[tid] = T(0);
+  }
+  if (tid == 0) {
+    S.Tm[0] = T(1);
+    s_inv = T(1);
+    s_on = 1;
+  }
+  __syncthreads();
+
+  int it = 0;
+  while (it < limit) {
+    const int nv = it + 1;
+    T* y = Z + (int64_t)nv * ld;
+    apply<T, BS, DG>(A, b, Z + (int64_t)it * ld, s_inv, y, u, w);
+    pass<T, BS, false>(Z, ldb, nv, y, W, S.Q, red);
+    __syncthreads();
+    if (wave == 0) {  // p = Z^T y; g1 = Tm^T p; q1 = Tm g1
+      if (lane < nv) {
+        T s = T(0);
+#pragma unroll
+        for (int k = 0; k < NW; ++k) s += red[k * kLd + lane];
+        S.P[lane] = s;
+      }
+      wave_sync();
+      if (lane < nv) {
+        T s = T(0);
+#pragma unroll 8
+        for (int i = 0; i <= lane; ++i) s += S.Tm[i * kLd + lane] * S.P[i];
+        S.G1[lane] = s;
+      }
+      wave_sync();
+      if (lane < nv) {
+        T s = T(0);
+#pragma unroll 8
+        for (int j = lane; j < nv; ++j) s += S.Tm[lane * kLd + j] * S.G1[j];
+        S.Q[lane] = s;
+      }
+    }
+    __syncthreads();
+    pass<T, BS, true>(Z, ldb, nv, y, W, S.Q, red);
+    __syncthreads();
+    if (wave == 0) {  // the step's algebra (k_gm_tri, MODE 2)
+      if (lane < nv || lane == kLd - 1) {
+        T s = T(0);
+#pragma unroll
+        for (int k = 0; k < NW; ++k) s += red[k * kLd + lane];
+        S.P[lane] = s;
+      }
+      wave_sync();
+      T g2 = T(0);
+      if (lane < nv) {
+#pragma unroll 8
+        for (int i = 0; i <= lane; ++i) g2 += S.Tm[i * kLd + lane] * S.P[i];
+        S.Gv[lane] = g2;
+        T cj = T(0);
+#pragma unroll 8
+        for (int k = lane > 0 ? lane - 1 : 0; k < it; ++k) cj += S.Hu[lane * kLd + k] * S.U2[k];
+        const T col = (S.G1[lane] + g2) - cj;
+        S.Col[lane] = col;
+        S.Hu[lane * kLd + it] = col;
+      }
+      wave_sync();
+      const T ss = fold<32>(lane < nv ? g2 * g2 : T(0));
+      const T n1 = S.P[kLd - 1];
+      const T d2 = n1 - ss;
+      const T next_norm = d2 < T(0) ? T(0) : __builtin_sqrt(d2);  // NaN stays NaN
+      // the rotations of the earlier steps, in order, on every lane alike
+      T carry = S.Col[0];
+      for (int ri = 0; ri < it; ++ri) {
+        const T cc = S.Cs[ri], sn = S.Sn[ri], nx = S.Col[ri + 1];
+        if (lane == 0) S.H[ri * kLd + it] = cc * carry + sn * nx;
+        carry = -sn * carry + cc * nx;
+      }
+      const T rnorm = hypotv(carry, next_norm);
+      const T safe = maxp(rnorm, eps);
+      const T nc = rnorm > eps ? carry / safe : T(1);
+      const T ns = rnorm > eps ? next_norm / safe : T(0);
+      const T pc = S.g[it], pn = S.g[it + 1];
+      const T rc = nc * pc + ns * pn, rn = -ns * pc + nc * pn;
+      const T inv = T(1) / maxp(next_norm, eps);
+      const T est = absv(rn);
+      const bool on = finite(est) && finite(rnorm) && finite(n1) && !(next_norm <= brk) && est > thr;
+      // column it + 1 of Tm: v_{it+1} = (Z_{it+1} - Z Tm g2) / nu, and u = g2 / nu
+      T tc = T(0);
+      if (lane < nv) {
+#pragma unroll 8
+        for (int j = lane; j < nv; ++j) tc += S.Tm[lane * kLd + j] * S.Gv[j];
+      }
+      wave_sync();
+      if (lane < nv) {
+        S.Tm[lane * kLd + nv] = -(tc * inv);
+        S.U2[lane] = g2 * inv;
+      }
+      if (lane == 0) {
+        S.Hu[nv * kLd + it] = next_norm;
+        S.Cs[it] = nc;
+        S.Sn[it] = ns;
+        S.H[it * kLd + it] = rnorm;
+        S.g[it] = rc;
+        S.g[nv] = rn;
+        S.Tm[nv * kLd + nv] = inv;
+        s_inv = inv;
+        s_on = on ? 1 : 0;
+      }
+    }
+    __syncthreads();
+    ++it;
+    if (!s_on) break;
+  }
+  // back substitution (operators.py:902-917) and Wc = Tm coeff, so that
+  // x += sum_j coeff_j v_j = sum_i Wc_i Z_i
+  if (wave == 0) {
+    T num = lane < it ? S.g[lane] : T(0);
+    for (int row = it - 1; row >= 0; --row) {
+      const T d = S.H[row * kLd + row];
+      if (lane == row) S.Gv[row] = num / (absv(d) > eps ? d : T(1));
+      wave_sync();
+      if (lane < row) num -= S.H[lane * kLd + row] * S.Gv[row];
+    }
+    wave_sync();
+    if (lane < it) {
+      T s = T(0);
+#pragma unroll 8
+      for (int j = lane; j < it; ++j) s += S.Tm[lane * kLd + j] * S.Gv[j];
+      S.Wc[lane] = s;
+    }
+  }
+  __syncthreads();
+  int fin = 1;
+  for (int e = tid; e < W; e += BS) {
+    T s = T(0);
+#pragma unroll 8
+    for (int i = 0; i < it; ++i) s += S.Wc[i] * Z[(int64_t)i * ld + e];
+    const T x = X[e] + s;
+    X[e] = x;
+    if (!finite(x)) fin = 0;
+  }
+  __syncthreads();
+  // the candidate's residual r = g - A x (operators.py:1084-1091); the basis is free
+  apply<T, BS, DG>(A, b, X, T(1), Z, u, w);
+  T big = T(0);
+  for (int e = tid; e < W; e += BS) {
+    const T r = G[e] - Z[e];
+    Rr[e] = r;
+    big = maxp(big, absv(r));
+  }
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) {
+    big = maxp(big, __shfl_xor(big, h));
+    fin &= __shfl_xor(fin, h);
+  }
+  if (lane == 0) {
+    red[wave * kLd] = big;
+    red[wave * kLd + 1] = fin ? T(1) : T(0);
+  }
+  __syncthreads();
+  if (tid == 0) {
+#pragma unroll
+    for (int k = 1; k < NW; ++k) {
+      big = maxp(big, red[k * kLd]);
+      fin &= red[k * kLd + 1] != T(0) ? 1 : 0;
+    }
+    A.rinf[b] = big;
+    A.xfin[b] = fin ? T(1) : T(0);
+    A.total[b] += it;
+    atomicMax(&A.ctrl[c], it);
+  }
+}
+
+constexpr size_t kLdsMax = 160 * 1024;
+
+template <typename T, int BS, bool DG, bool ZL>
+int launch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base, int64_t max_it) {
+  const size_t lds = lds_elems(A.n, A.m, A.W, A.restart, BS, ZL) * sizeof(T);
+  if (int rc = raise_lds_cap((const void*)k_gmr_cycle<T, BS, DG, ZL>, lds)) return rc;
+  k_gmr_cycle<T, BS, DG, ZL><<<(unsigned)batch, BS, lds, st>>>(A, c, base, max_it);
+  return PURIN_CP_OK;
+}
+
+template <typename T, bool DG>
+int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base, int64_t max_it) {
+  // Small problems keep the basis in LDS too (half the LDS, so that two workgroups
+  // share a CU), with 4 wavefronts, the smallest (two elements a lane) with one:
+  // 20,000 samples of W = 38 took 2.5 ms with four.
+  if (A.W <= 128) return launch<T, 64, DG, true>(st, A, batch, c, base, max_it);
+  if (lds_elems(A.n, A.m, A.W, A.restart, 256, true) * sizeof(T) <= kLdsMax / 2)
+    return launch<T, 256, DG, true>(st, A, batch, c, base, max_it);
+  if (A.W <= 512) return launch<T, 256, DG, false>(st, A, batch, c, base, max_it);
+  return launch<T, 512, DG, false>(st, A, batch, c, base, max_it);
+}
+
+}  // namespace
+
+bool gmr_fits(const purin_cp_plan* p, int64_t restart) {
+  return p->sl_ok && restart <= kGmrRestart &&
+         lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 <= kLdsMax;
+}
+
+template <typename T>
+int gmr_cycle(hipStream_t st, const Gmr<T>& A, int64_t batch, bool dg, int c, int64_t base,
+              int64_t max_iterations) {
+  return dg ? dispatch<T, true>(st, A, batch, c, base, max_iterations)
+            : dispatch<T, false>(st, A, batch, c, base, max_iterations);
+}
+
+template int gmr_cycle<double>(hipStream_t, const Gmr<double>&, int64_t, bool, int, int64_t, int64_t);
+template int gmr_cycle<float>(hipStream_t, const Gmr<float>&, int64_t, bool, int, int64_t, int64_t);
+
+}  // namespace purin

@@ -1003,6 +1003,62 @@ static int build(purin_cp_plan* p, const int64_t* indptr, const int32_t* indices
   UP(p->bptr, bptr);
   UP(p->brow, brow32);
   UP(p->dbcoef, bcoefT);
+  // --- sliced rows and columns (16-bit positions) ------------------------------
+  p->sl_ok = n < 65535 && m < 65535;
+  if (p->sl_ok) {
+    auto by_degree = [](int64_t count, const std::vector<int32_t>& ptr) {
+      std::vector<int32_t> order(count);
+      for (int64_t i = 0; i < count; ++i) order[i] = (int32_t)i;
+      std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+        return ptr[a + 1] - ptr[a] > ptr[b + 1] - ptr[b];
+      });
+      return order;
+    };
+    const std::vector<int32_t> rperm = by_degree(m, H.ptr), cperm = by_degree(n, H.cptr);
+    std::vector<int32_t> rpos(m), cpos(n);
+    for (int64_t k = 0; k < m; ++k) rpos[rperm[k]] = (int32_t)k;
+    for (int64_t k = 0; k < n; ++k) cpos[cperm[k]] = (int32_t)k;
+    auto slice = [&](int64_t count, const std::vector<int32_t>& perm, const std::vector<int32_t>& ptr,
+                     const std::vector<int32_t>& idx, const std::vector<T>& val,
+                     const std::vector<int32_t>& pos, int64_t pad, std::vector<int32_t>& off,
+                     std::vector<uint16_t>& sidx, std::vector<T>& sval, std::vector<int32_t>& ssrc) {
+      off.assign(1, 0);
+      for (int64_t s0 = 0; s0 < count; s0 += 64) {
+        const int64_t width = ptr[perm[s0] + 1] - ptr[perm[s0]];  // the slice's widest
+        const size_t at = sidx.size();
+        sidx.resize(at + width * 64, (uint16_t)pad);
+        sval.resize(at + width * 64, T(0));
+        ssrc.resize(at + width * 64, -1);
+        for (int64_t l = 0; l < 64 && s0 + l < count; ++l)
+          for (int32_t k = ptr[perm[s0 + l]]; k < ptr[perm[s0 + l] + 1]; ++k) {
+            const size_t e = at + (size_t)(k - ptr[perm[s0 + l]]) * 64 + l;
+            sidx[e] = (uint16_t)pos[idx[k]];
+            sval[e] = val[k];
+            ssrc[e] = k;
+          }
+        off.push_back((int32_t)sidx.size());
+      }
+    };
+    std::vector<int32_t> roff, coff, rsrc, csrc;
+    std::vector<uint16_t> sridx, scidx;
+    std::vector<T> srval, scval;
+    slice(m, rperm, H.ptr, H.idx, H.val_s, cpos, n, roff, sridx, srval, rsrc);
+    slice(n, cperm, H.cptr, H.cidx, H.cval_s, rpos, m, coff, scidx, scval, csrc);
+    p->sl_nsr = (int32_t)roff.size() - 1;
+    p->sl_nsc = (int32_t)coff.size() - 1;
+    p->sl_rn = (int64_t)sridx.size();
+    p->sl_cn = (int64_t)scidx.size();
+    UP(p->sl_rperm, rperm);
+    UP(p->sl_cperm, cperm);
+    UP(p->sl_roff, roff);
+    UP(p->sl_coff, coff);
+    UP(p->sl_ridx, sridx);
+    UP(p->sl_cidx, scidx);
+    UP(p->sl_rval, srval);
+    UP(p->sl_cval, scval);
+    UP(p->sl_rsrc, rsrc);
+    UP(p->sl_csrc, csrc);
+  }
 #undef UP
   return PURIN_CP_OK;
 }

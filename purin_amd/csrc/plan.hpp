@@ -107,6 +107,23 @@ struct purin_cp_plan {
   hipStream_t upload = nullptr;      // the plan's own stream for schedule uploads
   std::mutex mu;                     // guards the schedule, timing, adjoint stats and steps
 
+  // sliced rows and columns of the scaled kept matrix (the adjoint's per-sample
+  // kernels): positions in decreasing degree, 64 to a slice, each slice's entries
+  // in [entry][lane] order padded to its widest row / column (index n / m, value 0)
+  bool sl_ok = false;
+  int32_t sl_nsr = 0, sl_nsc = 0;    // slices
+  int64_t sl_rn = 0, sl_cn = 0;      // entries, padding included
+  int32_t* sl_rperm = nullptr;       // m: kept row of each position
+  int32_t* sl_cperm = nullptr;       // n: column of each position
+  int32_t* sl_roff = nullptr;        // nsr + 1 / nsc + 1: first entry of each slice
+  int32_t* sl_coff = nullptr;
+  uint16_t* sl_ridx = nullptr;       // column position / row position of each entry
+  uint16_t* sl_cidx = nullptr;
+  void* sl_rval = nullptr;           // scaled coefficients
+  void* sl_cval = nullptr;
+  int32_t* sl_rsrc = nullptr;        // kept CSR / CSC entry, or -1 (padding)
+  int32_t* sl_csrc = nullptr;
+
   int device = 0;             // the device the plan was created on (its buffers live there)
 
   std::vector<void*> owned;   // device allocations freed with the plan

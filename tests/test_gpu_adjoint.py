@@ -263,3 +263,47 @@ def test_vjp_restart_lengths(dtype, restart):
     else:
         assert rel_err(to_np(adj.g_target), want.g_target) <= 1e-4
         assert rel_err(to_np(adj.g_rhs), want.g_rhs) <= 1e-4
+
+
+@pytest.mark.parametrize("n,me,mi,width,B,restart,dtype", [
+    (3, 1, 1, 2, 1, 30, np.float64),       # W = 8: the restart length is cut to W
+    (40, 0, 0, 2, 65, 30, np.float64),     # no rows
+    (58, 4, 8, 3, 5, 30, np.float64),      # W = 128: the last with one wavefront
+    (58, 4, 9, 3, 5, 30, np.float64),      # W = 129: four
+    (130, 20, 44, 4, 3, 30, np.float64),   # basis in LDS, more than one slice of rows and columns
+    (215, 20, 62, 4, 3, 30, np.float64),   # W = 512: the last with four wavefronts
+    (215, 20, 63, 4, 66, 30, np.float64),  # W = 513: eight
+    (700, 65, 130, 5, 4, 32, np.float64),  # the longest restart of the per-sample cycles
+    (60, 10, 20, 4, 5, 33, np.float64),    # the batch-minor passes
+    (300, 40, 90, 5, 7, 30, np.float32),
+])
+def test_vjp_gmres_dispatch_edges(n, me, mi, width, B, restart, dtype):
+    """The per-sample GMRES cycles at the edges of their workgroup sizes, slices and
+    restart lengths, against the oracle at the same saved state (the bars of
+    test_vjp_matches_oracle_at_the_same_state; a sample whose GMRES does not reach
+    1e-14 is fixed only to its residual, and is left out)."""
+    from oracle import adjoint as oadj
+
+    if me + mi:
+        w = workloads.small_random(51, n=n, me=me, mi=mi, width=width, batch=B)
+        canon, rhs = canonical_from_workload(w), np.tile(w.rhs, (B, 1)).astype(dtype)
+        target = w.target.astype(dtype)
+    else:
+        canon = op.Canonical(n=n, me=0, rows=[[j] for j in range(n)], coef=[[1.0]] * n)
+        rhs = np.ones((B, n), dtype)
+        target = np.random.default_rng(3).normal(0.0, 2.0, (B, n)).astype(dtype)
+    cot = np.random.default_rng(17).normal(size=(B, n)).astype(dtype)
+    gtol = 1e-14 if dtype == np.float64 else 1e-5
+    cfg = op.Config(max_iterations=400, early_stop=False, gmres_tolerance=gtol,
+                    gmres_restart=restart, gmres_max_iterations=400)
+    plan, pre, o, saved = _solve_state(canon, target, rhs, cfg, dtype)
+    ksup, kmask = pre.support[pre.rows], pre.mask[pre.rows]
+    want = oadj.adjoint(pre.kept_values[0], ksup, kmask, canon.me, to_np(o.y), to_np(o.dual),
+                        np.ones(B, bool), target, pre.kept_rhs, pre.lower, pre.upper, cot, cfg)
+    adj = plan.adjoint(saved, target, pre.kept_rhs, cot, force_eligible=True, rhs_rows=plan.m,
+                       tolerance=gtol, restart=restart, max_iterations=400)
+    conv = (want.info == 0) & (to_np(adj.info) == 0)
+    assert conv.sum() >= (B + 1) // 2
+    bar = 1e-10 if dtype == np.float64 else 1e-4
+    assert rel_err(to_np(adj.g_target)[conv], want.g_target[conv]) <= bar
+    assert rel_err(to_np(adj.g_rhs)[conv], want.g_rhs[conv]) <= bar
