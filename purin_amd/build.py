@@ -22,7 +22,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(os.path.dirname(HERE), "_build")
 LIB = os.path.join(HERE, "libpurin_cp.so")
-SOURCES = ["plan.hip", "forward.hip", "adjoint.hip", "gmres.hip"]
+SOURCES = ["plan.hip", "forward.hip", "adjoint.hip", "gmres.hip", "solo.hip"]
 RESIDENT_SOURCE = "resident_launch.hip"
 RESIDENT_VARIANTS = [(f64, slr) for f64 in (1, 0) for slr in (1, 2, 3, 4)]
 PROBE_LIB = os.path.join(HERE, "libpurin_probe.so")

@@ -20,6 +20,7 @@
 #include "post.hpp"
 #include "forward.hpp"
 #include "resident.hpp"
+#include "solo.hpp"
 #include "persample.hpp"
 
 namespace purin {
@@ -285,6 +286,79 @@ static size_t resident_lds(const purin_cp_plan* p, bool early = false) {
   return lds <= 160 * 1024 ? lds : 0;
 }
 
+// The launch check and, with timing, the launch's time (e0 was recorded before it).
+static int finish_resident(purin_cp_plan* p, hipStream_t st, const purin_cp_solve_options& o,
+                           hipEvent_t e0, hipEvent_t e1) {
+  PURIN_HIP(hipGetLastError());
+  if (!o.timing) return PURIN_CP_OK;
+  PURIN_HIP(hipEventRecord(e1, st));
+  PURIN_HIP(hipEventSynchronize(e1));
+  float ms = 0;
+  PURIN_HIP(hipEventElapsedTime(&ms, e0, e1));
+  purin_cp_timing t{};
+  t.iterations = o.max_iterations;
+  t.loop_ms = ms;
+  t.resident = 1;
+  record_timing(p, t);
+  (void)hipEventDestroy(e0);
+  (void)hipEventDestroy(e1);
+  return PURIN_CP_OK;
+}
+
+// The CP loop with one workgroup per sample (solo.hip); the arguments of run_resident.
+template <typename T>
+static int run_solo(purin_cp_plan* p, hipStream_t st, const Layout& L, char* sv,
+                    const purin_cp_solve_options& o, bool early, int64_t batch, T tol,
+                    const T* tolv, int32_t* done, int32_t* count, const void* sched,
+                    const QPRun<T>* qp, const PerSample<T>* ps) {
+  Solo<T> A{};
+  A.n = (int)p->n;
+  A.m = (int)p->m;
+  A.me = (int)p->me;
+  A.Bp = L.Bp;
+  A.batch = batch;
+  A.iters = o.max_iterations;
+  A.nsr = p->sl_nsr;
+  A.nsc = p->sl_nsc;
+  A.roff = p->sl_roff;
+  A.coff = p->sl_coff;
+  A.rperm = p->sl_rperm;
+  A.cperm = p->sl_cperm;
+  A.ridx = p->sl_ridx;
+  A.cidx = p->sl_cidx;
+  A.rsrc = p->sl_rsrc;
+  A.csrc = p->sl_csrc;
+  if (ps && ps->RVs) {
+    A.RV = ps->RVs;
+    A.CV = ps->CVs;
+    A.vbp = 1;
+  } else if (ps) {
+    A.RV = ps->RV;
+    A.CV = ps->CV;
+    A.vbp = L.Bp;
+  } else {
+    A.rval = (const T*)p->sl_rval;
+    A.cval = (const T*)p->sl_cval;
+  }
+  A.tgt = qp ? qp->Cc : (const T*)(sv + L.Tt);
+  A.Q = qp ? qp->Q : nullptr;
+  A.R = (const T*)(sv + L.R);
+  A.LO = (const T*)(sv + L.LO);
+  A.HI = (const T*)(sv + L.HI);
+  A.shared_bounds = o.shared_bounds;
+  A.sched = (const T*)sched;
+  A.step0 = ps ? ps->tau_b : nullptr;  // [5][Bp]: tau, sigma, a, delta, theta
+  A.gam = qp && p->opts.accelerated ? qp->gamma : nullptr;
+  A.accel = p->opts.accelerated;
+  A.tol = tol;
+  A.tolv = tolv;
+  A.done = done;
+  A.count = count;
+  A.Y = (T*)(sv + L.Y);
+  A.D = (T*)(sv + L.D);
+  return solo_launch<T>(st, p, A, qp ? kSoloQP : (ps ? kSoloValues : kSoloShared), early);
+}
+
 // The CP loop on the resident kernel; fills Y and D like the passes (and, with
 // early stop, the per-sample done flags and iteration counts).  qp (with ps):
 // the diagonal QP, q and c per sample, y0 from Y, the per-sample steps of ps.
@@ -309,6 +383,18 @@ static int run_resident(purin_cp_plan* p, hipStream_t st, const Layout& L, char*
   const void* sched = p->res_sched;  // per-sample steps (QP, coefficients) instead
   if (!ps)
     if (int rc = ensure_schedule(p, o.max_iterations, st, false, &sched)) return rc;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  const bool solo = solo_fits(p, batch, early, ps && !ps->RVs);
+  if (solo) {
+    if (o.timing) {
+      PURIN_HIP(hipEventCreate(&e0));
+      PURIN_HIP(hipEventCreate(&e1));
+      PURIN_HIP(hipEventRecord(e0, st));
+    }
+    if (int rc = run_solo<T>(p, st, L, sv, o, early, batch, tol, tolv, done, count, sched, qp, ps))
+      return rc;
+    return finish_resident(p, st, o, e0, e1);
+  }
   Res<T> R{};
   R.n = (int)p->n;
   R.m = (int)p->m;
@@ -393,7 +479,6 @@ static int run_resident(purin_cp_plan* p, hipStream_t st, const Layout& L, char*
   R.iters = o.max_iterations;
   R.Y = (T*)(sv + L.Y);
   R.D = (T*)(sv + L.D);
-  hipEvent_t e0 = nullptr, e1 = nullptr;
   if (o.timing) {
     PURIN_HIP(hipEventCreate(&e0));
     PURIN_HIP(hipEventCreate(&e1));
@@ -419,21 +504,7 @@ static int run_resident(purin_cp_plan* p, hipStream_t st, const Layout& L, char*
                                   o.shared_bounds != 0, early, BT,
                                   qp ? (ps->RVs ? 1 : 3) : (ps ? 2 : 0)))
     return rc;
-  PURIN_HIP(hipGetLastError());
-  if (o.timing) {
-    PURIN_HIP(hipEventRecord(e1, st));
-    PURIN_HIP(hipEventSynchronize(e1));
-    float ms = 0;
-    PURIN_HIP(hipEventElapsedTime(&ms, e0, e1));
-    purin_cp_timing t{};
-    t.iterations = o.max_iterations;
-    t.loop_ms = ms;
-    t.resident = 1;
-    record_timing(p, t);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-  }
-  return PURIN_CP_OK;
+  return finish_resident(p, st, o, e0, e1);
 }
 
 // The CP loop on prepared internal arrays plus the final diagnostics.

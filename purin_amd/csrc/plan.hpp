@@ -112,6 +112,7 @@ struct purin_cp_plan {
   // in [entry][lane] order padded to its widest row / column (index n / m, value 0)
   bool sl_ok = false;
   int32_t sl_nsr = 0, sl_nsc = 0;    // slices
+  std::vector<int32_t> sl_rw, sl_cw; // entries per lane of each slice (decreasing)
   int64_t sl_rn = 0, sl_cn = 0;      // entries, padding included
   int32_t* sl_rperm = nullptr;       // m: kept row of each position
   int32_t* sl_cperm = nullptr;       // n: column of each position

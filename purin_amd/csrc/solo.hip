@@ -1,0 +1,551 @@
+// CP loop for small problems and batches: one workgroup per sample, one thread per
+// row and per column, the thread's matrix entries in registers.
+//
+// The tile kernels of resident.hpp stream the shared matrix from L2 every iteration
+// through 16 wavefronts whatever the problem's size, so below a few hundred
+// thousand entries of work an iteration is latency: L2 loads, three barriers of 16
+// wavefronts and a decision phase, 2.3-2.9 us.  Here
+//   * the workgroup has as many wavefronts as the problem's rows or columns fill,
+//     so small batches use more of the chip and small problems wait for less;
+//   * a thread's first W entries of its row and of its column are in registers,
+//     the rest (the widest slices only) in LDS, so an iteration touches no memory
+//     beyond LDS: gather, sum, update, two barriers;
+//   * the stop test trails the loop: a wavefront of its own sums and judges iteration
+//     k's terms while the others run iteration k + 1, so the test is not on the path of
+//     the iterates.  The state of two iterations back is kept, and a sample accepted at
+//     k returns exactly that state and count.  (With all 16 wavefronts taken by rows or
+//     columns each reduces its own terms and the last one judges.)
+// One iteration (kernels.py:91-150): the column pass gathers d+, forms y+ and its
+// diagnostics; the row pass gathers y+: K y+, the residual, and the next d+ from
+// K ybar = (1 + theta) K y+ - theta K y (resident.hpp, k_resident_early).  Without the
+// stop test the passes are k_resident's.
+#include <algorithm>
+#include <type_traits>
+
+#include "solo.hpp"
+
+#include "resident.hpp"
+
+namespace purin {
+
+namespace {
+
+constexpr int kSoloMax = 1024;  // rows / columns: one thread each
+constexpr int kSoloW = 8;       // matrix entries of a row and of a column in registers
+
+// sum over N register entries: coefficient times the LDS element at its byte offset
+template <int N, typename T, int W>
+__device__ __forceinline__ T dot_regs(const T (&v)[W], const uint32_t (&ix)[W / 2],
+                                      const unsigned char* lds) {
+  T x[N], acc = T(0);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const uint32_t off = (k & 1) ? ix[k / 2] >> 16 : ix[k / 2] & 0xffffu;
+    x[k] = *reinterpret_cast<const T*>(lds + off);
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) acc = __builtin_elementwise_fma(v[k], x[k], acc);
+  return acc;
+}
+
+// A slice's sum: groups of 4 entries in registers (the count is the wavefront's),
+// then the entries past W from LDS.
+template <typename T, int W>
+__device__ __forceinline__ T slice_sum(const T (&v)[W], const uint32_t (&ix)[W / 2], int groups,
+                                       const unsigned char* lds, const T* rv, const uint16_t* ri,
+                                       int rest) {
+  T acc = groups <= 1 ? dot_regs<4>(v, ix, lds) : dot_regs<8>(v, ix, lds);
+  for (int k = 0; k < rest; ++k)
+    acc = __builtin_elementwise_fma(rv[k * 64], *reinterpret_cast<const T*>(lds + ri[k * 64]), acc);
+  return acc;
+}
+
+// [a's sum over the wavefront in lanes 0-31, b's in lanes 32-63]
+template <typename T>
+__device__ __forceinline__ T two_sums(T a, T b) {
+  constexpr int N = sizeof(T) / 4;
+  typedef uint32_t U __attribute__((ext_vector_type(N)));
+  U x = __builtin_bit_cast(U, a), y = __builtin_bit_cast(U, b);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false);
+    x[i] = r[0];
+    y[i] = r[1];
+  }
+  T v = __builtin_bit_cast(T, x) + __builtin_bit_cast(T, y);
+  x = y = __builtin_bit_cast(U, v);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+    x[i] = r[0];
+    y[i] = r[1];
+  }
+  v = __builtin_bit_cast(T, x) + __builtin_bit_cast(T, y);
+  return row16_combine(v, OpAdd());
+}
+
+template <typename T>
+__device__ __forceinline__ T wave_fmax(T a) {
+  constexpr int N = sizeof(T) / 4;
+  typedef uint32_t U __attribute__((ext_vector_type(N)));
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    U x = __builtin_bit_cast(U, a), y = x;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const auto r = h == 0 ? __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false)
+                            : __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+      x[i] = r[0];
+      y[i] = r[1];
+    }
+    a = __builtin_fmax(__builtin_bit_cast(T, x), __builtin_bit_cast(T, y));
+  }
+  return row16_combine(a, OpFMax());
+}
+
+// Entries past the first W of every slice, in LDS.
+__host__ __device__ inline int rest_of(int width, int W) { return width > W ? width - W : 0; }
+
+// Up to 1024 threads, so up to 128 VGPRs.
+// HELP: the workgroup has one wavefront more than its rows or columns fill, for the stop test.
+template <typename T, int W, int MODE, bool EARLY, bool HELP>
+__global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int NW = (blockDim.x >> 6) - (HELP ? 1 : 0);  // wavefronts of rows and columns
+  const int NT = NW * 64;
+  const int64_t b = blockIdx.x, Bp = A.Bp;
+  const int n = A.n, m = A.m;
+  const int j = t < n ? A.cperm[t] : -1, i = t < m ? A.rperm[t] : -1;
+  if (b >= A.batch) {  // padding samples: zero state (the whole workgroup)
+    if (j >= 0) A.Y[(int64_t)j * Bp + b] = T(0);
+    if (i >= 0) A.D[(int64_t)i * Bp + b] = T(0);
+    return;
+  }
+  constexpr bool QP = MODE == kSoloQP, PS = MODE != kSoloShared;
+  const T zero = T(0), half = T(0.5), inf = T(__builtin_inf());
+  // LDS: Gy [n] | zero | Gd [m] | zero | partials [16][4] or (HELP) [2][3][NT] | verdict |
+  // rest values | rest offsets
+  T* Gy = reinterpret_cast<T*>(lds);
+  T* Gd = Gy + n + 1;
+  T* red = Gd + m + 1;
+  T* fl = red + (HELP ? 6 * NT : 64);
+  volatile int* flag = reinterpret_cast<volatile int*>(fl);
+  T* restv = fl + 2;
+  int nrest = 0, rbase = 0, cbase = 0;
+  for (int s = 0; s < A.nsr; ++s) {
+    if (s == wave) rbase = nrest;
+    nrest += rest_of((A.roff[s + 1] - A.roff[s]) >> 6, W) * 64;
+  }
+  for (int s = 0; s < A.nsc; ++s) {
+    if (s == wave) cbase = nrest;
+    nrest += rest_of((A.coff[s + 1] - A.coff[s]) >> 6, W) * 64;
+  }
+  uint16_t* resti = reinterpret_cast<uint16_t*>(restv + nrest);
+  // this wavefront's slices
+  const bool has_r = wave < A.nsr, has_c = wave < A.nsc;
+  const int ro = has_r ? A.roff[wave] : 0, co = has_c ? A.coff[wave] : 0;
+  const int rw = has_r ? (A.roff[wave + 1] - ro) >> 6 : 0, cw = has_c ? (A.coff[wave + 1] - co) >> 6 : 0;
+  const int rgr = (rw < W ? rw + 3 : W) >> 2, cgr = (cw < W ? cw + 3 : W) >> 2;
+  const int rrest = rest_of(rw, W), crest = rest_of(cw, W);
+  T rv[W], cv[W];
+  uint32_t rx[W / 2], cx[W / 2];
+  const uint32_t zr = (uint32_t)n * sizeof(T), zc = (uint32_t)(n + 1 + m) * sizeof(T);
+  const uint32_t base_d = (uint32_t)(n + 1) * sizeof(T);
+  auto value = [&](const T* shared, const T* own, const int32_t* src, int e) -> T {
+    if (shared) return shared[e];
+    const int k = src[e];
+    return k < 0 ? T(0) : own[(int64_t)k * A.vbp + (A.vbp > 1 ? b : 0)];
+  };
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    const int er = ro + k * 64 + lane, ec = co + k * 64 + lane;
+    const bool okr = k < rw, okc = k < cw;
+    rv[k] = okr ? value(A.rval, A.RV, A.rsrc, er) : zero;
+    cv[k] = okc ? value(A.cval, A.CV, A.csrc, ec) : zero;
+    const uint32_t xr = okr ? (uint32_t)A.ridx[er] * (uint32_t)sizeof(T) : zr;
+    const uint32_t xc = okc ? base_d + (uint32_t)A.cidx[ec] * (uint32_t)sizeof(T) : zc;
+    if (k & 1) {
+      rx[k / 2] |= xr << 16;
+      cx[k / 2] |= xc << 16;
+    } else {
+      rx[k / 2] = xr;
+      cx[k / 2] = xc;
+    }
+  }
+  for (int k = 0; k < rrest; ++k) {
+    const int e = ro + (W + k) * 64 + lane;
+    restv[rbase + k * 64 + lane] = value(A.rval, A.RV, A.rsrc, e);
+    resti[rbase + k * 64 + lane] = (uint16_t)(A.ridx[e] * sizeof(T));
+  }
+  for (int k = 0; k < crest; ++k) {
+    const int e = co + (W + k) * 64 + lane;
+    restv[cbase + k * 64 + lane] = value(A.cval, A.CV, A.csrc, e);
+    resti[cbase + k * 64 + lane] = (uint16_t)(base_d + A.cidx[e] * sizeof(T));
+  }
+  const T* rrv = restv + rbase + lane;
+  const T* crv = restv + cbase + lane;
+  const uint16_t* rri = resti + rbase + lane;
+  const uint16_t* cri = resti + cbase + lane;
+  // the thread's column and row
+  const T tg = j >= 0 ? A.tgt[(int64_t)j * Bp + b] : zero;
+  const T lo = j >= 0 ? A.LO[A.shared_bounds ? j : (int64_t)j * Bp + b] : zero;
+  const T hi = j >= 0 ? A.HI[A.shared_bounds ? j : (int64_t)j * Bp + b] : zero;
+  const T q = QP ? (j >= 0 ? A.Q[(int64_t)j * Bp + b] : T(1)) : T(1);
+  const bool odd = lo != lo || hi != hi || lo > hi;  // a NaN or crossed bound
+  T y = QP ? (j >= 0 ? A.Y[(int64_t)j * Bp + b] : zero) : tg;  // y0 = ybar0
+  const T rr = i >= 0 ? A.R[(int64_t)i * Bp + b] : zero;
+  T d = i >= 0 ? A.D[(int64_t)i * Bp + b] : zero;
+  const bool ineq = i >= A.me;
+  // per-sample steps, the same in every thread
+  T tau = zero, sig = zero, th = T(1), gam = T(1), pa = zero, pd = zero;
+  if constexpr (PS) {
+    tau = res_uniform(A.step0[b]);
+    sig = res_uniform(A.step0[Bp + b]);
+    pa = res_uniform(A.step0[2 * Bp + b]);
+    pd = res_uniform(A.step0[3 * Bp + b]);
+    th = res_uniform(A.accel ? A.step0[4 * Bp + b] : T(1));
+    gam = res_uniform(A.gam ? A.gam[b] : T(1));
+  }
+  auto prox = [&]() {  // the general-q prox a, delta (kernels.py:68-73)
+    if constexpr (QP) {
+      pa = EARLY ? T(1) / (T(1) + tau * q) : res_recip(T(1) + tau * q);
+      pd = tau * pa;
+    }
+  };
+  auto advance = [&]() {  // the accelerated update (kernels.py:279-283)
+    if constexpr (PS) {
+      if (A.accel) {
+        T g1[1] = {gam}, t1[1] = {tau}, s1[1] = {sig}, h1[1] = {th}, a1[1], d1[1];
+        res_qp_schedule<T, 1>(g1, t1, s1, h1, a1, d1);
+        tau = t1[0];
+        sig = s1[0];
+        th = h1[0];
+        if constexpr (!QP) {
+          pa = a1[0];
+          pd = d1[0];
+        }
+        prox();
+      }
+    }
+  };
+  prox();
+  if (t < n) Gy[t] = y;
+  if (t < m) Gd[t] = d;
+  if (t == 0) {
+    Gy[n] = zero;
+    Gd[m] = zero;
+    *flag = 0;
+  }
+  __syncthreads();
+  typedef const __attribute__((address_space(4))) T* CP;
+  const CP sched = (CP)A.sched;
+
+  // s = a y - delta K^T d + delta yhat (or - delta c)
+  auto primal_step = [&](T tt, T a, T delta) -> T {
+    if constexpr (QP) {
+      const T o = -delta * tg;
+      return a * y - delta * tt + o;
+    } else {
+      return a * y - delta * tt + delta * tg;
+    }
+  };
+
+  if constexpr (!EARLY) {
+    // each iteration's scalars are loaded before the barrier that ends the previous one:
+    // a scalar load outstanding among the gathers would make their waits wait for it too
+    T f_sig = zero, f_a = zero, f_d = zero, f_th = zero;
+    auto load = [&](int64_t k) {
+      if constexpr (!PS) {
+        f_sig = sched[4 * k];
+        f_a = sched[4 * k + 1];
+        f_d = sched[4 * k + 2];
+        f_th = sched[4 * k + 3];
+        asm volatile("" : "+s"(f_sig), "+s"(f_a), "+s"(f_d), "+s"(f_th));
+      }
+    };
+    load(0);
+    for (int64_t it = 0; it < A.iters; ++it) {
+      const T sigma = PS ? sig : f_sig, a = PS ? pa : f_a, delta = PS ? pd : f_d,
+              theta = PS ? th : f_th;
+      if (has_r) {
+        const T acc = slice_sum<T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
+        T p = d + sigma * (acc - rr);
+        if (ineq) p = res_pos(p);
+        d = p;
+        if (t < m) Gd[t] = p;
+      }
+      __syncthreads();
+      if (has_c) {
+        const T tt = slice_sum<T, W>(cv, cx, cgr, lds, crv, cri, crest);
+        const T s = primal_step(tt, a, delta);
+        const T yn = odd ? clipp(s, lo, hi) : res_clip(s, lo, hi);
+        if (t < n) Gy[t] = yn + theta * (yn - y);
+        y = yn;
+      }
+      advance();
+      if (it + 1 < A.iters) load(it + 1);
+      __syncthreads();
+    }
+    if (j >= 0) A.Y[(int64_t)j * Bp + b] = y;
+    if (i >= 0) A.D[(int64_t)i * Bp + b] = d;
+    return;
+  }
+
+  // K y0 and the first d+
+  T ky = zero;
+  if (has_r) {
+    ky = slice_sum<T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
+    T p = d + (PS ? sig : sched[0]) * (ky - rr);
+    if (ineq) p = res_pos(p);
+    d = p;
+    if (t < m) Gd[t] = p;
+  }
+  __syncthreads();
+  const T tol = A.tolv ? A.tolv[b] : A.tol;
+  const T one = T(1);
+  auto judge = [&](T pri, T dual, T mx) -> bool {  // kernels.py:167-175, 260-278
+    const T gap = maxp(pri - dual, zero) / maxp(one, maxp(absv(pri), absv(dual)));
+    return finite(gap) && mx <= tol && gap <= tol;
+  };
+  if (HELP && wave == NW) {
+    for (int64_t it = 0;; ++it) {
+      if ((it >= 2 && __builtin_amdgcn_readfirstlane(*flag)) || it > A.iters) return;
+      T pri = zero, dual = zero, mx = inf;
+      if (it > 0) {
+        const T* pt = red + ((it - 1) & 1) * 3 * NT + lane;
+        mx = zero;
+        for (int w = 0; w < NW; ++w) {
+          pri += pt[w * 64];
+          dual += pt[NT + w * 64];
+          mx = __builtin_fmax(mx, pt[2 * NT + w * 64]);
+        }
+        const T s2 = two_sums(pri, dual);
+        pri = read_lane(s2, 0);
+        dual = read_lane(s2, 32);
+        mx = wave_fmax(mx);
+      }
+      __syncthreads();
+      const bool ok = judge(pri, dual, mx);
+      if (lane == 0) *flag = ok ? 1 : 0;
+      __syncthreads();
+    }
+  }
+  // the scalars of this iteration and the next sigma, loaded as in the loop above
+  T f_a = zero, f_d = zero, f_th = zero, f_sn = zero;
+  auto load = [&](int64_t k) {
+    if constexpr (!PS) {
+      const int64_t c = k < A.iters ? k : A.iters - 1, s = k + 1 < A.iters ? k + 1 : A.iters - 1;
+      f_a = sched[4 * c + 1];
+      f_d = sched[4 * c + 2];
+      f_th = sched[4 * c + 3];
+      f_sn = sched[4 * s];
+      asm volatile("" : "+s"(f_a), "+s"(f_d), "+s"(f_th), "+s"(f_sn));
+    }
+  };
+  load(0);
+  T yp = y, dk = d, dkp = d;           // y and d+ one iteration back, d+ two back
+  T q_pri = zero, q_dual = zero, q_max = inf;  // the last iteration's partials
+  int64_t it = 0;
+  bool accepted = false;
+  for (;; ++it) {
+    if (it >= 2 && __builtin_amdgcn_readfirstlane(*flag)) {  // the verdict on iteration it - 2
+      accepted = true;
+      break;
+    }
+    if (it > A.iters) break;  // one pass beyond the last judges the last
+    const bool run = it < A.iters;
+    const T r_pri = q_pri, r_dual = q_dual, r_max = q_max;
+    yp = y;
+    // ---- column pass, and the previous iteration's partials over the wavefront
+    q_pri = q_dual = q_max = zero;
+    if (run && has_c) {
+      const T a = PS ? pa : f_a, delta = PS ? pd : f_d;
+      const T tt = slice_sum<T, W>(cv, cx, cgr, lds, crv, cri, crest);
+      const T s = primal_step(tt, a, delta);
+      const T yn = odd ? clipp(s, lo, hi) : res_clip(s, lo, hi);
+      y = yn;
+      if (t < n) {
+        Gy[t] = yn;
+        if constexpr (QP) {  // general q, c (kernels.py:158-174, 272-274)
+          q_pri = half * q * yn * yn + tg * yn;
+          const T tf = tg + tt;
+          const T mz = q > T(1e-12) ? clipp(-tf / q, lo, hi) : (tf >= zero ? lo : hi);
+          q_dual = half * q * (mz * mz) + tf * mz;
+          T g = maxp(absv(yn - clipp(yn - ((q * yn + tg) + tt), lo, hi)),
+                     maxp(maxp(lo - yn, zero), maxp(yn - hi, zero)));
+          if (!finite(g)) g = inf;
+          q_max = g;
+        } else if (!odd) {  // q = 1, c = -yhat; see k_resident_early
+          const T cq = -tg;
+          q_pri = half * yn * yn + cq * yn;
+          const T tf = cq + tt;
+          const T mz = __builtin_fmin(__builtin_fmax(-tf, lo), hi);
+          q_dual = half * mz * mz + tf * mz;
+          q_max = __builtin_fmax(zero, absv(yn - mz));
+        } else {
+          const T cq = -tg;
+          q_pri = half * yn * yn + cq * yn;
+          const T tf = cq + tt;
+          const T mz = clipp(-tf, lo, hi);
+          q_dual = half * mz * mz + tf * mz;
+          const T xs = yn - ((yn + cq) + tt);
+          T g = maxp(absv(yn - clipp(xs, lo, hi)),
+                     maxp(maxp(lo - yn, zero), maxp(yn - hi, zero)));
+          if (!finite(g)) g = inf;
+          q_max = g;
+        }
+      }
+    }
+    if constexpr (!HELP) {
+      const T s2 = two_sums(r_pri, r_dual);
+      const T mx = wave_fmax(r_max);
+      if ((lane & 31) == 0) red[wave * 4 + (lane >> 5)] = s2;
+      if (lane == 0) red[wave * 4 + 2] = mx;
+    }
+    __syncthreads();
+    // ---- row pass, and the last wavefront's verdict on iteration it - 1
+    dkp = dk;
+    dk = d;
+    const bool more = it + 1 < A.iters;
+    const T theta = PS ? th : f_th;  // this iteration's; the steps then advance to the next
+    if (PS && run) advance();
+    if (run && has_r) {
+      const T sigma_n = PS ? sig : f_sn;
+      const T acc = slice_sum<T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
+      if (t < m) {  // kernels.py:158-166; d * 0 is NaN for a non-finite d
+        const T e = acc - rr, w = ineq ? zero : T(-1);
+        q_max = __builtin_fmax(q_max, __builtin_fmax(e, w * e));
+        q_dual = (q_dual - rr * d) - d * zero;
+      }
+      if (more) {
+        T p = d + sigma_n * (((T(1) + theta) * acc - theta * ky) - rr);
+        if (ineq) p = res_pos(p);
+        d = p;
+        if (t < m) Gd[t] = p;
+      }
+      ky = acc;
+    }
+    if constexpr (HELP) {
+      T* pt = red + (it & 1) * 3 * NT + t;
+      pt[0] = q_pri;
+      pt[NT] = q_dual;
+      pt[2 * NT] = q_max;
+    } else if (wave == NW - 1) {
+      const T* rl = red + (lane & 15) * 4;
+      const bool in = (lane & 15) < NW;
+      const T xp = row16_combine(in ? rl[0] : zero, OpAdd());
+      const T xd = row16_combine(in ? rl[1] : zero, OpAdd());
+      const T mx = row16_combine(in ? rl[2] : zero, OpFMax());
+      const bool ok = it > 0 && judge(xp, xd, mx);
+      if (lane == 0) *flag = ok ? 1 : 0;
+    }
+    load(it + 1);
+    __syncthreads();
+  }
+  // accepted at iteration it - 2: its y and d+ are the ones of one iteration back
+  if (accepted) {
+    y = yp;
+    dk = dkp;
+  }
+  if (j >= 0) A.Y[(int64_t)j * Bp + b] = y;
+  if (i >= 0) A.D[(int64_t)i * Bp + b] = dk;
+  if (t == 0) {
+    A.count[b] = (int32_t)(accepted ? it - 1 : A.iters);
+    A.done[b] = accepted ? 1 : 0;
+  }
+}
+
+int rest_entries(const purin_cp_plan* p, int W) {
+  int k = 0;
+  for (int w : p->sl_rw) k += rest_of(w, W) * 64;
+  for (int w : p->sl_cw) k += rest_of(w, W) * 64;
+  return k;
+}
+
+int solo_waves(const purin_cp_plan* p) { return std::max(p->sl_nsr, p->sl_nsc); }
+
+int cu_count(const purin_cp_plan* p) {
+  int cus = 0;
+  return hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) == hipSuccess
+             ? cus
+             : 256;
+}
+
+// The workgroup: wavefronts of rows and columns (with idle ones) and whether one more
+// runs the stop test.
+struct SoloBlock {
+  int waves;
+  bool help;
+};
+
+// A CU holds 16 wavefronts of these kernels (fp64).  The wavefront of the stop test pays
+// wherever it costs no workgroup per CU, and in a launch of one round: us per iteration at
+// B = 256 without / with it 1.32 / 0.71 (n = 60), 1.25 / 1.03 (n = 500), 1.68 / 1.4 (n =
+// 950), at B = 8192 10.9 / 18.7 with four wavefronts (four workgroups per CU against three),
+// 23.7 / 30.3 with eight (two against one).  Five to seven become eight, which
+// spreads over the four SIMDs alike: six (n = 310) took 31 us at B = 8192, eight 18.5.
+SoloBlock solo_block(const purin_cp_plan* p, int64_t batch, bool early) {
+  const int w = solo_waves(p);
+  if (!early) return {w > 4 && w < 8 ? 8 : w, false};
+  if (w > 15) return {w, false};
+  const int64_t cus = cu_count(p);
+  if ((w == 4 && batch > 2 * cus) || (w == 8 && batch > cus)) return {w, false};
+  return {w > 3 && w < 8 ? 7 : w, true};
+}
+
+// LDS of the larger of the two loops (with the stop test)
+size_t solo_lds(const purin_cp_plan* p, SoloBlock k) {
+  const size_t es = elem_size(p);
+  const size_t parts = k.help ? 6 * 64 * (size_t)k.waves : 64;
+  return (size_t)(p->n + 1 + p->m + 1 + parts + 2) * es + (size_t)rest_entries(p, kSoloW) * (es + 2);
+}
+
+template <typename T, int MODE>
+int launch_mode(hipStream_t st, const Solo<T>& A, SoloBlock k, size_t lds, bool early) {
+  auto kern = !early ? k_solo<T, kSoloW, MODE, false, false>
+                     : (k.help ? k_solo<T, kSoloW, MODE, true, true>
+                               : k_solo<T, kSoloW, MODE, true, false>);
+  if (int rc = raise_lds_cap((const void*)kern, lds)) return rc;
+  kern<<<(unsigned)A.Bp, 64u * (unsigned)(k.waves + (k.help ? 1 : 0)), lds, st>>>(A);
+  return PURIN_CP_OK;
+}
+
+}  // namespace
+
+// Against the tile kernels (two fp64 or eight fp32 samples per workgroup, one workgroup per
+// CU), us per iteration with the stop test / without:
+//   fp64  n = 60, B = 256: 0.71 / 0.37 (tile 2.09 / 0.67); n = 500, B = 8192: 23.7 / 9.3
+//         (37.9 / 13.5); n = 800: 38.1 / 17.0 (39.3 / 14.1); n = 1020: 49.0 / 19.6 (40.8 / 16.7)
+//   fp32  n = 250, B = 8192: 6.5 / 2.5 (16.1 / 4.3); n = 500: 13.5 / 6.4 (16.4 / 4.6);
+//         n = 800: 32.3 / 15.5 (17.7 / 4.7), B = 512: 2.0 / 1.0 (4.2 / 1.2)
+// so a sample per workgroup while its wavefronts leave a CU at least two of them, and above
+// that for the batches of the first rounds.  Per-sample coefficients stay in registers
+// here and stream from HBM there, whatever the batch.
+bool solo_fits(const purin_cp_plan* p, int64_t batch, bool early, bool values) {
+  if (!p->sl_ok || p->n > kSoloMax || p->m > kSoloMax) return false;
+  if (solo_lds(p, solo_block(p, batch, early)) > 160 * 1024) return false;
+  const int w = solo_waves(p);
+  const int64_t cus = cu_count(p);
+  if (values || w <= 4) return true;
+  if (p->dtype == PURIN_CP_F64) return early ? (w <= 13 || batch <= cus) : (w <= 8 || batch <= cus);
+  if (early) return w <= 8 || batch <= 3 * cus;
+  return batch <= (w <= 8 ? 4 : 2) * cus;
+}
+
+template <typename T>
+int solo_launch(hipStream_t st, const purin_cp_plan* p, const Solo<T>& A, int mode, bool early) {
+  const SoloBlock k = solo_block(p, A.batch, early);
+  const size_t lds = solo_lds(p, k);
+  switch (mode) {
+    case kSoloShared: return launch_mode<T, kSoloShared>(st, A, k, lds, early);
+    case kSoloValues: return launch_mode<T, kSoloValues>(st, A, k, lds, early);
+    default: return launch_mode<T, kSoloQP>(st, A, k, lds, early);
+  }
+}
+
+template int solo_launch<double>(hipStream_t, const purin_cp_plan*, const Solo<double>&, int, bool);
+template int solo_launch<float>(hipStream_t, const purin_cp_plan*, const Solo<float>&, int, bool);
+
+}  // namespace purin

@@ -1,0 +1,123 @@
+"""The CP loop with one workgroup per sample (solo.hip) at the edges of its dispatch:
+wavefront counts with and without the wavefront of the stop test, idle wavefronts, rows
+and columns wider than the entries held in registers, and the batches where the tile
+kernels take over.  Held to the streaming passes on the whole batch, whose sums run in
+another order: the bars of the resident kernels' tests (fp64 counts identical; in fp32 a
+stop may fall elsewhere in at most 1 of 10 samples)."""
+
+import numpy as np
+import pytest
+
+from purin_amd import workloads
+from tests._gpu import canonical_from_workload, plan_for, rel_err, require_gpu, to_np
+
+pytestmark = pytest.mark.gpu
+
+TOL = {np.float64: 1e-10, np.float32: 1e-4}
+
+
+@pytest.mark.parametrize("n,me,mi,wmin,wmax,B,dtype", [
+    (64, 10, 20, 2, 9, 5, np.float64),       # one wavefront of columns; columns past 8 entries
+    (65, 10, 20, 2, 12, 5, np.float64),      # two; rows past 8 entries
+    (40, 30, 170, 2, 4, 3, np.float64),      # more rows than columns, wide columns
+    (250, 40, 60, 2, 6, 512, np.float64),    # four wavefronts, padded to seven and the test's
+    (250, 40, 60, 2, 6, 513, np.float64),    # four without the test's wavefront
+    (330, 40, 60, 2, 6, 9, np.float64),      # six, padded
+    (500, 40, 60, 2, 6, 256, np.float64),    # eight with the test's wavefront
+    (500, 40, 60, 2, 6, 257, np.float64),    # eight without
+    (600, 60, 150, 2, 6, 257, np.float64),   # ten: fixed iterations go to the tiles
+    (960, 90, 200, 2, 6, 7, np.float64),     # fifteen and the test's
+    (961, 90, 200, 2, 6, 7, np.float64),     # sixteen
+    (900, 90, 200, 2, 6, 300, np.float64),   # fifteen: the tiles
+    (1024, 100, 924, 2, 5, 4, np.float64),   # the largest
+    (200, 30, 60, 2, 7, 70, np.float32),
+    (600, 60, 150, 2, 6, 600, np.float32),   # fixed iterations on the tiles
+    (600, 60, 150, 2, 6, 800, np.float32),   # both loops on the tiles
+])
+@pytest.mark.parametrize("accelerated", [False, True])
+def test_solo_matches_streaming(n, me, mi, wmin, wmax, B, dtype, accelerated):
+    require_gpu()
+    w = workloads.ragged_rows(700 + n, n=n, me=me, mi=mi, wmin=wmin, wmax=wmax, batch=B,
+                              accelerated=accelerated)
+    canon = canonical_from_workload(w)
+    plan = plan_for(canon, dtype=dtype, accelerated=accelerated)
+    rhs = np.tile(w.rhs, (B, 1)).astype(dtype)
+    target = w.target.astype(dtype)
+    bar = TOL[dtype]
+    # bounds shared, and scaled per sample (their rows are the last 2 n)
+    scaled = rhs.copy()
+    scaled[:, me + mi:] *= np.linspace(0.8, 1.2, B).astype(dtype)[:, None]
+    for r, shared in ((rhs, True), (scaled, False)):
+        kw = dict(max_iterations=90, early_stop=False, shared_bounds=shared, timing=True)
+        a = plan.project(target, r, **kw)
+        assert plan.last_timing()["resident"] == 1
+        s = plan.project(target, r, streaming=True, **kw)
+        assert rel_err(to_np(a.y), to_np(s.y)) <= bar / 10
+        assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= bar
+        kw = dict(max_iterations=600, tolerance=2e-2, shared_bounds=shared)
+        a = plan.project(target, r, **kw)
+        s = plan.project(target, r, streaming=True, **kw)
+        ia, is_ = to_np(a.iterations), to_np(s.iterations)
+        same = ia == is_
+        assert same.all() if dtype == np.float64 else same.mean() >= 0.9
+        if 2 * (me + mi) < n:
+            assert (ia < 600).any()  # some samples stop, at their own iterations
+        assert rel_err(to_np(a.y)[same], to_np(s.y)[same]) <= bar
+        assert rel_err(to_np(a.multipliers)[same], to_np(s.multipliers)[same]) <= bar
+        np.testing.assert_array_equal(to_np(a.status)[same], to_np(s.status)[same])
+
+
+@pytest.mark.parametrize("iters", [1, 2, 3])
+def test_solo_short_runs(iters):
+    """The stop test trails the loop: runs that end before its first verdicts, and samples
+    accepted at their first iterations (targets inside the polyhedron)."""
+    require_gpu()
+    B, n = 6, 70
+    w = workloads.ragged_rows(9, n=n, me=0, mi=12, wmin=2, wmax=5, batch=B)
+    canon = canonical_from_workload(w)
+    plan = plan_for(canon, dtype=np.float64)
+    rhs = np.tile(w.rhs, (B, 1))
+    target = w.target.copy()
+    target[::2] = 1e-3 * target[::2]  # feasible (the rows allow the origin's neighbourhood)
+    rhs[:, :12] = np.abs(rhs[:, :12]) + 1.0
+    kw = dict(max_iterations=iters, tolerance=1e-6)
+    a = plan.project(target, rhs, **kw)
+    s = plan.project(target, rhs, streaming=True, **kw)
+    np.testing.assert_array_equal(to_np(a.iterations), to_np(s.iterations))
+    np.testing.assert_array_equal(to_np(a.status), to_np(s.status))
+    assert (to_np(a.status)[::2] == 0).all()
+    assert rel_err(to_np(a.y), to_np(s.y)) <= 1e-12
+
+
+@pytest.mark.parametrize("n,me,mi,B", [(70, 12, 30, 9), (300, 40, 90, 5), (1000, 80, 200, 3)])
+@pytest.mark.parametrize("early", [False, True])
+def test_solo_values_and_qp_match_streaming(n, me, mi, B, early):
+    """Per-sample coefficients and the diagonal QP (shared and per-sample coefficients)."""
+    require_gpu()
+    rng = np.random.default_rng(n)
+    w = workloads.ragged_rows(300 + n, n=n, me=me, mi=mi, wmin=2, wmax=10, batch=B)
+    canon = canonical_from_workload(w)
+    m = me + mi
+    values = np.tile(w.data, (B, 1))
+    general = w.indptr[m]
+    values[:, :general] *= rng.uniform(0.8, 1.2, (B, general))
+    rhs = np.tile(w.rhs, (B, 1))
+    kw = dict(max_iterations=400, tolerance=1e-3, early_stop=early)
+    for accelerated in (False, True):
+        plan = plan_for(canon, dtype=np.float64, accelerated=accelerated)
+        a = plan.project(w.target, rhs, values=values, **kw)
+        s = plan.project(w.target, rhs, values=values, streaming=True, **kw)
+        np.testing.assert_array_equal(to_np(a.iterations), to_np(s.iterations))
+        assert rel_err(to_np(a.y), to_np(s.y)) <= 1e-10
+        assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= 1e-10
+        rows = type(canon)(n=n, me=me, rows=canon.rows[:m], coef=canon.coef[:m])
+        plan = plan_for(rows, dtype=np.float64, accelerated=accelerated, bound_presolve=False)
+        q, c = rng.uniform(0.5, 2.0, (B, n)), rng.normal(0.0, 1.5, (B, n))
+        lo, hi = np.full((B, n), -1.0), np.full((B, n), 1.0)
+        y0 = 0.1 * rng.normal(size=(B, n))
+        for v in (None, values[:, :general]):
+            a = plan.qp_solve(q, c, rhs[:, :m], lo, hi, values=v, y0=y0, **kw)
+            s = plan.qp_solve(q, c, rhs[:, :m], lo, hi, values=v, y0=y0, streaming=True, **kw)
+            np.testing.assert_array_equal(to_np(a.iterations), to_np(s.iterations))
+            assert rel_err(to_np(a.y), to_np(s.y)) <= 1e-10
+            assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= 1e-10
