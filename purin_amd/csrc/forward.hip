@@ -359,6 +359,54 @@ static int run_solo(purin_cp_plan* p, hipStream_t st, const Layout& L, char* sv,
   return solo_launch<T>(st, p, A, qp ? kSoloQP : (ps ? kSoloValues : kSoloShared), early);
 }
 
+// The dense adapter's loop with one workgroup per sample (solo.hip).
+template <typename T>
+static int run_solo_dense(purin_cp_plan* p, hipStream_t st, const Layout& L, char* sv, char* ws,
+                          const purin_cp_solve_options& o, bool early, int64_t batch, int32_t* done,
+                          int32_t* count, int32_t* last, const QPRun<T>& qp,
+                          const PerSample<T>& ps) {
+  SoloDense<T> A{};
+  A.n = (int)p->n;
+  A.m = (int)p->m;
+  A.me = (int)p->me;
+  A.Bp = L.Bp;
+  A.batch = batch;
+  A.iters = o.max_iterations;
+  A.rptr = p->rptr;
+  A.ridx = p->ridx;
+  A.cptr = p->cptr;
+  A.cidx = p->cidx;
+  A.RV = ps.RVs ? ps.RVs : ps.RV;
+  A.CV = ps.RVs ? ps.CVs : ps.CV;
+  A.vbp = ps.RVs ? 1 : L.Bp;
+  A.Q = qp.Q;
+  A.C = qp.Cc;
+  A.R = (const T*)(sv + L.R);
+  A.LO = (const T*)(sv + L.LO);
+  A.HI = (const T*)(sv + L.HI);
+  A.step0 = ps.tau_b;
+  A.gam = p->opts.accelerated ? qp.gamma : nullptr;
+  A.accel = p->opts.accelerated;
+  A.tolv = ps.tol_b;
+  A.Y = (T*)(sv + L.Y);
+  A.YB = (T*)(ws + L.YB);
+  A.D = (T*)(sv + L.D);
+  A.done = done;
+  A.count = count;
+  A.last = last;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (o.timing) {
+    PURIN_HIP(hipEventCreate(&e0));
+    PURIN_HIP(hipEventCreate(&e1));
+    PURIN_HIP(hipEventRecord(e0, st));
+  }
+  k_fill<int32_t><<<1, 64, 0, st>>>(last, 1, 0);
+  if (!early)  // ybar0 = y0
+    PURIN_HIP(hipMemcpyAsync(A.YB, A.Y, (size_t)p->n * L.Bp * sizeof(T), hipMemcpyDeviceToDevice, st));
+  if (int rc = solo_dense_launch<T>(st, p, A, early)) return rc;
+  return finish_resident(p, st, o, e0, e1);
+}
+
 // The CP loop on the resident kernel; fills Y and D like the passes (and, with
 // early stop, the per-sample done flags and iteration counts).  qp (with ps):
 // the diagonal QP, q and c per sample, y0 from Y, the per-sample steps of ps.
@@ -575,8 +623,13 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
   const bool res_qp = qp && !qp->dense && ps && !o.shared_bounds;
   // per-sample coefficients: each tile streams its own
   const bool res_vals = !qp && ps && !ps->RVs;
-  if (lds && !o.streaming && !p->diag && ((!ps && !qp) || res_qp || res_vals)) {
-    if (int rc = run_resident<T>(p, st, L, sv, ws, o, lds, early, batch, tol_scalar, tolv, done,
+  const bool solo_dense = qp && qp->dense && ps && !o.streaming && solo_dense_fits(p);
+  if (solo_dense || (lds && !o.streaming && !p->diag && ((!ps && !qp) || res_qp || res_vals))) {
+    if (solo_dense) {
+      if (int rc = run_solo_dense<T>(p, st, L, sv, ws, o, early, batch, done, count, ndone + 2,
+                                     *qp, *ps))
+        return rc;
+    } else if (int rc = run_resident<T>(p, st, L, sv, ws, o, lds, early, batch, tol_scalar, tolv, done,
                                  count, noalloc, res_qp ? qp : nullptr,
                                  (res_qp || res_vals) ? ps : nullptr))
       return rc;

@@ -457,6 +457,263 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The dense adapter (dense.py:85-106): rows and columns of tens of entries, so several lanes
+// share each, and the loop runs until the last sample is accepted.  The streaming passes
+// walked each row serially on a few wavefronts: 244 us per iteration at n = 60, m = 37,
+// B = 64.  Launch 1 (FIRST) runs every sample to its own acceptance and leaves the largest
+// count; launch 2 takes each sample from its state there to that count.
+// ---------------------------------------------------------------------------
+constexpr int kSoloDenseW = 12;
+
+// sum over the 2^l lanes that share a row, in every one of them
+template <typename T>
+__device__ __forceinline__ T lane_sum(T v, int l) {
+  if (l >= 1) v += dpp_move<0xB1>(v);   // lane ^ 1
+  if (l >= 2) v += dpp_move<0x4E>(v);   // lane ^ 2
+  if (l >= 3) v += dpp_move<0x141>(v);  // the other quad of 8
+  if (l >= 4) v += dpp_move<0x140>(v);  // the other half of 16
+  if (l >= 5) v += __shfl_xor(v, 16);
+  if (l >= 6) v += __shfl_xor(v, 32);
+  return v;
+}
+
+template <typename T>
+__device__ __forceinline__ T dense_sum(const T (&v)[kSoloDenseW],
+                                       const uint32_t (&ix)[kSoloDenseW / 2], int groups, int l,
+                                       const unsigned char* lds) {
+  const T acc = groups <= 1 ? dot_regs<4>(v, ix, lds)
+                            : (groups == 2 ? dot_regs<8>(v, ix, lds) : dot_regs<12>(v, ix, lds));
+  return lane_sum(acc, l);
+}
+
+template <typename T, bool FIRST, bool HELP, int MAXB>
+__global__ __launch_bounds__(MAXB) void k_solo_dense(SoloDense<T> A) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  constexpr int W = kSoloDenseW;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int NW = (blockDim.x >> 6) - (HELP ? 1 : 0), NT = NW * 64;
+  const int64_t b = blockIdx.x, Bp = A.Bp;
+  const int n = A.n, m = A.m;
+  const int jt = t >> A.lc, gc = t & ((1 << A.lc) - 1), it_ = t >> A.lr, gr = t & ((1 << A.lr) - 1);
+  const bool col = jt < n && t < NT, row = it_ < m && t < NT;
+  const bool wc = col && gc == 0, wr = row && gr == 0;  // the lane that writes
+  const int j = col ? jt : 0, i = row ? it_ : 0;
+  if (b >= A.batch) {
+    if (FIRST && wc) A.Y[(int64_t)j * Bp + b] = A.YB[(int64_t)j * Bp + b] = T(0);
+    if (FIRST && wr) A.D[(int64_t)i * Bp + b] = T(0);
+    return;
+  }
+  const T zero = T(0), one = T(1), half = T(0.5), inf = T(__builtin_inf());
+  T* Gy = reinterpret_cast<T*>(lds);
+  T* Gd = Gy + n + 1;
+  T* red = Gd + m + 1;
+  volatile int* flag = reinterpret_cast<volatile int*>(red + (HELP ? 6 * NT : 64));
+  T rv[W], cv[W];
+  uint32_t rx[W / 2], cx[W / 2];
+  const int rs = A.rptr[i], re = row ? A.rptr[i + 1] : rs;
+  const int cs = n ? A.cptr[j] : 0, ce = col ? A.cptr[j + 1] : cs;
+  const int64_t vb = A.vbp > 1 ? b : 0;
+#pragma unroll
+  for (int k = 0; k < W; ++k) {
+    const int er = rs + (k << A.lr) + gr, ec = cs + (k << A.lc) + gc;
+    const bool okr = er < re, okc = ec < ce;
+    rv[k] = okr ? A.RV[(int64_t)er * A.vbp + vb] : zero;
+    cv[k] = okc ? A.CV[(int64_t)ec * A.vbp + vb] : zero;
+    const uint32_t xr = (uint32_t)((okr ? A.ridx[er] : n) * (int)sizeof(T));
+    const uint32_t xc = (uint32_t)((n + 1 + (okc ? A.cidx[ec] : m)) * (int)sizeof(T));
+    if (k & 1) {
+      rx[k / 2] |= xr << 16;
+      cx[k / 2] |= xc << 16;
+    } else {
+      rx[k / 2] = xr;
+      cx[k / 2] = xc;
+    }
+  }
+  const int rgr = (A.rw + 3) >> 2, cgr = (A.cw + 3) >> 2;
+  const int64_t jb = (int64_t)j * Bp + b, ib = (int64_t)i * Bp + b;
+  const T q = col ? A.Q[jb] : one, cj = col ? A.C[jb] : zero;
+  const T lo = col ? A.LO[jb] : zero, hi = col ? A.HI[jb] : zero;
+  const T rr = row ? A.R[ib] : zero;
+  T y = col ? A.Y[jb] : zero, d = row ? A.D[ib] : zero;
+  const bool ineq = i >= A.me;
+  T tau = res_uniform(A.step0[b]), sig = res_uniform(A.step0[Bp + b]);
+  T th = res_uniform(A.accel ? A.step0[4 * Bp + b] : one);
+  const T gam = res_uniform(A.gam ? A.gam[b] : one);
+  T pa = one / (one + tau * q);
+  auto advance = [&]() {  // the accelerated update (kernels.py:279-283)
+    if (!A.accel) return;
+    T g1[1] = {gam}, t1[1] = {tau}, s1[1] = {sig}, h1[1] = {th}, a1[1], d1[1];
+    res_qp_schedule<T, 1>(g1, t1, s1, h1, a1, d1);
+    tau = t1[0];
+    sig = s1[0];
+    th = h1[0];
+    pa = one / (one + tau * q);
+  };
+  auto step = [&](T tt) -> T {  // the factored prox (kernels.py:140-142)
+    return clipp(pa * ((y - tau * tt) - tau * cj), lo, hi);
+  };
+  if (t == 0) {
+    Gy[n] = zero;
+    Gd[m] = zero;
+    *flag = 0;
+  }
+
+  if constexpr (!FIRST) {
+    const int64_t from = A.count ? A.count[b] : 0;
+    const int64_t to = A.last ? *A.last : A.iters;
+    for (int64_t k = 0; k < from && A.accel; ++k) advance();
+    if (wc) Gy[j] = A.YB[jb];
+    if (wr) Gd[i] = d;
+    __syncthreads();
+    for (int64_t it = from; it < to; ++it) {
+      const T acc = dense_sum(rv, rx, rgr, A.lr, lds);
+      T p = d + sig * (acc - rr);
+      if (ineq) p = maxp(p, zero);
+      d = p;
+      if (wr) Gd[i] = p;
+      __syncthreads();
+      const T tt = dense_sum(cv, cx, cgr, A.lc, lds);
+      const T yn = step(tt);
+      if (wc) Gy[j] = yn + th * (yn - y);
+      y = yn;
+      advance();
+      __syncthreads();
+    }
+    if (wc) A.Y[jb] = y;
+    if (wr) A.D[ib] = d;
+    if (t == 0 && A.last) A.count[b] = (int32_t)to;
+    return;
+  }
+
+  if (wc) Gy[j] = y;
+  __syncthreads();
+  T ky = dense_sum(rv, rx, rgr, A.lr, lds);
+  {
+    T p = d + sig * (ky - rr);
+    if (ineq) p = maxp(p, zero);
+    d = p;
+    if (wr) Gd[i] = p;
+  }
+  __syncthreads();
+  const T tol = A.tolv[b];
+  auto judge = [&](T pri, T dual, T mx) -> bool {
+    const T gap = maxp(pri - dual, zero) / maxp(one, maxp(absv(pri), absv(dual)));
+    return finite(gap) && mx <= tol && gap <= tol;
+  };
+  if (HELP && wave == NW) {
+    for (int64_t it = 0;; ++it) {
+      if ((it >= 2 && __builtin_amdgcn_readfirstlane(*flag)) || it > A.iters) return;
+      T pri = zero, dual = zero, mx = inf;
+      if (it > 0) {
+        const T* pt = red + ((it - 1) & 1) * 3 * NT + lane;
+        mx = zero;
+        for (int w = 0; w < NW; ++w) {
+          pri += pt[w * 64];
+          dual += pt[NT + w * 64];
+          mx = __builtin_fmax(mx, pt[2 * NT + w * 64]);
+        }
+        const T s2 = two_sums(pri, dual);
+        pri = read_lane(s2, 0);
+        dual = read_lane(s2, 32);
+        mx = wave_fmax(mx);
+      }
+      __syncthreads();
+      const bool ok = judge(pri, dual, mx);
+      if (lane == 0) *flag = ok ? 1 : 0;
+      __syncthreads();
+    }
+  }
+  T yp = y, ypp = y, dk = d, dkp = d, th1 = one, th2 = one;
+  T q_pri = zero, q_dual = zero, q_max = inf;
+  int64_t it = 0;
+  bool accepted = false;
+  for (;; ++it) {
+    if (it >= 2 && __builtin_amdgcn_readfirstlane(*flag)) {
+      accepted = true;
+      break;
+    }
+    if (it > A.iters) break;
+    const bool run = it < A.iters;
+    const T r_pri = q_pri, r_dual = q_dual, r_max = q_max;
+    ypp = yp;
+    yp = y;
+    q_pri = q_dual = q_max = zero;
+    if (run) {
+      const T tt = dense_sum(cv, cx, cgr, A.lc, lds);
+      const T yn = step(tt);
+      y = yn;
+      if (wc) {
+        Gy[j] = yn;
+        q_pri = half * q * yn * yn + cj * yn;
+        const T tf = cj + tt;
+        const T mz = q > T(1e-12) ? clipp(-tf / q, lo, hi) : (tf >= zero ? lo : hi);
+        q_dual = half * q * (mz * mz) + tf * mz;
+        T g = maxp(maxp(lo - yn, zero), maxp(yn - hi, zero));
+        if (!finite(g)) g = inf;
+        q_max = g;
+      }
+    }
+    if constexpr (!HELP) {
+      const T s2 = two_sums(r_pri, r_dual);
+      const T mx = wave_fmax(r_max);
+      if ((lane & 31) == 0) red[wave * 4 + (lane >> 5)] = s2;
+      if (lane == 0) red[wave * 4 + 2] = mx;
+    }
+    __syncthreads();
+    dkp = dk;
+    dk = d;
+    th2 = th1;
+    th1 = th;
+    const T theta = th;
+    if (run) advance();
+    if (run) {
+      const T acc = dense_sum(rv, rx, rgr, A.lr, lds);
+      if (wr) {
+        const T e = acc - rr, w = ineq ? zero : -one;
+        q_max = __builtin_fmax(q_max, __builtin_fmax(e, w * e));
+        q_dual = (q_dual - rr * d) - d * zero;
+      }
+      if (it + 1 < A.iters) {
+        T p = d + sig * (((one + theta) * acc - theta * ky) - rr);
+        if (ineq) p = maxp(p, zero);
+        d = p;
+        if (wr) Gd[i] = p;
+      }
+      ky = acc;
+    }
+    if constexpr (HELP) {
+      T* pt = red + (it & 1) * 3 * NT + t;
+      pt[0] = q_pri;
+      pt[NT] = q_dual;
+      pt[2 * NT] = q_max;
+    } else if (wave == NW - 1) {
+      const T* rl = red + (lane & 15) * 4;
+      const bool in = (lane & 15) < NW;
+      const T xp = row16_combine(in ? rl[0] : zero, OpAdd());
+      const T xd = row16_combine(in ? rl[1] : zero, OpAdd());
+      const T mx = row16_combine(in ? rl[2] : zero, OpFMax());
+      const bool ok = it > 0 && judge(xp, xd, mx);
+      if (lane == 0) *flag = ok ? 1 : 0;
+    }
+    __syncthreads();
+  }
+  if (accepted) {  // the state of iteration it - 2, and its ybar
+    if (wc) A.YB[jb] = yp + th2 * (yp - ypp);
+    y = yp;
+    dk = dkp;
+  }
+  if (wc) A.Y[jb] = y;
+  if (wr) A.D[ib] = dk;
+  if (t == 0) {
+    const int32_t k = (int32_t)(accepted ? it - 1 : A.iters);
+    A.count[b] = k;
+    A.done[b] = accepted ? 1 : 0;
+    atomicMax(A.last, k);
+  }
+}
+
 int rest_entries(const purin_cp_plan* p, int W) {
   int k = 0;
   for (int w : p->sl_rw) k += rest_of(w, W) * 64;
@@ -544,6 +801,43 @@ int solo_launch(hipStream_t st, const purin_cp_plan* p, const Solo<T>& A, int mo
     default: return launch_mode<T, kSoloQP>(st, A, k, lds, early);
   }
 }
+
+// Lanes per row (log2) and entries per lane for rows of up to ``width`` entries.
+static void dense_lanes(int width, int* l, int* entries) {
+  *l = 0;
+  while (*l < 6 && (width + (1 << *l) - 1) >> *l > kSoloDenseW) ++*l;
+  *entries = (width + (1 << *l) - 1) >> *l;
+}
+
+bool solo_dense_fits(const purin_cp_plan* p) {
+  if (!p->sl_ok || p->n > kSoloMax || p->m > kSoloMax || p->m < 1) return false;
+  int lr, lc, rw, cw;
+  dense_lanes(p->sl_rw[0], &lr, &rw);
+  dense_lanes(p->sl_cw[0], &lc, &cw);
+  return rw <= kSoloDenseW && cw <= kSoloDenseW && p->m << lr <= 1024 && p->n << lc <= 1024;
+}
+
+template <typename T>
+int solo_dense_launch(hipStream_t st, const purin_cp_plan* p, SoloDense<T> A, bool early) {
+  dense_lanes(p->sl_rw[0], &A.lr, &A.rw);
+  dense_lanes(p->sl_cw[0], &A.lc, &A.cw);
+  const int waves = (int)((std::max<int64_t>(p->m << A.lr, p->n << A.lc) + 63) / 64);
+  const size_t lds = (size_t)(p->n + 1 + p->m + 1 + 6 * 64 * waves + 2) * sizeof(T);
+  if (early) {  // up to 512 threads the kernel has registers to spare (above, fp64 spills 128 B)
+    auto kern = waves < 8 ? k_solo_dense<T, true, true, 512>
+                          : (waves < 16 ? k_solo_dense<T, true, true, 1024>
+                                        : k_solo_dense<T, true, false, 1024>);
+    if (int rc = raise_lds_cap((const void*)kern, lds)) return rc;
+    kern<<<(unsigned)A.Bp, 64u * (unsigned)(waves + (waves < 16 ? 1 : 0)), lds, st>>>(A);
+  } else {
+    A.count = A.last = nullptr;
+  }
+  if (int rc = raise_lds_cap((const void*)k_solo_dense<T, false, false, 1024>, lds)) return rc;
+  k_solo_dense<T, false, false, 1024><<<(unsigned)A.Bp, 64u * (unsigned)waves, lds, st>>>(A);
+  return PURIN_CP_OK;
+}
+template int solo_dense_launch<double>(hipStream_t, const purin_cp_plan*, SoloDense<double>, bool);
+template int solo_dense_launch<float>(hipStream_t, const purin_cp_plan*, SoloDense<float>, bool);
 
 template int solo_launch<double>(hipStream_t, const purin_cp_plan*, const Solo<double>&, int, bool);
 template int solo_launch<float>(hipStream_t, const purin_cp_plan*, const Solo<float>&, int, bool);

@@ -59,4 +59,37 @@ bool solo_fits(const purin_cp_plan* p, int64_t batch, bool early, bool values);
 template <typename T>
 int solo_launch(hipStream_t st, const purin_cp_plan* p, const Solo<T>& A, int mode, bool early);
 
+// The dense adapter's loop (factored prox, no freezing, no stationarity test): every sample
+// iterates until the last is accepted.  A row is shared by 2^lr lanes, a column by 2^lc.
+template <typename T>
+struct SoloDense {
+  int n, m, me, lr, lc, rw, cw;  // rw / cw: entries of a lane's row / column (at most kSoloDenseW)
+  int64_t Bp, batch, iters;
+  const int32_t* __restrict__ rptr;
+  const int32_t* __restrict__ ridx;
+  const int32_t* __restrict__ cptr;
+  const int32_t* __restrict__ cidx;
+  const T* __restrict__ RV;  // kept CSR / CSC entries, [entry * vbp + b * (vbp > 1)]
+  const T* __restrict__ CV;
+  int64_t vbp;
+  const T* __restrict__ Q;
+  const T* __restrict__ C;
+  const T* __restrict__ R;
+  const T* __restrict__ LO;
+  const T* __restrict__ HI;
+  const T* __restrict__ step0;  // [5][Bp]
+  const T* __restrict__ gam;    // [Bp] or nullptr
+  int accel;
+  const T* __restrict__ tolv;
+  T* Y;                         // n x Bp: y0, then y
+  T* YB;                        // n x Bp: ybar between the two launches
+  T* D;
+  int32_t* done;
+  int32_t* count;
+  int32_t* last;                // the iteration at which the last sample is accepted
+};
+bool solo_dense_fits(const purin_cp_plan* p);
+template <typename T>
+int solo_dense_launch(hipStream_t st, const purin_cp_plan* p, SoloDense<T> A, bool early);
+
 }  // namespace purin

@@ -67,6 +67,40 @@ def test_dense_solve_matches_oracle(dtype, accelerated, early_stop):
     assert rel_err(to_np(gm), np.concatenate((lam, mu), axis=1)) <= TOL[dtype]
 
 
+@pytest.mark.parametrize("n,me,mi,B,accelerated,dtype", [
+    (7, 1, 1, 3, False, np.float64),      # one lane per row and column
+    (13, 2, 3, 5, True, np.float64),      # two lanes per row
+    (60, 12, 25, 7, False, np.float64),   # eight and four lanes
+    (60, 12, 25, 7, True, np.float64),
+    (120, 20, 44, 4, False, np.float64),  # sixteen wavefronts: none left for the stop test
+    (150, 10, 21, 3, False, np.float32),
+    (200, 20, 44, 2, False, np.float64),  # too large for the one-workgroup loop
+])
+def test_dense_one_workgroup_loop(n, me, mi, B, accelerated, dtype):
+    """Lanes per row and column, wavefront counts and the two launches (to each sample's own
+    acceptance, then to the last one's) against the oracle; fixed iterations too."""
+    require_gpu()
+    q, c, A, b, C, d, lo, hi = (x.astype(dtype) for x in _problem(61, B=B, n=n, me=me, mi=mi))
+    plan = _dense_plan(n, me, mi, dtype, accelerated=accelerated)
+    values = np.concatenate((A, C), axis=1).reshape(B, -1)
+    tol = (1e-4 if accelerated else 1e-6) if dtype == np.float64 else 1e-2
+    for early, iters, t in ((True, 3000, tol), (False, 60, 1e-30)):
+        y, lam, mu, it, _ = od.solve_dense(q, c, A, b, C, d, lo, hi, accelerated=accelerated,
+                                           max_iterations=iters, tolerance=max(t, 1e-300))
+        gy, gm, git, _ = plan.dense_solve(q, c, np.concatenate((b, d), axis=1), lo, hi,
+                                          values=values, tolerance=t, max_iterations=iters,
+                                          early_stop=early)
+        if dtype == np.float64:
+            np.testing.assert_array_equal(to_np(git), it)
+            assert rel_err(to_np(gy), y) <= TOL[dtype]
+            assert rel_err(to_np(gm), np.concatenate((lam, mu), axis=1)) <= TOL[dtype]
+        else:  # a stop a few iterations away moves the iterate by the tolerance at most
+            assert abs(int(to_np(git)[0]) - int(it[0])) <= 0.1 * int(it[0])
+            assert rel_err(to_np(gy), y) <= (5 * tol if early else TOL[dtype])
+        if early:
+            assert it[0] < iters
+
+
 def test_dense_packed_inequality_support():
     """A packed inequality support (sparse_layer.py:44-122): the inequality rows
     keep only their listed columns; the same iteration otherwise."""
