@@ -1426,10 +1426,10 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   if (restart > kMaxRestart) return set_error(PURIN_CP_ERR_UNSUPPORTED, "restart above 128");
   const bool dense = qa && qa->dense;
   static_assert((kMaxRestart + 2) * 4 <= kPinnedBytes, "per-step counts must fit the pinned buffer");
-  // GMRES runs one workgroup per sample where its vectors u and w fit LDS and the
+  // The solver runs one workgroup per sample where its vectors u and w fit LDS and the
   // restart length its one-lane-per-vector algebra; otherwise on batch-minor passes
   // (very large problems, long restarts)
-  const bool wg = !dense && gmr_fits(p, restart);
+  const bool wg = gmr_fits(p, restart);
   // workspace
   const int nchunk = (int)((W + kChunk - 1) / kChunk);
   // Gram--Schmidt passes: about 1024 blocks of 4 wavefronts over the batch tiles
@@ -1484,7 +1484,7 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   const size_t oPS = per_sample ? take(Lv.ws_end) : 0;
   const size_t oSw = per_sample ? take(m * Bp * es) : 0;
   const size_t oGV = per_sample ? take((size_t)p->nnz_full * Bp * es) : 0;
-  const size_t oBi = (qa && qa->dense) ? take((size_t)(kBiBlocks + kSlots) * es) : 0;
+  const size_t oBi = dense ? take((wg ? (size_t)(kBiScalars + 3 * batch) : (size_t)(kBiBlocks + kSlots)) * es) : 0;
   const size_t oSp = qa ? take(n * Bp * es) : 0;    // pre-clip values (q gradient)
   const size_t oGq = qa ? take(n * Bp * es) : 0;    // g_q
   const size_t oCd = (qa && qa->cot_dual) ? take((size_t)std::max<int64_t>(M, 1) * Bp * es) : 0;
@@ -1760,8 +1760,104 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
                                     dense ? 1 : o.force_eligible, Gr);
   T* lam_w = (T*)(ws + oLw);
   purin_cp_adjoint_stats stats{};
-  if (dense) {
-    // BiCGSTAB on (I - J^T) v = g over the whole batch (fixed_point.py:8-40)
+  if (wg) {
+    Gmr<T> Q{};
+    Q.n = (int)n;
+    Q.m = (int)m;
+    Q.W = (int)W;
+    Q.restart = restart;
+    Q.Wp = Wp;
+    Q.nsr = p->sl_nsr;
+    Q.nsc = p->sl_nsc;
+    Q.roff = p->sl_roff;
+    Q.coff = p->sl_coff;
+    Q.ridx = p->sl_ridx;
+    Q.cidx = p->sl_cidx;
+    Q.rval = (const T*)p->sl_rval;
+    Q.cval = (const T*)p->sl_cval;
+    Q.a = S.a;
+    Q.delta = S.delta;
+    Q.sigma = S.sigma;
+    Q.mask = (const T*)(ws + zM);
+    Q.G = (const T*)(ws + zG);
+    Q.X = (T*)(ws + zX);
+    Q.R = (T*)(ws + zR);
+    Q.Z = (T*)(ws + zZ);
+    Q.thr = G.thr;
+    Q.rinf = G.rinf;
+    Q.xfin = S2;
+    Q.total = G.total;
+    Q.ctrl = G.counter;
+    Q.rparts = gmr_parts(W, p->sl_nsr, p->sl_rw.empty() ? 0 : p->sl_rw[0]);
+    Q.cparts = gmr_parts(W, p->sl_nsc, p->sl_cw.empty() ? 0 : p->sl_cw[0]);
+    const unsigned by = (unsigned)((batch + 63) / 64);
+    if (S.dg) {
+      Q.av = (const T*)(ws + zA);
+      Q.dv = (const T*)(ws + zD);
+      Q.sv = (const T*)(ws + zS);
+    }
+    const int64_t stage = S.dg ? 3 * n + 2 * m : n + m;
+    k_gmr_stage<T><<<dim3((unsigned)((stage + 63) / 64), by), kBlock, 0, st>>>(
+        S, p->sl_cperm, p->sl_rperm, batch, (T*)(ws + zM), (T*)(ws + zA), (T*)(ws + zD),
+        (T*)(ws + zS));
+    if (per_sample) {  // the samples' entries, or one copy of a shared set (S.K.rval)
+      const bool each = S.K.rvb != nullptr;
+      const int64_t copies = each ? batch : 1, ld = each ? Bp : 1;
+      const unsigned cy = (unsigned)((copies + 63) / 64);
+      if (p->sl_rn)
+        k_gmr_entries<T><<<dim3((unsigned)((p->sl_rn + 63) / 64), cy), kBlock, 0, st>>>(
+            each ? S.K.rvb : S.K.rval, ld, p->sl_rsrc, p->sl_rn, copies, (T*)(ws + zRv));
+      if (p->sl_cn)
+        k_gmr_entries<T><<<dim3((unsigned)((p->sl_cn + 63) / 64), cy), kBlock, 0, st>>>(
+            each ? S.K.cvb : S.K.cval, ld, p->sl_csrc, p->sl_cn, copies, (T*)(ws + zCv));
+      Q.rval = (const T*)(ws + zRv);
+      Q.cval = (const T*)(ws + zCv);
+      Q.rstride = each ? p->sl_rn : 0;
+      Q.cstride = each ? p->sl_cn : 0;
+    }
+    k_gmr_init<T><<<(unsigned)batch, kBlock, 0, st>>>(
+        Q, (T*)(ws + zG), cot_y, metric, cotd, Bp, p->sl_cperm, p->sl_rperm, conv,
+        dense ? 1 : o.force_eligible, (T)o.tolerance, (T)o.atol);
+    if (dense) {  // BiCGSTAB on (I - J^T) v = g over the whole batch (fixed_point.py:8-40)
+      T* sc = (T*)(ws + oBi);
+      const GmrBi<T> B{sc, sc + kBiScalars, G.counter, batch, (T)o.tolerance, (T)o.atol,
+                       o.max_iterations};
+      k_fill<int32_t><<<1, 64, 0, st>>>(G.counter, 1, 0);
+      const T* host = (const T*)hw.get();
+      bool start = true;
+      do {
+        if (int rc = gmr_bicgstab<T>(st, Q, B, kBiGroup, start)) return rc;
+        PURIN_HIP(hipMemcpyAsync(hw.get(), sc, kBiScalars * sizeof(T), hipMemcpyDeviceToHost, st));
+        PURIN_HIP(hipStreamSynchronize(st));
+        start = false;
+      } while (host[kBiGo] != T(0));
+      stats.arnoldi_steps = (int64_t)host[kBiIt];
+      stats.cycles = (int32_t)host[kBiK];  // iterations, or -10 / -11 at breakdown
+      k_fill_weights<T><<<sb, 256, 0, st>>>(batch, Bp, lam_w);
+      if (o.arnoldi_iterations)
+        k_fill<int32_t><<<sb, 256, 0, st>>>(o.arnoldi_iterations, batch, (int32_t)host[kBiIt]);
+    }
+    // cycles, a few per host read: a cycle that no sample runs ends the solve
+    int64_t completed = 0;
+    for (bool more = !dense; more && completed < o.max_iterations;) {
+      k_fill<int32_t><<<1, 64, 0, st>>>(G.counter, kGmrGroup, 0);
+      for (int c = 0; c < kGmrGroup; ++c)
+        if (int rc = gmr_cycle<T>(st, Q, batch, S.dg != 0, c, completed, o.max_iterations)) return rc;
+      PURIN_HIP(hipMemcpyAsync(hw.get(), G.counter, kGmrGroup * sizeof(int32_t),
+                               hipMemcpyDeviceToHost, st));
+      PURIN_HIP(hipStreamSynchronize(st));
+      for (int c = 0; c < kGmrGroup && more; ++c) {
+        const int32_t steps = hw.get()[c];
+        more = steps > 0;
+        completed += steps;
+        stats.arnoldi_steps += steps;
+        stats.cycles += steps > 0;
+      }
+    }
+    k_gmr_solution<T><<<dim3((unsigned)((W + 63) / 64), by), kBlock, 0, st>>>(
+        Q.X, Wp, (int)n, (int)m, p->sl_cperm, p->sl_rperm, batch, Bp, X);
+  } else if (dense) {
+    // the same on batch-minor vectors
     T* bpart = (T*)(ws + oBi);
     T* bsc = bpart + kBiBlocks;
     T* RH = Vb;
@@ -1811,81 +1907,6 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
     k_fill_weights<T><<<sb, 256, 0, st>>>(batch, Bp, lam_w);
     if (o.arnoldi_iterations)
       k_fill<int32_t><<<sb, 256, 0, st>>>(o.arnoldi_iterations, batch, (int32_t)iters);
-  } else if (wg) {
-    Gmr<T> Q{};
-    Q.n = (int)n;
-    Q.m = (int)m;
-    Q.W = (int)W;
-    Q.restart = restart;
-    Q.Wp = Wp;
-    Q.nsr = p->sl_nsr;
-    Q.nsc = p->sl_nsc;
-    Q.roff = p->sl_roff;
-    Q.coff = p->sl_coff;
-    Q.ridx = p->sl_ridx;
-    Q.cidx = p->sl_cidx;
-    Q.rval = (const T*)p->sl_rval;
-    Q.cval = (const T*)p->sl_cval;
-    Q.a = S.a;
-    Q.delta = S.delta;
-    Q.sigma = S.sigma;
-    Q.mask = (const T*)(ws + zM);
-    Q.G = (const T*)(ws + zG);
-    Q.X = (T*)(ws + zX);
-    Q.R = (T*)(ws + zR);
-    Q.Z = (T*)(ws + zZ);
-    Q.thr = G.thr;
-    Q.rinf = G.rinf;
-    Q.xfin = S2;
-    Q.total = G.total;
-    Q.ctrl = G.counter;
-    const unsigned by = (unsigned)((batch + 63) / 64);
-    if (S.dg) {
-      Q.av = (const T*)(ws + zA);
-      Q.dv = (const T*)(ws + zD);
-      Q.sv = (const T*)(ws + zS);
-    }
-    const int64_t stage = S.dg ? 3 * n + 2 * m : n + m;
-    k_gmr_stage<T><<<dim3((unsigned)((stage + 63) / 64), by), kBlock, 0, st>>>(
-        S, p->sl_cperm, p->sl_rperm, batch, (T*)(ws + zM), (T*)(ws + zA), (T*)(ws + zD),
-        (T*)(ws + zS));
-    if (per_sample) {  // the samples' entries, or one copy of a shared set (S.K.rval)
-      const bool each = S.K.rvb != nullptr;
-      const int64_t copies = each ? batch : 1, ld = each ? Bp : 1;
-      const unsigned cy = (unsigned)((copies + 63) / 64);
-      if (p->sl_rn)
-        k_gmr_entries<T><<<dim3((unsigned)((p->sl_rn + 63) / 64), cy), kBlock, 0, st>>>(
-            each ? S.K.rvb : S.K.rval, ld, p->sl_rsrc, p->sl_rn, copies, (T*)(ws + zRv));
-      if (p->sl_cn)
-        k_gmr_entries<T><<<dim3((unsigned)((p->sl_cn + 63) / 64), cy), kBlock, 0, st>>>(
-            each ? S.K.cvb : S.K.cval, ld, p->sl_csrc, p->sl_cn, copies, (T*)(ws + zCv));
-      Q.rval = (const T*)(ws + zRv);
-      Q.cval = (const T*)(ws + zCv);
-      Q.rstride = each ? p->sl_rn : 0;
-      Q.cstride = each ? p->sl_cn : 0;
-    }
-    k_gmr_init<T><<<(unsigned)batch, kBlock, 0, st>>>(
-        Q, (T*)(ws + zG), cot_y, metric, cotd, Bp, p->sl_cperm, p->sl_rperm, conv,
-        o.force_eligible, (T)o.tolerance, (T)o.atol);
-    // cycles, a few per host read: a cycle that no sample runs ends the solve
-    int64_t completed = 0;
-    for (bool more = true; more && completed < o.max_iterations;) {
-      k_fill<int32_t><<<1, 64, 0, st>>>(G.counter, kGmrGroup, 0);
-      for (int c = 0; c < kGmrGroup; ++c)
-        if (int rc = gmr_cycle<T>(st, Q, batch, S.dg != 0, c, completed, o.max_iterations)) return rc;
-      PURIN_HIP(hipMemcpyAsync(hw.get(), G.counter, kGmrGroup * sizeof(int32_t),
-                               hipMemcpyDeviceToHost, st));
-      PURIN_HIP(hipStreamSynchronize(st));
-      for (int c = 0; c < kGmrGroup && more; ++c) {
-        const int32_t steps = hw.get()[c];
-        more = steps > 0;
-        completed += steps;
-        stats.arnoldi_steps += steps;
-        stats.cycles += steps > 0;
-      }
-    }
-    k_gmr_solution<T><<<dim3((unsigned)((W + 63) / 64), by), kBlock, 0, st>>>(
-        Q.X, Wp, (int)n, (int)m, p->sl_cperm, p->sl_rperm, batch, Bp, X);
   } else {
   // threshold = max(atol, tol * max|g|) and residual_inf = max|g - A 0| = max|g|
   k_gs<T, 4><<<ggs, kBlock, 0, st>>>(nullptr, 0, 0, Gr, nullptr, W, Bp, part, nchunk, Bp);

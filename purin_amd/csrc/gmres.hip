@@ -17,6 +17,7 @@
 // step i - 1 after one projection, v_j = sum_{i <= j} Z_i Tm[i][j], so a step reads
 // the prefix twice.  The dot pass walks the elements last to first and the update
 // pass first to last, so the update begins on rows the caches still hold.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -157,8 +158,8 @@ __device__ __forceinline__ void wave_sync() {
 
 // --- LDS of one workgroup ---------------------------------------------------------
 
-// Elements: u [n + 1], w [m + 1], the wavefronts' partial sums [BS / 64][33], then
-// per-sample algebra (below), then the basis where it fits.
+// Elements: u [n + 1], w [m + 1], the wavefronts' partial sums [BS / 64][33], shares of
+// slices [BS], then per-sample algebra (below), then the basis where it fits.
 constexpr int kAlg = 3 * kLd * kLd + 10 * kLd;
 
 template <typename T>
@@ -182,17 +183,51 @@ struct Alg {  // pointers into the algebra block
 };
 
 inline size_t lds_elems(int64_t n, int64_t m, int64_t W, int restart, int bs, bool basis) {
-  return (size_t)(n + 1 + m + 1 + (bs / 64) * kLd + kAlg + (basis ? (restart + 1) * W : 0));
+  return (size_t)(n + 1 + m + 1 + (bs / 64) * kLd + bs + kAlg + (basis ? (restart + 1) * W : 0));
 }
 
 // --- the operator -----------------------------------------------------------------
+
+// put(s, sum) of every slice by one wavefront: the products of its entries with x.  With
+// parts > 1 (a multiple of few wide slices) that many wavefronts take every parts-th entry
+// and meet in LDS: 60 serial loads of a dense row are 6 us otherwise.
+template <typename T, int BS, typename Put>
+__device__ __forceinline__ void slices(int ns, int parts, const int32_t* __restrict__ off,
+                                       const uint16_t* __restrict__ idx, const T* __restrict__ val,
+                                       const T* x, T* share, Put put) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (parts <= 1) {
+    for (int s = wave; s < ns; s += BS / 64) {
+      const int o0 = off[s], o1 = off[s + 1];
+      T acc = T(0);
+#pragma unroll 4
+      for (int o = o0 + lane; o < o1; o += 64) acc += val[o] * x[idx[o]];
+      put(s, acc);
+    }
+    return;
+  }
+  const int s = wave / parts, part = wave % parts;  // ns * parts <= wavefronts
+  T acc = T(0);
+  if (s < ns) {
+    const int o0 = off[s], o1 = off[s + 1];
+#pragma unroll 4
+    for (int o = o0 + part * 64 + lane; o < o1; o += parts * 64) acc += val[o] * x[idx[o]];
+    share[wave * 64 + lane] = acc;
+  }
+  __syncthreads();
+  if (s < ns && part == 0) {
+    for (int k = 1; k < parts; ++k) acc += share[(wave + k) * 64 + lane];
+    put(s, acc);
+  }
+}
 
 // out = v sc - pullback(v sc) (adjoint.hip's k_op_*): u = C (gy + 2 gb),
 // w = D (gd - delta K u), out = (gy - (a u - gb), gd - w, gb - sigma K^T w).  One
 // thread per row / column of a slice; u and w meet in LDS.
 template <typename T, int BS, bool DG>
 __device__ __forceinline__ void apply(const Gmr<T>& A, int64_t b, const T* __restrict__ v, T sc,
-                                      T* __restrict__ out, T* u, T* w) {
+                                      T* __restrict__ out, T* u, T* w, T* share) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = A.n, m = A.m;
@@ -208,11 +243,7 @@ __device__ __forceinline__ void apply(const Gmr<T>& A, int64_t b, const T* __res
   }
   __syncthreads();
   const T* __restrict__ rval = A.rval + (size_t)b * A.rstride;
-  for (int s = wave; s < A.nsr; s += BS / 64) {
-    const int o0 = A.roff[s], o1 = A.roff[s + 1];
-    T acc = T(0);
-#pragma unroll 4
-    for (int o = o0 + lane; o < o1; o += 64) acc += rval[o] * u[A.ridx[o]];
+  slices<T, BS>(A.nsr, A.rparts, A.roff, A.ridx, rval, u, share, [&](int s, T acc) {
     const int i = s * 64 + lane;
     if (i < m) {
       const T gd = v[n + i] * sc;
@@ -220,20 +251,16 @@ __device__ __forceinline__ void apply(const Gmr<T>& A, int64_t b, const T* __res
       w[i] = DG ? sv[i] * wi : wi;
       out[n + i] = gd - wi;
     }
-  }
+  });
   __syncthreads();
   const T* __restrict__ cval = A.cval + (size_t)b * A.cstride;
-  for (int s = wave; s < A.nsc; s += BS / 64) {
-    const int o0 = A.coff[s], o1 = A.coff[s + 1];
-    T acc = T(0);
-#pragma unroll 4
-    for (int o = o0 + lane; o < o1; o += 64) acc += cval[o] * w[A.cidx[o]];
+  slices<T, BS>(A.nsc, A.cparts, A.coff, A.cidx, cval, w, share, [&](int s, T acc) {
     const int j = s * 64 + lane;
     if (j < n) {
       const T gb = v[n + m + j] * sc;
       out[n + m + j] = DG ? gb - acc : gb - A.sigma * acc;
     }
-  }
+  });
   __syncthreads();
 }
 
@@ -344,7 +371,8 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
   T* u = reinterpret_cast<T*>(gmr_raw);
   T* w = u + n + 1;
   T* red = w + m + 1;
-  const Alg<T> S(red + NW * kLd);
+  T* share = red + NW * kLd;
+  const Alg<T> S(share + BS);
   T* zl = S.Wc + kLd;
   __shared__ T s_inv;
   __shared__ int s_on;
@@ -387,7 +415,7 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
   while (it < limit) {
     const int nv = it + 1;
     T* y = Z + (int64_t)nv * ld;
-    apply<T, BS, DG>(A, b, Z + (int64_t)it * ld, s_inv, y, u, w);
+    apply<T, BS, DG>(A, b, Z + (int64_t)it * ld, s_inv, y, u, w, share);
     pass<T, BS, false>(Z, ldb, nv, y, W, S.Q, red);
     __syncthreads();
     if (wave == 0) {  // p = Z^T y; g1 = Tm^T p; q1 = Tm g1
@@ -513,7 +541,7 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
   }
   __syncthreads();
   // the candidate's residual r = g - A x (operators.py:1084-1091); the basis is free
-  apply<T, BS, DG>(A, b, X, T(1), Z, u, w);
+  apply<T, BS, DG>(A, b, X, T(1), Z, u, w, share);
   T big = T(0);
   for (int e = tid; e < W; e += BS) {
     const T r = G[e] - Z[e];
@@ -543,6 +571,184 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
   }
 }
 
+// --- BiCGSTAB over the batch --------------------------------------------------------
+
+// The batch's sums of the workgroups' N values: each leaves its own in ``part``, and the
+// last to arrive adds them in sample order and hands them to ``then`` (one thread).
+template <typename T, int BS, int N, typename Then>
+__device__ __forceinline__ void batch_sums(const GmrBi<T>& B, T (&v)[N], T* red, Then then) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NW = BS / 64;
+  __shared__ int s_last;
+  auto block = [&](T (&x)[N]) {  // sums over the workgroup, in thread 0
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const T s = fold<32>(x[k]);
+      if (lane == 0) red[wave * kLd + k] = s;
+    }
+    __syncthreads();
+    if (tid == 0) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        x[k] = red[k];
+        for (int w = 1; w < NW; ++w) x[k] += red[w * kLd + k];
+      }
+    }
+    __syncthreads();
+  };
+  block(v);
+  if (tid == 0) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) B.part[k * B.batch + blockIdx.x] = v[k];
+    __threadfence();
+    s_last = atomicAdd(B.ticket, 1) == (int)gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  __threadfence();
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = T(0);
+  for (int64_t b = tid; b < B.batch; b += BS) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      v[k] += __hip_atomic_load(&B.part[k * B.batch + b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  block(v);
+  if (tid == 0) {
+    *B.ticket = 0;
+    then(v);
+  }
+}
+
+// The LDS of the products: u [n + 1], w [m + 1], partial sums, shares of slices.
+template <typename T, int BS>
+struct BiLds {
+  T *u, *w, *red, *share;
+  __device__ BiLds(unsigned char* raw, int n, int m) {
+    u = reinterpret_cast<T*>(raw);
+    w = u + n + 1;
+    red = w + m + 1;
+    share = red + (BS / 64) * kLd;
+    if (threadIdx.x == 0) {
+      u[n] = T(0);
+      w[m] = T(0);
+    }
+  }
+};
+
+// scalars for the next iteration: rho_ = rhat . r, beta, and whether it runs
+template <typename T>
+__device__ __forceinline__ void bi_next(const GmrBi<T>& B, T rs, T rho) {
+  T* sc = B.sc;
+  sc[kBiRhoN] = rho;
+  sc[kBiBeta] = rho / sc[kBiRho] * sc[kBiAlpha] / sc[kBiOmega];
+  sc[kBiGo] = rs > sc[kBiAtol2] && sc[kBiK] < (T)B.max_iterations && sc[kBiK] >= T(0) ? T(1) : T(0);
+}
+
+// rhat = p = q = r0 = b; rho = alpha = omega = 1
+template <typename T, int BS>
+__global__ __launch_bounds__(BS) void k_bic_start(Gmr<T> A, GmrBi<T> B) {
+  extern __shared__ __align__(16) unsigned char gmr_raw[];
+  const BiLds<T, BS> S(gmr_raw, A.n, A.m);
+  const T* g = A.G + (size_t)blockIdx.x * A.Wp;
+  T* Z = A.Z + (size_t)blockIdx.x * (A.restart + 1) * A.Wp;
+  T v[1] = {T(0)};
+  for (int e = threadIdx.x; e < A.W; e += BS) {
+    const T x = g[e];
+    Z[e] = Z[A.Wp + e] = Z[2 * A.Wp + e] = x;
+    v[0] += x * x;
+  }
+  batch_sums<T, BS, 1>(B, v, S.red, [&](T (&t)[1]) {
+    T* sc = B.sc;
+    sc[kBiBS] = t[0];
+    sc[kBiAtol2] = maxp(B.tol * B.tol * t[0], B.atol * B.atol);
+    sc[kBiRho] = sc[kBiAlpha] = sc[kBiOmega] = T(1);
+    sc[kBiK] = sc[kBiIt] = T(0);
+    bi_next(B, t[0], t[0]);
+  });
+}
+
+// p = r + beta (p - omega q), q = A p, alpha = rho / (rhat . q)
+template <typename T, int BS>
+__global__ __launch_bounds__(BS) void k_bic_p(Gmr<T> A, GmrBi<T> B) {
+  extern __shared__ __align__(16) unsigned char gmr_raw[];
+  if (B.sc[kBiGo] == T(0)) return;
+  const BiLds<T, BS> S(gmr_raw, A.n, A.m);
+  const int64_t b = blockIdx.x;
+  const T* R = A.R + (size_t)b * A.Wp;
+  T* Z = A.Z + (size_t)b * (A.restart + 1) * A.Wp;
+  T *P = Z + A.Wp, *Q = Z + 2 * A.Wp;
+  const T beta = B.sc[kBiBeta], omega = B.sc[kBiOmega];
+  for (int e = threadIdx.x; e < A.W; e += BS) P[e] = R[e] + beta * (P[e] - omega * Q[e]);
+  __syncthreads();
+  apply<T, BS, true>(A, b, P, T(1), Q, S.u, S.w, S.share);
+  T v[1] = {T(0)};
+  for (int e = threadIdx.x; e < A.W; e += BS) v[0] += Z[e] * Q[e];
+  batch_sums<T, BS, 1>(B, v, S.red, [&](T (&t)[1]) { B.sc[kBiAlphaN] = B.sc[kBiRhoN] / t[0]; });
+}
+
+// s = r - alpha q, t = A s, omega = (t . s) / (t . t)
+template <typename T, int BS>
+__global__ __launch_bounds__(BS) void k_bic_s(Gmr<T> A, GmrBi<T> B) {
+  extern __shared__ __align__(16) unsigned char gmr_raw[];
+  if (B.sc[kBiGo] == T(0)) return;
+  const BiLds<T, BS> S(gmr_raw, A.n, A.m);
+  const int64_t b = blockIdx.x;
+  const T* R = A.R + (size_t)b * A.Wp;
+  T* Z = A.Z + (size_t)b * (A.restart + 1) * A.Wp;
+  T *Q = Z + 2 * A.Wp, *Sv = Z + 3 * A.Wp, *Tv = Z + 4 * A.Wp;
+  const T alpha = B.sc[kBiAlphaN];
+  for (int e = threadIdx.x; e < A.W; e += BS) Sv[e] = R[e] - alpha * Q[e];
+  __syncthreads();
+  apply<T, BS, true>(A, b, Sv, T(1), Tv, S.u, S.w, S.share);
+  T v[3] = {T(0), T(0), T(0)};
+  for (int e = threadIdx.x; e < A.W; e += BS) {
+    const T s = Sv[e], t = Tv[e];
+    v[0] += s * s;
+    v[1] += t * s;
+    v[2] += t * t;
+  }
+  batch_sums<T, BS, 3>(B, v, S.red, [&](T (&t)[3]) {
+    B.sc[kBiSS] = t[0];
+    B.sc[kBiOmegaN] = t[1] / t[2];
+  });
+}
+
+// x and r, with the early exit; the iteration's end and the next one's scalars
+template <typename T, int BS>
+__global__ __launch_bounds__(BS) void k_bic_x(Gmr<T> A, GmrBi<T> B) {
+  extern __shared__ __align__(16) unsigned char gmr_raw[];
+  if (B.sc[kBiGo] == T(0)) return;
+  const BiLds<T, BS> S(gmr_raw, A.n, A.m);
+  const int64_t b = blockIdx.x;
+  T* X = A.X + (size_t)b * A.Wp;
+  T* R = A.R + (size_t)b * A.Wp;
+  const T* Z = A.Z + (size_t)b * (A.restart + 1) * A.Wp;
+  const T *P = Z + A.Wp, *Sv = Z + 3 * A.Wp, *Tv = Z + 4 * A.Wp;
+  const T alpha = B.sc[kBiAlphaN], omega = B.sc[kBiOmegaN];
+  const bool early = B.sc[kBiSS] < B.sc[kBiAtol2];
+  T v[2] = {T(0), T(0)};
+  for (int e = threadIdx.x; e < A.W; e += BS) {
+    const T s = Sv[e];
+    const T r = early ? s : s - omega * Tv[e];
+    X[e] = early ? X[e] + alpha * P[e] : X[e] + (alpha * P[e] + omega * s);
+    R[e] = r;
+    v[0] += r * r;
+    v[1] += Z[e] * r;
+  }
+  batch_sums<T, BS, 2>(B, v, S.red, [&](T (&t)[2]) {
+    T* sc = B.sc;
+    T k = (sc[kBiOmegaN] == T(0) || sc[kBiAlphaN] == T(0)) ? T(-11) : sc[kBiK] + T(1);
+    if (sc[kBiRhoN] == T(0)) k = T(-10);
+    sc[kBiK] = k;
+    sc[kBiIt] += T(1);
+    sc[kBiRho] = sc[kBiRhoN];
+    sc[kBiAlpha] = sc[kBiAlphaN];
+    sc[kBiOmega] = sc[kBiOmegaN];
+    bi_next(B, t[0], t[1]);
+  });
+}
+
 constexpr size_t kLdsMax = 160 * 1024;
 
 template <typename T, int BS, bool DG, bool ZL>
@@ -559,7 +765,7 @@ int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base
   // share a CU), with 4 wavefronts, the smallest (two elements a lane) with one:
   // 20,000 samples of W = 38 took 2.5 ms with four.
   if (A.W <= 128) return launch<T, 64, DG, true>(st, A, batch, c, base, max_it);
-  if (lds_elems(A.n, A.m, A.W, A.restart, 256, true) * sizeof(T) <= kLdsMax / 2)
+  if (A.W <= 512 && lds_elems(A.n, A.m, A.W, A.restart, 256, true) * sizeof(T) <= kLdsMax / 2)
     return launch<T, 256, DG, true>(st, A, batch, c, base, max_it);
   if (A.W <= 512) return launch<T, 256, DG, false>(st, A, batch, c, base, max_it);
   return launch<T, 512, DG, false>(st, A, batch, c, base, max_it);
@@ -578,6 +784,33 @@ int gmr_cycle(hipStream_t st, const Gmr<T>& A, int64_t batch, bool dg, int c, in
   return dg ? dispatch<T, true>(st, A, batch, c, base, max_iterations)
             : dispatch<T, false>(st, A, batch, c, base, max_iterations);
 }
+
+int gmr_parts(int64_t W, int slices, int widest) {
+  const int waves = W <= 128 ? 1 : (W <= 512 ? 4 : 8);
+  return slices > 0 && widest >= 16 ? std::max(1, waves / slices) : 1;
+}
+
+template <typename T>
+int gmr_bicgstab(hipStream_t st, const Gmr<T>& A, const GmrBi<T>& B, int iterations, bool start) {
+  auto go = [&](auto bs) -> int {
+    constexpr int BS = decltype(bs)::value;
+    const size_t lds = lds_elems(A.n, A.m, 0, 0, BS, false) * sizeof(T);
+    for (const void* k : {(const void*)k_bic_start<T, BS>, (const void*)k_bic_p<T, BS>,
+                          (const void*)k_bic_s<T, BS>, (const void*)k_bic_x<T, BS>})
+      if (int rc = raise_lds_cap(k, lds)) return rc;
+    const unsigned g = (unsigned)B.batch;
+    if (start) k_bic_start<T, BS><<<g, BS, lds, st>>>(A, B);
+    for (int k = 0; k < iterations; ++k) {
+      k_bic_p<T, BS><<<g, BS, lds, st>>>(A, B);
+      k_bic_s<T, BS><<<g, BS, lds, st>>>(A, B);
+      k_bic_x<T, BS><<<g, BS, lds, st>>>(A, B);
+    }
+    return PURIN_CP_OK;
+  };
+  return A.W <= 512 ? go(std::integral_constant<int, 256>{}) : go(std::integral_constant<int, 512>{});
+}
+template int gmr_bicgstab<double>(hipStream_t, const Gmr<double>&, const GmrBi<double>&, int, bool);
+template int gmr_bicgstab<float>(hipStream_t, const Gmr<float>&, const GmrBi<float>&, int, bool);
 
 template int gmr_cycle<double>(hipStream_t, const Gmr<double>&, int64_t, bool, int, int64_t, int64_t);
 template int gmr_cycle<float>(hipStream_t, const Gmr<float>&, int64_t, bool, int, int64_t, int64_t);

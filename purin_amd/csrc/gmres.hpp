@@ -21,6 +21,7 @@ struct Gmr {
   // 64 s .. 64 s + 63, entries off[s] .. off[s + 1) in [entry][lane] order, padded
   // with index n (rows) / m (columns), whose LDS element is zero
   int nsr, nsc;
+  int rparts, cparts;    // wavefronts that share a slice's entries (1: short rows / columns)
   const int32_t* __restrict__ roff;
   const int32_t* __restrict__ coff;
   const uint16_t* __restrict__ ridx;
@@ -53,5 +54,27 @@ bool gmr_fits(const purin_cp_plan* p, int64_t restart);
 template <typename T>
 int gmr_cycle(hipStream_t st, const Gmr<T>& A, int64_t batch, bool dg, int c, int64_t base,
               int64_t max_iterations);
+
+// BiCGSTAB over the whole batch as one vector (fixed_point.py:8-40), one workgroup per
+// sample: the vectors rhat, p, q, s, t in the basis slots 0..4, the scalars in ``sc``
+// (kBiScalars), per-sample partial sums in ``part`` [3][batch], a ticket counter.
+enum BiScalar { kBiBS = 0, kBiAtol2, kBiRho, kBiAlpha, kBiOmega, kBiRhoN, kBiAlphaN, kBiOmegaN,
+                kBiBeta, kBiSS, kBiK, kBiIt, kBiGo, kBiScalars };
+template <typename T>
+struct GmrBi {
+  T* sc;
+  T* part;
+  int32_t* ticket;
+  int64_t batch;
+  T tol, atol;
+  int64_t max_iterations;
+};
+constexpr int kBiGroup = 16;  // iterations enqueued between two host reads
+
+template <typename T>
+int gmr_bicgstab(hipStream_t st, const Gmr<T>& A, const GmrBi<T>& B, int iterations, bool start);
+
+// The wavefronts that share a slice in the kernels' products (for Gmr::rparts, cparts).
+int gmr_parts(int64_t W, int slices, int widest);
 
 }  // namespace purin

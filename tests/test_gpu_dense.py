@@ -176,3 +176,30 @@ def test_dense_adjoint_matches_oracle_at_the_same_state(with_dual_cotangent, tol
     for name, w in (("g_c", want[0]), ("g_values", want[1].reshape(B, -1)), ("g_rhs", want[2]),
                     ("g_lower", want[3]), ("g_upper", want[4])):
         assert rel_err(to_np(getattr(got, name)), w) <= bar, name
+
+
+@pytest.mark.parametrize("n,me,mi,B", [
+    (60, 12, 25, 5),    # four wavefronts sharing a slice of rows and of columns
+    (100, 30, 70, 66),  # two slices each
+    (230, 20, 40, 3),   # eight wavefronts
+])
+def test_dense_adjoint_wide_rows(n, me, mi, B):
+    """The per-sample BiCGSTAB kernels where wavefronts share a slice's entries, at the
+    GPU's state and converged: the solution is fixed to the residual (1e-12) times the
+    system's condition, below 1e4 here."""
+    require_gpu()
+    q, c, A, b, C, d, lo, hi = _problem(71, B=B, n=n, me=me, mi=mi)
+    plan = _dense_plan(n, me, mi, np.float64)
+    values = np.concatenate((A, C), axis=1)
+    rhs = np.concatenate((b, d), axis=1)
+    y, m, it, saved = plan.dense_solve(q, c, rhs, lo, hi, values=values.reshape(B, -1),
+                                       tolerance=1e-6, max_iterations=20000, save=True)
+    cot = np.random.default_rng(5).normal(size=(B, n))
+    cotd = np.zeros((B, me + mi))
+    want = od.implicit_vjp(q, c, values, rhs, lo, hi, me, to_np(y), to_np(m), cot, cotd,
+                           tolerance=1e-12, adjoint_iterations=2000)
+    got = plan.dense_adjoint(saved, q, c, cot, values=values.reshape(B, -1), tolerance=1e-12,
+                             max_iterations=2000)
+    assert 0 < want[5] < 2000 and 0 < plan.last_adjoint_stats()["cycles"] < 2000
+    for name, w in (("g_c", want[0]), ("g_values", want[1].reshape(B, -1)), ("g_rhs", want[2])):
+        assert rel_err(to_np(getattr(got, name)), w) <= 1e-8, name
