@@ -1153,22 +1153,6 @@ __global__ void k_grhs_full(int m, int n, int64_t Bp, const int32_t* __restrict_
 // sample-major operands of the per-sample GMRES cycles (gmres.hpp)
 // ---------------------------------------------------------------------------
 
-// A 64 x 64 tile through LDS: rows k0 .. k0 + 63 of a batch-minor array (get(k, b),
-// lanes over samples) to put(k, b, value) with lanes over k.
-template <typename T, typename Get, typename Put>
-__device__ __forceinline__ void minor_to_major_tile(int64_t K, int64_t batch, Get get, Put put) {
-  __shared__ T tile[64][65];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int64_t k0 = (int64_t)blockIdx.x * 64, b0 = (int64_t)blockIdx.y * 64;
-#pragma unroll 4
-  for (int r = ty; r < 64; r += kBlock / 64)
-    tile[r][tx] = k0 + r < K && b0 + tx < batch ? get(k0 + r, b0 + tx) : T(0);
-  __syncthreads();
-#pragma unroll 4
-  for (int r = ty; r < 64; r += kBlock / 64)
-    if (b0 + r < batch && k0 + tx < K) put(k0 + tx, b0 + r, tile[tx][r]);
-}
-
 // The masks and, with steps per element, a, delta and sigma, in position order.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_gmr_stage(Adj<T> S, const int32_t* __restrict__ cperm,
@@ -1195,17 +1179,6 @@ __global__ __launch_bounds__(kBlock) void k_gmr_stage(Adj<T> S, const int32_t* _
         else
           sv[b * m + k - 3 * n - m] = v;
       });
-}
-
-// dst[b][k] = src[map[k]][b], 0 where map[k] < 0: the entries of the slices
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_gmr_entries(const T* __restrict__ src, int64_t Bp,
-                                                        const int32_t* __restrict__ map, int64_t K,
-                                                        int64_t batch, T* __restrict__ dst) {
-  minor_to_major_tile<T>(
-      K, batch,
-      [&](int64_t k, int64_t b) -> T { return map[k] < 0 ? T(0) : src[(size_t)map[k] * Bp + b]; },
-      [&](int64_t k, int64_t b, T v) { dst[b * K + k] = v; });
 }
 
 // The right-hand side g = [cot * eligible, cotd * eligible, 0] of every sample (see
@@ -1805,10 +1778,10 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
       const int64_t copies = each ? batch : 1, ld = each ? Bp : 1;
       const unsigned cy = (unsigned)((copies + 63) / 64);
       if (p->sl_rn)
-        k_gmr_entries<T><<<dim3((unsigned)((p->sl_rn + 63) / 64), cy), kBlock, 0, st>>>(
+        k_to_major_map<T><<<dim3((unsigned)((p->sl_rn + 63) / 64), cy), kBlock, 0, st>>>(
             each ? S.K.rvb : S.K.rval, ld, p->sl_rsrc, p->sl_rn, copies, (T*)(ws + zRv));
       if (p->sl_cn)
-        k_gmr_entries<T><<<dim3((unsigned)((p->sl_cn + 63) / 64), cy), kBlock, 0, st>>>(
+        k_to_major_map<T><<<dim3((unsigned)((p->sl_cn + 63) / 64), cy), kBlock, 0, st>>>(
             each ? S.K.cvb : S.K.cval, ld, p->sl_csrc, p->sl_cn, copies, (T*)(ws + zCv));
       Q.rval = (const T*)(ws + zRv);
       Q.cval = (const T*)(ws + zCv);

@@ -66,6 +66,13 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
     L.X = take(std::max(n, m) * Bp * es);
     L.Z = take(std::max(n, m) * Bp * es);
   }
+  L.WTG = L.WRR = L.WLO = L.WHI = 0;
+  if ((extras & kLayoutWide) && (solo_wide_fits(p, true) || solo_wide_fits(p, false))) {
+    L.WTG = take(n * batch * es);
+    L.WRR = take(m * batch * es);
+    L.WLO = take(n * batch * es);
+    L.WHI = take(n * batch * es);
+  }
   if (p->res_ok) {  // resident path: slot-ordered copies of the per-sample inputs
     const size_t Kr = (size_t)p->res_mr * kResThreads, Kc = (size_t)p->res_mc * kResThreads;
     L.RTs = take(Kc * Bp * es);
@@ -359,6 +366,62 @@ static int run_solo(purin_cp_plan* p, hipStream_t st, const Layout& L, char* sv,
   return solo_launch<T>(st, p, A, qp ? kSoloQP : (ps ? kSoloValues : kSoloShared), early);
 }
 
+// The projection's loop with one workgroup per sample and several rows and columns per
+// thread (solo.hip).
+template <typename T>
+static int run_solo_wide(purin_cp_plan* p, hipStream_t st, const Layout& L, char* sv, char* ws,
+                         const purin_cp_solve_options& o, bool early, int64_t batch, T tol,
+                         const T* tolv, int32_t* done, int32_t* count) {
+  const void* sched = nullptr;
+  if (int rc = ensure_schedule(p, o.max_iterations, st, false, &sched)) return rc;
+  const int64_t n = p->n, m = p->m;
+  SoloWide<T> A{};
+  A.n = (int)n;
+  A.m = (int)m;
+  A.me = (int)p->me;
+  A.Bp = L.Bp;
+  A.batch = batch;
+  A.iters = o.max_iterations;
+  A.nsr = p->sl_nsr;
+  A.nsc = p->sl_nsc;
+  A.roff = p->sl_roff;
+  A.coff = p->sl_coff;
+  A.rperm = p->sl_rperm;
+  A.cperm = p->sl_cperm;
+  A.ridx = p->sl_ridx;
+  A.cidx = p->sl_cidx;
+  A.rval = (const T*)p->sl_rval;
+  A.cval = (const T*)p->sl_cval;
+  auto sorted = [&](const void* src, int64_t ld, const int32_t* perm, int64_t count, int64_t copies,
+                    size_t at) {
+    T* dst = (T*)(ws + at);
+    k_to_major_map<T><<<dim3((unsigned)((count + 63) / 64), (unsigned)((copies + 63) / 64)), kBlock,
+                        0, st>>>((const T*)src, ld, perm, count, copies, dst);
+    return (const T*)dst;
+  };
+  A.TG = sorted(sv + L.Tt, L.Bp, p->sl_cperm, n, batch, L.WTG);
+  A.RR = sorted(sv + L.R, L.Bp, p->sl_rperm, m, batch, L.WRR);
+  const bool shared = o.shared_bounds != 0;
+  A.LO = sorted(sv + L.LO, shared ? 1 : L.Bp, p->sl_cperm, n, shared ? 1 : batch, L.WLO);
+  A.HI = sorted(sv + L.HI, shared ? 1 : L.Bp, p->sl_cperm, n, shared ? 1 : batch, L.WHI);
+  A.bstride = shared ? 0 : n;
+  A.sched = (const T*)sched;
+  A.tol = tol;
+  A.tolv = tolv;
+  A.done = done;
+  A.count = count;
+  A.Y = (T*)(sv + L.Y);
+  A.D = (T*)(sv + L.D);
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  if (o.timing) {
+    PURIN_HIP(hipEventCreate(&e0));
+    PURIN_HIP(hipEventCreate(&e1));
+    PURIN_HIP(hipEventRecord(e0, st));
+  }
+  if (int rc = solo_wide_launch<T>(st, p, A, early)) return rc;
+  return finish_resident(p, st, o, e0, e1);
+}
+
 // The dense adapter's loop with one workgroup per sample (solo.hip).
 template <typename T>
 static int run_solo_dense(purin_cp_plan* p, hipStream_t st, const Layout& L, char* sv, char* ws,
@@ -624,10 +687,17 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
   // per-sample coefficients: each tile streams its own
   const bool res_vals = !qp && ps && !ps->RVs;
   const bool solo_dense = qp && qp->dense && ps && !o.streaming && solo_dense_fits(p);
-  if (solo_dense || (lds && !o.streaming && !p->diag && ((!ps && !qp) || res_qp || res_vals))) {
+  // (a longer call would extend the schedule, which the passes do not need)
+  const bool solo_wide = L.WTG && !ps && !qp && !o.streaming &&
+                         o.max_iterations <= p->res_sched_len && solo_wide_fits(p, early);
+  if (solo_dense || solo_wide || (lds && !o.streaming && !p->diag && ((!ps && !qp) || res_qp || res_vals))) {
     if (solo_dense) {
       if (int rc = run_solo_dense<T>(p, st, L, sv, ws, o, early, batch, done, count, ndone + 2,
                                      *qp, *ps))
+        return rc;
+    } else if (solo_wide) {
+      if (int rc = run_solo_wide<T>(p, st, L, sv, ws, o, early, batch, tol_scalar, tolv, done,
+                                    count))
         return rc;
     } else if (int rc = run_resident<T>(p, st, L, sv, ws, o, lds, early, batch, tol_scalar, tolv, done,
                                  count, noalloc, res_qp ? qp : nullptr,
@@ -1051,7 +1121,7 @@ static int solve_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T* 
   if ((rc = check_capture<T>(p, st, o, false))) return rc;
   Layout L;
   char *sv, *ws;
-  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false, 0, false, &o))) return rc;
+  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false, kLayoutWide, false, &o))) return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m;
   write_header<T>(st, sv, batch, Bp, 0, o.shared_bounds, p);
   to_minor<T>(st, target, batch, n, n, (T*)(sv + L.Tt), Bp, nullptr, 0);
@@ -1108,7 +1178,9 @@ static int project_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T
                          " iterations) in the no-allocation entry point");
   if ((rc = check_capture<T>(p, st, o, per_sample))) return rc;
   if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, per_sample,
-                               mult0 ? kLayoutWarm : 0, noalloc, &o)))
+                               (mult0 ? kLayoutWarm : 0) |
+                                   (per_sample || noalloc ? 0 : kLayoutWide),
+                               noalloc, &o)))
     return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m, M = p->M;
   constexpr int64_t TS = tile_samples<T>();
@@ -1374,8 +1446,8 @@ int64_t purin_cp_workspace_bytes(const purin_cp_plan* p, int32_t entry, int64_t 
   };
   switch (entry) {
     case PURIN_CP_ENTRY_SPMM: return forward(false, kLayoutSpmm);
-    case PURIN_CP_ENTRY_SOLVE: return forward(false, 0);
-    case PURIN_CP_ENTRY_PROJECT: return forward(false, kLayoutWarm);
+    case PURIN_CP_ENTRY_SOLVE: return forward(false, kLayoutWide);
+    case PURIN_CP_ENTRY_PROJECT: return forward(false, kLayoutWarm | kLayoutWide);
     case PURIN_CP_ENTRY_PROJECT_VALUES:
     case PURIN_CP_ENTRY_QP_SOLVE:
     case PURIN_CP_ENTRY_DENSE_SOLVE: return forward(true, kLayoutWarm);

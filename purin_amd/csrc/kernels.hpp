@@ -723,6 +723,33 @@ __global__ void k_fill(T* p, int64_t count, T v) {
     p[i] = v;
 }
 
+// A 64 x 64 tile through LDS: rows k0 .. k0 + 63 of a batch-minor array (get(k, b),
+// lanes over samples) to put(k, b, value) with lanes over k.
+template <typename T, typename Get, typename Put>
+__device__ __forceinline__ void minor_to_major_tile(int64_t K, int64_t batch, Get get, Put put) {
+  __shared__ T tile[64][65];
+  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+  const int64_t k0 = (int64_t)blockIdx.x * 64, b0 = (int64_t)blockIdx.y * 64;
+#pragma unroll 4
+  for (int r = ty; r < 64; r += kBlock / 64)
+    tile[r][tx] = k0 + r < K && b0 + tx < batch ? get(k0 + r, b0 + tx) : T(0);
+  __syncthreads();
+#pragma unroll 4
+  for (int r = ty; r < 64; r += kBlock / 64)
+    if (b0 + r < batch && k0 + tx < K) put(k0 + tx, b0 + r, tile[tx][r]);
+}
+
+// dst[b * K + k] = src[map[k] * Bp + b], 0 where map[k] < 0 (sample-major, gathered)
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_to_major_map(const T* __restrict__ src, int64_t Bp,
+                                                        const int32_t* __restrict__ map, int64_t K,
+                                                        int64_t batch, T* __restrict__ dst) {
+  minor_to_major_tile<T>(
+      K, batch,
+      [&](int64_t k, int64_t b) -> T { return map[k] < 0 ? T(0) : src[(size_t)map[k] * Bp + b]; },
+      [&](int64_t k, int64_t b, T v) { dst[b * K + k] = v; });
+}
+
 // Kept-row data from the full rows: R[i] = RF[kept[i]] * scale_i and
 // D[i] = MF[kept[i]] / scale_i (bounds.py:230-239).
 template <typename T>

@@ -458,6 +458,227 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
 }
 
 // ---------------------------------------------------------------------------
+// Several rows and columns per thread: y, d and two copies of K y in LDS, the matrix, the
+// targets, right-hand sides and bounds streamed from L2 (coalesced, in slice order).  The
+// streaming passes it stands in for pad a batch to 128 (fp64) or 256 (fp32) samples and
+// take four to six launches an iteration, and their time does not fall with the batch.
+// What bounds it is the latency of those streams, so a wavefront keeps the loads of
+// four slices in flight.
+// ---------------------------------------------------------------------------
+constexpr int kWideU = 4;  // slices of a wavefront in flight
+
+// sums of slices s0, s0 + 16, ... (kWideU of them): acc[u] = entries times x
+template <typename T>
+__device__ __forceinline__ void wide_sums(int s0, int ns, const int32_t* __restrict__ off,
+                                          const uint16_t* __restrict__ idx,
+                                          const T* __restrict__ val, const T* x,
+                                          T (&acc)[kWideU]) {
+  const int lane = threadIdx.x & 63;
+  int o[kWideU], w[kWideU];
+#pragma unroll
+  for (int u = 0; u < kWideU; ++u) {
+    const int s = s0 + 16 * u;
+    o[u] = s < ns ? off[s] : 0;
+    w[u] = s < ns ? (off[s + 1] - o[u]) >> 6 : 0;
+    acc[u] = T(0);
+  }
+  // slices are in decreasing width, so the first is the widest of the four
+  for (int k = 0; k < w[0]; k += 4) {
+    T v[kWideU][4];
+    int e[kWideU][4];
+#pragma unroll
+    for (int u = 0; u < kWideU; ++u) {
+      if (k >= w[u]) continue;
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const int at = o[u] + (k + h < w[u] ? k + h : w[u] - 1) * 64 + lane;
+        v[u][h] = val[at];
+        e[u][h] = idx[at];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kWideU; ++u) {
+      if (k >= w[u]) continue;
+#pragma unroll
+      for (int h = 0; h < 4; ++h)
+        if (k + h < w[u]) acc[u] = __builtin_elementwise_fma(v[u][h], x[e[u][h]], acc[u]);
+    }
+  }
+}
+
+template <typename T, bool EARLY>
+__global__ __launch_bounds__(1024) void k_solo_wide(SoloWide<T> A) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int64_t b = blockIdx.x, Bp = A.Bp;
+  const int n = A.n, m = A.m;
+  if (b >= A.batch) {
+    for (int e = t; e < n; e += 1024) A.Y[(int64_t)e * Bp + b] = T(0);
+    for (int e = t; e < m; e += 1024) A.D[(int64_t)e * Bp + b] = T(0);
+    return;
+  }
+  const T zero = T(0), one = T(1), half = T(0.5), inf = T(__builtin_inf());
+  T* Gy = reinterpret_cast<T*>(lds);  // y [n] | zero
+  T* Gd = Gy + n + 1;                 // d+ [m] | zero
+  T* KY = Gd + m + 1;                 // K y of the previous y [m]
+  // K y+ waits for the stop test's verdict in registers where a wavefront has one group of
+  // row slices (m <= 4096), else in LDS
+  const bool one_group = A.nsr <= 16 * kWideU;
+  T* KN = KY + m;
+  T* red = KN + (EARLY && !one_group ? m : 0);  // [16][4]
+  const T* TG = A.TG + (size_t)b * n;
+  const T* RR = A.RR + (size_t)b * m;
+  const T* LO = A.LO + (size_t)b * A.bstride;
+  const T* HI = A.HI + (size_t)b * A.bstride;
+  for (int e = t; e < n; e += 1024) Gy[e] = TG[e];  // y0 = ybar0 = yhat
+  for (int e = t; e < m; e += 1024) Gd[e] = A.D[(int64_t)A.rperm[e] * Bp + b];
+  if (t == 0) Gy[n] = Gd[m] = zero;
+  __syncthreads();
+  typedef const __attribute__((address_space(4))) T* CP;
+  const CP sched = (CP)A.sched;
+  // K y0 and the first d+
+  {
+    const T sigma = sched[0];
+    for (int s0 = wave; s0 < A.nsr; s0 += 16 * kWideU) {
+      T acc[kWideU];
+      wide_sums(s0, A.nsr, A.roff, A.ridx, A.rval, Gy, acc);
+#pragma unroll
+      for (int u = 0; u < kWideU; ++u) {
+        const int i = (s0 + 16 * u) * 64 + lane;
+        if (s0 + 16 * u >= A.nsr || i >= m) continue;
+        T p = Gd[i] + sigma * (acc[u] - RR[i]);
+        if (A.rperm[i] >= A.me) p = res_pos(p);
+        Gd[i] = p;
+        KY[i] = acc[u];
+      }
+    }
+  }
+  __syncthreads();
+  const T tol = EARLY ? (A.tolv ? A.tolv[b] : A.tol) : zero;
+  bool accepted = false;
+  int64_t it = 0;
+  for (; it < A.iters; ++it) {
+    const T a = sched[4 * it + 1], delta = sched[4 * it + 2], theta = sched[4 * it + 3];
+    const bool more = it + 1 < A.iters;
+    const T sigma_n = more ? sched[4 * (it + 1)] : zero;
+    T pri = zero, dual = zero, mx = zero;
+    // ---- column pass: y+ and its diagnostics
+    for (int s0 = wave; s0 < A.nsc; s0 += 16 * kWideU) {
+      T tg[kWideU], lo[kWideU], hi[kWideU], acc[kWideU];
+#pragma unroll
+      for (int u = 0; u < kWideU; ++u) {
+        const int j = (s0 + 16 * u) * 64 + lane;
+        const bool in = s0 + 16 * u < A.nsc && j < n;
+        tg[u] = in ? TG[j] : zero;
+        lo[u] = in ? LO[j] : zero;
+        hi[u] = in ? HI[j] : zero;
+      }
+      wide_sums(s0, A.nsc, A.coff, A.cidx, A.cval, Gd, acc);
+#pragma unroll
+      for (int u = 0; u < kWideU; ++u) {
+        const int j = (s0 + 16 * u) * 64 + lane;
+        if (s0 + 16 * u >= A.nsc || j >= n) continue;
+        const T tt = acc[u];
+        const bool odd = lo[u] != lo[u] || hi[u] != hi[u] || lo[u] > hi[u];
+        const T s = a * Gy[j] - delta * tt + delta * tg[u];
+        const T yn = odd ? clipp(s, lo[u], hi[u]) : res_clip(s, lo[u], hi[u]);
+        Gy[j] = yn;
+        if constexpr (EARLY) {  // as in k_solo
+          const T cq = -tg[u], tf = cq + tt;
+          pri += half * yn * yn + cq * yn;
+          if (!odd) {
+            const T mz = __builtin_fmin(__builtin_fmax(-tf, lo[u]), hi[u]);
+            dual += half * mz * mz + tf * mz;
+            mx = __builtin_fmax(mx, absv(yn - mz));
+          } else {
+            const T mz = clipp(-tf, lo[u], hi[u]);
+            dual += half * mz * mz + tf * mz;
+            const T xs = yn - ((yn + cq) + tt);
+            T g = maxp(absv(yn - clipp(xs, lo[u], hi[u])),
+                       maxp(maxp(lo[u] - yn, zero), maxp(yn - hi[u], zero)));
+            if (!finite(g)) g = inf;
+            mx = __builtin_fmax(mx, g);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // ---- row pass: K y+, the residual, and the next d+ from K ybar = (1 + theta) K y+ -
+    // theta K y (with the stop test after its verdict: the thread's own rows)
+    T kn[kWideU];
+    for (int s0 = wave; s0 < A.nsr; s0 += 16 * kWideU) {
+      T rr[kWideU], acc[kWideU];
+#pragma unroll
+      for (int u = 0; u < kWideU; ++u) {
+        const int i = (s0 + 16 * u) * 64 + lane;
+        rr[u] = s0 + 16 * u < A.nsr && i < m ? RR[i] : zero;
+      }
+      wide_sums(s0, A.nsr, A.roff, A.ridx, A.rval, Gy, acc);
+#pragma unroll
+      for (int u = 0; u < kWideU; ++u) {
+        const int i = (s0 + 16 * u) * 64 + lane;
+        if (s0 + 16 * u >= A.nsr || i >= m) continue;
+        const T d = Gd[i];
+        const bool ineq = A.rperm[i] >= A.me;
+        if constexpr (EARLY) {
+          const T e = acc[u] - rr[u], w = ineq ? zero : -one;
+          mx = __builtin_fmax(mx, __builtin_fmax(e, w * e));
+          dual = (dual - rr[u] * d) - d * zero;
+          kn[u] = acc[u];
+          if (!one_group) KN[i] = acc[u];
+        } else if (more) {
+          T p = d + sigma_n * (((one + theta) * acc[u] - theta * KY[i]) - rr[u]);
+          if (ineq) p = res_pos(p);
+          Gd[i] = p;
+          KY[i] = acc[u];
+        }
+      }
+    }
+    if constexpr (EARLY) {
+      const T s2 = two_sums(pri, dual);
+      const T wm = wave_fmax(mx);
+      if ((lane & 31) == 0) red[wave * 4 + (lane >> 5)] = s2;
+      if (lane == 0) red[wave * 4 + 2] = wm;
+      __syncthreads();
+      const T* rl = red + (lane & 15) * 4;
+      const T xp = row16_combine(rl[0], OpAdd()), xd = row16_combine(rl[1], OpAdd());
+      const T xm = row16_combine(rl[2], OpFMax());
+      const T gap = maxp(xp - xd, zero) / maxp(one, maxp(absv(xp), absv(xd)));
+      // the 64 lanes hold the four rows' identical totals in each row's lane 0
+      if (__builtin_amdgcn_readfirstlane(finite(gap) && xm <= tol && gap <= tol ? 1 : 0)) {
+        accepted = true;
+        ++it;
+        break;
+      }
+      auto move = [&](int s, T acc) {
+        const int i = s * 64 + lane;
+        if (s >= A.nsr || i >= m) return;
+        T p = Gd[i] + sigma_n * (((one + theta) * acc - theta * KY[i]) - RR[i]);
+        if (A.rperm[i] >= A.me) p = res_pos(p);
+        Gd[i] = p;
+        KY[i] = acc;
+      };
+      if (more && one_group) {
+#pragma unroll
+        for (int u = 0; u < kWideU; ++u) move(wave + 16 * u, kn[u]);
+      } else if (more) {
+        for (int s = wave; s < A.nsr; s += 16)
+          move(s, s * 64 + lane < m ? KN[s * 64 + lane] : zero);
+      }
+    }
+    __syncthreads();
+  }
+  __syncthreads();
+  for (int e = t; e < n; e += 1024) A.Y[(int64_t)A.cperm[e] * Bp + b] = Gy[e];
+  for (int e = t; e < m; e += 1024) A.D[(int64_t)A.rperm[e] * Bp + b] = Gd[e];
+  if (EARLY && t == 0) {
+    A.count[b] = (int32_t)it;
+    A.done[b] = accepted ? 1 : 0;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // The dense adapter (dense.py:85-106): rows and columns of tens of entries, so several lanes
 // share each, and the loop runs until the last sample is accepted.  The streaming passes
 // walked each row serially on a few wavefronts: 244 us per iteration at n = 60, m = 37,
@@ -801,6 +1022,33 @@ int solo_launch(hipStream_t st, const purin_cp_plan* p, const Solo<T>& A, int mo
     default: return launch_mode<T, kSoloQP>(st, A, k, lds, early);
   }
 }
+
+static size_t wide_lds(const purin_cp_plan* p, bool early) {
+  const int64_t vectors = early && p->sl_nsr > 16 * kWideU ? 3 : 2;  // d, K y (and K y+)
+  return (size_t)(p->n + 1 + 1 + vectors * p->m + 64) * elem_size(p);
+}
+
+// Problems beyond the tile kernels.  us per iteration with the stop test / without, against
+// the streaming passes: n = 12001 (flow, m = 3001) fp32 13.4 / 9.9 at B = 64 (107 / 23.5),
+// 55.9 / 40.1 at B = 1024 (162 / 59.8); n = 6000, m = 2100 fp64 12.6 / 10.1 (85.6 / 17.9) and
+// 51.4 / 40.5 (140 / 59.1).  Fixed iterations of more than 4096 rows stay on the passes,
+// whose narrow column tiles serve them.
+bool solo_wide_fits(const purin_cp_plan* p, bool early) {
+  if (!p->sl_ok || p->res_ok || p->diag || p->m < 1) return false;
+  if (!early && p->sl_nsr > 16 * kWideU) return false;
+  return wide_lds(p, early) <= 160 * 1024;
+}
+
+template <typename T>
+int solo_wide_launch(hipStream_t st, const purin_cp_plan* p, const SoloWide<T>& A, bool early) {
+  const size_t lds = wide_lds(p, early);
+  auto kern = early ? k_solo_wide<T, true> : k_solo_wide<T, false>;
+  if (int rc = raise_lds_cap((const void*)kern, lds)) return rc;
+  kern<<<(unsigned)A.Bp, 1024, lds, st>>>(A);
+  return PURIN_CP_OK;
+}
+template int solo_wide_launch<double>(hipStream_t, const purin_cp_plan*, const SoloWide<double>&, bool);
+template int solo_wide_launch<float>(hipStream_t, const purin_cp_plan*, const SoloWide<float>&, bool);
 
 // Lanes per row (log2) and entries per lane for rows of up to ``width`` entries.
 static void dense_lanes(int width, int* l, int* entries) {

@@ -59,6 +59,39 @@ bool solo_fits(const purin_cp_plan* p, int64_t batch, bool early, bool values);
 template <typename T>
 int solo_launch(hipStream_t st, const purin_cp_plan* p, const Solo<T>& A, int mode, bool early);
 
+// The projection's loop for problems whose vectors fill a CU's LDS (Solo's fields; the
+// thread walks several rows and columns).  Targets, right-hand sides and bounds are
+// sample-major in slice order: each is read every iteration.
+template <typename T>
+struct SoloWide {
+  int n, m, me;
+  int64_t Bp, batch, iters;
+  int nsr, nsc;
+  const int32_t* __restrict__ roff;
+  const int32_t* __restrict__ coff;
+  const int32_t* __restrict__ rperm;
+  const int32_t* __restrict__ cperm;
+  const uint16_t* __restrict__ ridx;
+  const uint16_t* __restrict__ cidx;
+  const T* __restrict__ rval;
+  const T* __restrict__ cval;
+  const T* __restrict__ TG;   // [batch][n]
+  const T* __restrict__ RR;   // [batch][m]
+  const T* __restrict__ LO;   // [n], or [batch][n] (bstride n)
+  const T* __restrict__ HI;
+  int64_t bstride;
+  const T* __restrict__ sched;
+  T tol;
+  const T* __restrict__ tolv;
+  int32_t* done;
+  int32_t* count;
+  T* Y;
+  T* D;
+};
+bool solo_wide_fits(const purin_cp_plan* p, bool early);
+template <typename T>
+int solo_wide_launch(hipStream_t st, const purin_cp_plan* p, const SoloWide<T>& A, bool early);
+
 // The dense adapter's loop (factored prox, no freezing, no stationarity test): every sample
 // iterates until the last is accepted.  A row is shared by 2^lr lanes, a column by 2^lc.
 template <typename T>

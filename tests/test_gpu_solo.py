@@ -121,3 +121,42 @@ def test_solo_values_and_qp_match_streaming(n, me, mi, B, early):
             np.testing.assert_array_equal(to_np(a.iterations), to_np(s.iterations))
             assert rel_err(to_np(a.y), to_np(s.y)) <= 1e-10
             assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= 1e-10
+
+
+@pytest.mark.parametrize("n,me,mi,B,dtype", [
+    (4097, 60, 200, 3, np.float64),     # just beyond the tile kernels
+    (4200, 500, 3596, 2, np.float64),   # 4096 rows: K y+ in registers, both loops
+    (4200, 500, 3597, 2, np.float64),   # 4097: K y+ in LDS; fixed iterations on the passes
+    (15000, 100, 300, 2, np.float64),
+    (9000, 700, 1500, 66, np.float32),
+    (30000, 500, 1500, 2, np.float32),
+])
+def test_solo_wide_matches_streaming(n, me, mi, B, dtype):
+    """Several rows and columns per thread (k_solo_wide), against the streaming passes."""
+    require_gpu()
+    w = workloads.ragged_rows(800, n=n, me=me, mi=mi, wmin=2, wmax=9, batch=B)
+    from purin_amd.plan import Plan
+
+    rhs = np.tile(w.rhs, (B, 1)).astype(dtype)
+    target = w.target.astype(dtype)
+    bar = TOL[dtype]
+    scaled = rhs.copy()
+    scaled[:, me + mi:] *= np.linspace(0.8, 1.2, B).astype(dtype)[:, None]
+    for accelerated in (False, True):
+        plan = Plan(n, me, w.rows_total - me, w.indptr, w.indices, w.data, dtype=dtype,
+                    accelerated=accelerated)
+        for r, shared in ((rhs, True), (scaled, False)):
+            kw = dict(max_iterations=80, early_stop=False, shared_bounds=shared, timing=True)
+            a = plan.project(target, r, **kw)
+            assert plan.last_timing()["resident"] == (1 if me + mi <= 4096 else 0)
+            s = plan.project(target, r, streaming=True, **kw)
+            assert rel_err(to_np(a.y), to_np(s.y)) <= bar / 10
+            assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= bar
+            kw = dict(max_iterations=400, tolerance=5e-2, shared_bounds=shared, timing=True)
+            a = plan.project(target, r, **kw)
+            assert plan.last_timing()["resident"] == 1
+            s = plan.project(target, r, streaming=True, **kw)
+            same = to_np(a.iterations) == to_np(s.iterations)
+            assert same.all() if dtype == np.float64 else same.mean() >= 0.9
+            assert rel_err(to_np(a.y)[same], to_np(s.y)[same]) <= bar
+            assert rel_err(to_np(a.multipliers)[same], to_np(s.multipliers)[same]) <= bar
