@@ -213,7 +213,23 @@ __global__ __launch_bounds__(256) void k_ps_dots(int64_t R, int64_t Bp, const T*
   const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= Bp) return;
   T s1 = T(0), s2 = T(0);
-  for (int64_t r = 0; r < R; ++r) {
+  // 16 rows' loads in flight: a load per addition was 0.27 us a row (160 us a call at R =
+  // 600, twenty calls a norm estimate)
+  int64_t r = 0;
+  for (; r + 16 <= R; r += 16) {
+    T xv[16], yv[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      yv[k] = y[(r + k) * Bp + b];
+      xv[k] = x ? x[(r + k) * Bp + b] : T(0);
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (x) s1 = s1 + xv[k] * yv[k];
+      s2 = s2 + yv[k] * yv[k];
+    }
+  }
+  for (; r < R; ++r) {
     const T yv = y[r * Bp + b];
     if (x) s1 = s1 + x[r * Bp + b] * yv;
     s2 = s2 + yv * yv;
