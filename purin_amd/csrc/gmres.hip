@@ -156,15 +156,32 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// The sum of v over lanes l and l ^ 32, in both
+template <typename T>
+__device__ __forceinline__ T both_halves(T v) {
+  return swap_add<32>(v, v);
+}
+
+// v of lane l (wave-uniform l), as a scalar
+template <typename T>
+__device__ __forceinline__ T lane_value(T v, int l) {
+  constexpr int N = Words<T>::N;
+  typedef int U __attribute__((ext_vector_type(N)));
+  U x = __builtin_bit_cast(U, v);
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = __builtin_amdgcn_readlane(x[i], l);
+  return __builtin_bit_cast(T, x);
+}
+
 // --- LDS of one workgroup ---------------------------------------------------------
 
 // Elements: u [n + 1], w [m + 1], the wavefronts' partial sums [BS / 64][33], shares of
 // slices [BS], then per-sample algebra (below), then the basis where it fits.
-constexpr int kAlg = 3 * kLd * kLd + 10 * kLd;
+constexpr int kAlg = 3 * kLd * kLd + 9 * kLd;
 
 template <typename T>
 struct Alg {  // pointers into the algebra block
-  T *Tm, *Hu, *H, *P, *Gv, *Q, *U2, *G1, *Cs, *Sn, *g, *Col, *Wc;
+  T *Tm, *Hu, *H, *P, *Gv, *Q, *U2, *G1, *Cs, *Sn, *g, *Wc;
   __device__ explicit Alg(T* p) {
     Tm = p;                 // [i][j], upper triangular
     Hu = Tm + kLd * kLd;    // unrotated Hessenberg matrix
@@ -177,8 +194,7 @@ struct Alg {  // pointers into the algebra block
     Cs = G1 + kLd;
     Sn = Cs + kLd;
     g = Sn + kLd;
-    Col = g + kLd;
-    Wc = Col + kLd;
+    Wc = g + kLd;
   }
 };
 
@@ -418,6 +434,9 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
     apply<T, BS, DG>(A, b, Z + (int64_t)it * ld, s_inv, y, u, w, share);
     pass<T, BS, false>(Z, ldb, nv, y, W, S.Q, red);
     __syncthreads();
+    // The algebra runs on one wavefront: lanes j and j + 32 share vector j's sums (even
+    // and odd terms), which halves their chains of LDS reads.
+    const int vj = lane & 31, half = lane >> 5;
     if (wave == 0) {  // p = Z^T y; g1 = Tm^T p; q1 = Tm g1
       if (lane < nv) {
         T s = T(0);
@@ -426,19 +445,21 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
         S.P[lane] = s;
       }
       wave_sync();
-      if (lane < nv) {
-        T s = T(0);
+      T s = T(0);
+      if (vj < nv) {
 #pragma unroll 8
-        for (int i = 0; i <= lane; ++i) s += S.Tm[i * kLd + lane] * S.P[i];
-        S.G1[lane] = s;
+        for (int i = half; i <= vj; i += 2) s += S.Tm[i * kLd + vj] * S.P[i];
       }
+      s = both_halves(s);
+      if (lane < nv) S.G1[lane] = s;
       wave_sync();
-      if (lane < nv) {
-        T s = T(0);
+      s = T(0);
+      if (vj < nv) {
 #pragma unroll 8
-        for (int j = lane; j < nv; ++j) s += S.Tm[lane * kLd + j] * S.G1[j];
-        S.Q[lane] = s;
+        for (int j = vj + half; j < nv; j += 2) s += S.Tm[vj * kLd + j] * S.G1[j];
       }
+      s = both_halves(s);
+      if (lane < nv) S.Q[lane] = s;
     }
     __syncthreads();
     pass<T, BS, true>(Z, ldb, nv, y, W, S.Q, red);
@@ -451,30 +472,39 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
         S.P[lane] = s;
       }
       wave_sync();
-      T g2 = T(0);
+      T g2 = T(0), cj = T(0);
+      if (vj < nv) {
+#pragma unroll 8
+        for (int i = half; i <= vj; i += 2) g2 += S.Tm[i * kLd + vj] * S.P[i];
+#pragma unroll 8
+        for (int k = (vj > 0 ? vj - 1 : 0) + half; k < it; k += 2)
+          cj += S.Hu[vj * kLd + k] * S.U2[k];
+      }
+      g2 = both_halves(g2);
+      cj = both_halves(cj);
+      T col = T(0), rc_ = T(0), rs_ = T(0);
       if (lane < nv) {
-#pragma unroll 8
-        for (int i = 0; i <= lane; ++i) g2 += S.Tm[i * kLd + lane] * S.P[i];
         S.Gv[lane] = g2;
-        T cj = T(0);
-#pragma unroll 8
-        for (int k = lane > 0 ? lane - 1 : 0; k < it; ++k) cj += S.Hu[lane * kLd + k] * S.U2[k];
-        const T col = (S.G1[lane] + g2) - cj;
-        S.Col[lane] = col;
+        col = (S.G1[lane] + g2) - cj;
         S.Hu[lane * kLd + it] = col;
+        rc_ = S.Cs[lane];
+        rs_ = S.Sn[lane];
       }
       wave_sync();
       const T ss = fold<32>(lane < nv ? g2 * g2 : T(0));
       const T n1 = S.P[kLd - 1];
       const T d2 = n1 - ss;
       const T next_norm = d2 < T(0) ? T(0) : __builtin_sqrt(d2);  // NaN stays NaN
-      // the rotations of the earlier steps, in order, on every lane alike
-      T carry = S.Col[0];
+      // the rotations of the earlier steps, in order, on every lane alike, from the
+      // registers of the lanes that hold them
+      T carry = lane_value(col, 0), hcol = T(0);
       for (int ri = 0; ri < it; ++ri) {
-        const T cc = S.Cs[ri], sn = S.Sn[ri], nx = S.Col[ri + 1];
-        if (lane == 0) S.H[ri * kLd + it] = cc * carry + sn * nx;
+        const T cc = lane_value(rc_, ri), sn = lane_value(rs_, ri), nx = lane_value(col, ri + 1);
+        const T h = cc * carry + sn * nx;
+        hcol = lane == ri ? h : hcol;
         carry = -sn * carry + cc * nx;
       }
+      if (lane < it) S.H[lane * kLd + it] = hcol;
       const T rnorm = hypotv(carry, next_norm);
       const T safe = maxp(rnorm, eps);
       const T nc = rnorm > eps ? carry / safe : T(1);
@@ -486,10 +516,11 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
       const bool on = finite(est) && finite(rnorm) && finite(n1) && !(next_norm <= brk) && est > thr;
       // column it + 1 of Tm: v_{it+1} = (Z_{it+1} - Z Tm g2) / nu, and u = g2 / nu
       T tc = T(0);
-      if (lane < nv) {
+      if (vj < nv) {
 #pragma unroll 8
-        for (int j = lane; j < nv; ++j) tc += S.Tm[lane * kLd + j] * S.Gv[j];
+        for (int j = vj + half; j < nv; j += 2) tc += S.Tm[vj * kLd + j] * S.Gv[j];
       }
+      tc = both_halves(tc);
       wave_sync();
       if (lane < nv) {
         S.Tm[lane * kLd + nv] = -(tc * inv);
