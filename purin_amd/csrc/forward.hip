@@ -35,6 +35,16 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
   const size_t n = p->n, m = p->m, M = p->M, mi = p->mi;
   L.nrb = (int)((m + 4 * kRowsPerWaveEarly - 1) / (4 * kRowsPerWaveEarly));
   L.ncb = (int)((n + 4 * kRowsPerWaveEarly - 1) / (4 * kRowsPerWaveEarly));
+  // The passes that leave partials take 8 rows or columns per wavefront, one after the
+  // other; small problems, where that leaves CUs idle, take one (n = 24, batch 1: column
+  // diagnostics 20.6 -> 7.6 us, row diagnostics 17.5 -> 6.8, multiplier recovery 30.5 ->
+  // 7.8 and 10.6 -> 4.6).  Not beyond 1024 columns: the per-sample folds walk the blocks'
+  // partials one after the other.
+  const int64_t tiles = L.Bp / (es == 8 ? tile_samples<double>() : tile_samples<float>());
+  const bool fine = (extras & kLayoutFine) && n <= 1024 && m <= 1024 && L.ncb * tiles < 256;
+  L.cpw = fine ? 1 : kRowsPerWaveEarly;
+  L.ncd = (int)((n + 4 * L.cpw - 1) / (4 * L.cpw));
+  L.nrd = (int)((m + 4 * L.cpw - 1) / (4 * L.cpw));
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t r = o; o = al(o + bytes); return r; };
   L.hdr = take(kSavedHeader);
@@ -53,8 +63,8 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
   L.MF = (extras & kLayoutWarm) ? take(M * Bp * es) : 0;
   L.DF = take(M * Bp * es);
   L.SL = take(mi * Bp * es);
-  L.colpart = take((size_t)5 * std::max(L.ncb, 1) * Bp * es);
-  L.rowpart = take((size_t)3 * std::max(L.nrb, 1) * Bp * es);
+  L.colpart = take((size_t)5 * std::max(L.ncd, 1) * Bp * es);
+  L.rowpart = take((size_t)3 * std::max(L.nrd, 1) * Bp * es);
   L.decpart = take((size_t)8 * kDecideSplit * Bp * es);  // k_decide's split pre-pass
   L.done = take(Bp * 4);
   L.count = take(Bp * 4);
@@ -618,6 +628,36 @@ static int run_resident(purin_cp_plan* p, hipStream_t st, const Layout& L, char*
   return finish_resident(p, st, o, e0, e1);
 }
 
+// The passes that leave partials, at the layout's rows / columns per wavefront.
+template <typename T, int MODE>
+static void diag_cols(hipStream_t st, const Iter<T>& A, const Layout& L) {
+  const dim3 g = tile_grid(L.Bp, tile_samples<T>(), L.ncd);
+  if (L.cpw == 1)
+    k_col_pass<T, MODE, 1><<<g, kBlock, 0, st>>>(A);
+  else
+    k_col_pass<T, MODE, kRowsPerWaveEarly><<<g, kBlock, 0, st>>>(A);
+}
+template <typename T>
+static void diag_rows(hipStream_t st, const Iter<T>& A, const Layout& L) {
+  const dim3 g = tile_grid(L.Bp, tile_samples<T>(), std::max(L.nrd, 1));
+  if (L.cpw == 1)
+    k_res_pass<T, 1><<<g, kBlock, 0, st>>>(A);
+  else
+    k_res_pass<T, kRowsPerWaveEarly><<<g, kBlock, 0, st>>>(A);
+}
+template <typename T>
+static void post_passes(hipStream_t st, const Post<T>& P, const Layout& L, int64_t m) {
+  constexpr int64_t TS = tile_samples<T>();
+  const dim3 gr = tile_grid(L.Bp, TS, L.nrd), gc = tile_grid(L.Bp, TS, L.ncd);
+  if (L.cpw == 1) {
+    if (m) k_post_rows<T, 1><<<gr, kBlock, 0, st>>>(P);
+    k_post_cols<T, 1><<<gc, kBlock, 0, st>>>(P);
+  } else {
+    if (m) k_post_rows<T, kRowsPerWaveEarly><<<gr, kBlock, 0, st>>>(P);
+    k_post_cols<T, kRowsPerWaveEarly><<<gc, kBlock, 0, st>>>(P);
+  }
+}
+
 // The CP loop on prepared internal arrays plus the final diagnostics.
 template <typename T>
 int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout& L, char* sv,
@@ -639,8 +679,8 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
   A.shared_bounds = o.shared_bounds;
   A.colpart = (T*)(ws + L.colpart);
   A.rowpart = (T*)(ws + L.rowpart);
-  A.ncb = L.ncb;
-  A.nrb = L.nrb;
+  A.ncb = L.ncd;
+  A.nrb = L.nrd;
   if (ps) {  // per-sample coefficients: per-sample matrix entries and steps
     if (ps->RVs) {  // the plan's own coefficients: one shared copy
       A.K.rval = ps->RVs;
@@ -713,11 +753,9 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
     A.TK = A.YB;
     A.KYo = (T*)(ws + L.DF);
     A.kyrow = p->dkept;
-    const dim3 gcolE0 = tile_grid(Bp, TS, L.ncb);
-    const dim3 gres0 = tile_grid(Bp, TS, std::max(L.nrb, 1));
     const dim3 gdec0((unsigned)(Bp / 64));  // k_decide: 64 samples per block
-    k_col_pass<T, 2, kRowsPerWaveEarly><<<gcolE0, kBlock, 0, st>>>(A);
-    if (m) k_res_pass<T, kRowsPerWaveEarly><<<gres0, kBlock, 0, st>>>(A);
+    diag_cols<T, 2>(st, A, L);
+    if (m) diag_rows<T>(st, A, L);
     k_decide<T, true><<<gdec0, 64 * kDecideGroups, 0, st>>>(A, batch, tol_scalar, tolv, done, count, ndone,
                                                 (const int32_t*)(sv + L.feas), (T*)(ws + L.ores),
                                                 (T*)(ws + L.ogap), (int32_t*)(sv + L.conv),
@@ -757,7 +795,6 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
   T tau = (T)p->tau0, sigma = (T)p->sigma0, theta = one;
   const dim3 grow = tile_grid(Bp, TS, (m + 3) / 4);
   const dim3 gcol = tile_grid(Bp, TS, (n + 3) / 4);
-  const dim3 gcolE = tile_grid(Bp, TS, L.ncb);
   // The fixed-iteration column pass takes a quarter wavefront per column
   // (k_col_pass_q: batch tiles of TS / 4 samples) where the slice of d+ a
   // wide tile gathers exceeds an XCD's L2 and the narrow tile's fits with
@@ -771,7 +808,6 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
                      (double)m * (TS / 4) * sizeof(T) <= 0.625 * kL2Bytes &&
                      (Bp / (TS / 4)) % 8 == 0;
   const dim3 gcolq = tile_grid(Bp, TS / 4, (n + 15) / 16);
-  const dim3 gres = tile_grid(Bp, TS, std::max(L.nrb, 1));
   const dim3 gdec((unsigned)(Bp / 64));  // k_decide: 64 samples per block
   // With fewer than 16 such blocks the per-sample stop test folds its chunk
   // partials in two passes: (Bp / 64) x kDecideSplit blocks each fold every
@@ -878,9 +914,9 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
       k_snap<<<1, 64, 0, st>>>(ndone, snap);
       if (m) k_row_pass<T, false><<<grow, kBlock, 0, st>>>(A);
       if (timing) PURIN_HIP(hipEventRecord(ev[3 * it + 1], st));
-      k_col_pass<T, 1, kRowsPerWaveEarly><<<gcolE, kBlock, 0, st>>>(A);
+      diag_cols<T, 1>(st, A, L);
       if (timing) PURIN_HIP(hipEventRecord(evd[it], st));
-      if (m) k_res_pass<T, kRowsPerWaveEarly><<<gres, kBlock, 0, st>>>(A);
+      if (m) diag_rows<T>(st, A, L);
       decide();
     } else {
       A.done = done;
@@ -894,10 +930,10 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
         k_row_pass<T, true><<<grow, kBlock, 0, st>>>(A);
       }
       if (timing) PURIN_HIP(hipEventRecord(ev[3 * it + 1], st));
-      k_col_pass<T, 1, kRowsPerWaveEarly><<<gcolE, kBlock, 0, st>>>(A);
+      diag_cols<T, 1>(st, A, L);
       if (timing) PURIN_HIP(hipEventRecord(evd[it], st));
       if (lin) A.KYo = kyb[(it + 1) & 1];  // K y+ for the next iteration's row pass
-      if (m) k_res_pass<T, kRowsPerWaveEarly><<<gres, kBlock, 0, st>>>(A);
+      if (m) diag_rows<T>(st, A, L);
       A.KYo = nullptr;
       decide();
     }
@@ -962,8 +998,8 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
   A.TK = A.YB;
   A.KYo = (T*)(ws + L.DF);
   A.kyrow = p->dkept;
-  k_col_pass<T, 2, kRowsPerWaveEarly><<<gcolE, kBlock, 0, st>>>(A);
-  if (m) k_res_pass<T, kRowsPerWaveEarly><<<gres, kBlock, 0, st>>>(A);
+  diag_cols<T, 2>(st, A, L);
+  if (m) diag_rows<T>(st, A, L);
   k_decide<T, true><<<gdec, 64 * kDecideGroups, 0, st>>>(A, batch, tol_scalar, tolv, done, count, ndone,
                                              (const int32_t*)(sv + L.feas), (T*)(ws + L.ores),
                                              (T*)(ws + L.ogap), (int32_t*)(sv + L.conv),
@@ -1121,7 +1157,8 @@ static int solve_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T* 
   if ((rc = check_capture<T>(p, st, o, false))) return rc;
   Layout L;
   char *sv, *ws;
-  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false, kLayoutWide, false, &o))) return rc;
+  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false, kLayoutWide | kLayoutFine,
+                               false, &o))) return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m;
   write_header<T>(st, sv, batch, Bp, 0, o.shared_bounds, p);
   to_minor<T>(st, target, batch, n, n, (T*)(sv + L.Tt), Bp, nullptr, 0);
@@ -1179,7 +1216,8 @@ static int project_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T
   if ((rc = check_capture<T>(p, st, o, per_sample))) return rc;
   if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, per_sample,
                                (mult0 ? kLayoutWarm : 0) |
-                                   (per_sample || noalloc ? 0 : kLayoutWide),
+                                   (per_sample || noalloc ? 0 : kLayoutWide) |
+                                   (noalloc ? 0 : kLayoutFine),
                                noalloc, &o)))
     return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m, M = p->M;
@@ -1255,11 +1293,9 @@ static int project_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T
   P.SL = (T*)(ws + L.SL);
   P.rowpart = (T*)(ws + L.rowpart);
   P.colpart = (T*)(ws + L.colpart);
-  P.nrb = L.nrb;
-  P.ncb = L.ncb;
-  if (m)
-    k_post_rows<T, kRowsPerWaveEarly><<<tile_grid(Bp, TS, L.nrb), kBlock, 0, st>>>(P);
-  k_post_cols<T, kRowsPerWaveEarly><<<tile_grid(Bp, TS, L.ncb), kBlock, 0, st>>>(P);
+  P.nrb = L.nrd;
+  P.ncb = L.ncd;
+  post_passes<T>(st, P, L, m);
   k_post_final<T><<<(unsigned)(Bp / 64), 64 * kDecideGroups, 0, st>>>(
       P, batch, (T)tol_cfg, (T)factor, (const int32_t*)(sv + L.conv), (const T*)(ws + L.ogap),
       (const int32_t*)(ws + L.count), status, iterations, residual, finite_out, eligible);
@@ -1300,8 +1336,8 @@ static int qp_solve_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const 
   if ((rc = check_capture<T>(p, st, o, true))) return rc;
   Layout L;
   char *sv, *ws;
-  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, true, dual0 ? kLayoutWarm : 0,
-                               false, &o)))
+  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, true,
+                               (dual0 ? kLayoutWarm : 0) | kLayoutFine, false, &o)))
     return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m, M = p->M;
   constexpr int64_t TS = tile_samples<T>();
@@ -1369,11 +1405,9 @@ static int qp_solve_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const 
   P.SL = (T*)(ws + L.SL);
   P.rowpart = (T*)(ws + L.rowpart);
   P.colpart = (T*)(ws + L.colpart);
-  P.nrb = L.nrb;
-  P.ncb = L.ncb;
-  if (m)
-    k_post_rows<T, kRowsPerWaveEarly><<<tile_grid(Bp, TS, L.nrb), kBlock, 0, st>>>(P);
-  k_post_cols<T, kRowsPerWaveEarly><<<tile_grid(Bp, TS, L.ncb), kBlock, 0, st>>>(P);
+  P.nrb = L.nrd;
+  P.ncb = L.ncd;
+  post_passes<T>(st, P, L, m);
   k_post_final<T><<<(unsigned)(Bp / 64), 64 * kDecideGroups, 0, st>>>(
       P, batch, (T)o.tolerance, T(1), (const int32_t*)(sv + L.conv), (const T*)(ws + L.ogap),
       (const int32_t*)(ws + L.count), status, iterations, residual, finite_out, converged_out);
@@ -1446,11 +1480,11 @@ int64_t purin_cp_workspace_bytes(const purin_cp_plan* p, int32_t entry, int64_t 
   };
   switch (entry) {
     case PURIN_CP_ENTRY_SPMM: return forward(false, kLayoutSpmm);
-    case PURIN_CP_ENTRY_SOLVE: return forward(false, kLayoutWide);
-    case PURIN_CP_ENTRY_PROJECT: return forward(false, kLayoutWarm | kLayoutWide);
+    case PURIN_CP_ENTRY_SOLVE: return forward(false, kLayoutWide | kLayoutFine);
+    case PURIN_CP_ENTRY_PROJECT: return forward(false, kLayoutWarm | kLayoutWide | kLayoutFine);
     case PURIN_CP_ENTRY_PROJECT_VALUES:
     case PURIN_CP_ENTRY_QP_SOLVE:
-    case PURIN_CP_ENTRY_DENSE_SOLVE: return forward(true, kLayoutWarm);
+    case PURIN_CP_ENTRY_DENSE_SOLVE: return forward(true, kLayoutWarm | kLayoutFine);
     case PURIN_CP_ENTRY_ADJOINT:
     case PURIN_CP_ENTRY_ADJOINT_VALUES:
     case PURIN_CP_ENTRY_QP_ADJOINT:

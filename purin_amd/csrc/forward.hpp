@@ -11,6 +11,7 @@ namespace purin {
 struct Layout {
   int64_t Bp;
   int ncb, nrb;
+  int cpw, ncd, nrd;  // rows / columns per wavefront of the diagnostic passes, and their blocks
   // saved region
   size_t hdr, Tt, Y, D, R, LO, HI, RF, conv, feas, saved_end;
   // forward workspace
@@ -31,6 +32,7 @@ struct Layout {
 // Optional parts of the forward workspace.
 constexpr int kLayoutSpmm = 1;  // X, Z: purin_cp_spmm's batch-minor staging
 constexpr int kLayoutWarm = 2;  // MF: warm-start multipliers / duals in batch-minor layout
+constexpr int kLayoutFine = 8;  // one row / column per wavefront in small diagnostic passes
 constexpr int kLayoutWide = 4;  // WTG..WHI where the plan takes k_solo_wide
 
 Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values = false, int extras = 0);

@@ -160,3 +160,25 @@ def test_solo_wide_matches_streaming(n, me, mi, B, dtype):
             assert same.all() if dtype == np.float64 else same.mean() >= 0.9
             assert rel_err(to_np(a.y)[same], to_np(s.y)[same]) <= bar
             assert rel_err(to_np(a.multipliers)[same], to_np(s.multipliers)[same]) <= bar
+
+
+@pytest.mark.parametrize("n,me,mi,few,many,dtype", [
+    (24, 4, 9, 1, 16384, np.float64), (1021, 61, 120, 3, 1025, np.float64),
+    (1024, 0, 2, 2, 1025, np.float64), (333, 1, 0, 2, 6144, np.float32)])
+def test_final_passes_one_column_per_wavefront(n, me, mi, few, many, dtype):
+    """The final diagnostics and the multiplier recovery take one row and column per
+    wavefront in small batches of small problems and eight otherwise: a few samples alone
+    give what they give within a batch beyond the rule's line."""
+    require_gpu()
+    w = workloads.ragged_rows(50 + n, n=n, me=me, mi=mi, wmin=2, wmax=4, batch=many)
+    plan = plan_for(canonical_from_workload(w), dtype=dtype, accelerated=False)
+    rhs = np.tile(w.rhs, (many, 1)).astype(dtype)
+    target = w.target.astype(dtype)
+    kw = dict(shared_bounds=False, max_iterations=40, early_stop=False)
+    a = plan.project(target, rhs, **kw)
+    s = plan.project(target[:few], rhs[:few], **kw)
+    bar = TOL[dtype]
+    for f in ("y", "multipliers", "slacks", "residual"):
+        assert rel_err(to_np(getattr(s, f)), to_np(getattr(a, f))[:few]) <= bar, f
+    for f in ("status", "finite", "eligible", "iterations"):
+        np.testing.assert_array_equal(to_np(getattr(s, f)), to_np(getattr(a, f))[:few])
