@@ -106,6 +106,44 @@ __device__ __forceinline__ T wave_fmax(T a) {
 // Entries past the first W of every slice, in LDS.
 __host__ __device__ inline int rest_of(int width, int W) { return width > W ? width - W : 0; }
 
+// The wavefronts' partial terms of a lane, in order.  The loads of up to 8 wavefronts are in
+// flight together: one after the other they held up the iterations of all (us per iteration
+// with the stop test, fp64: n = 300 1.06 -> 0.81, n = 400 1.05 -> 0.75, n = 777 1.35 -> 1.10,
+// n = 950 1.31 -> 1.02; fp32 n = 777 1.16 -> 0.92).  Eight wavefronts or fewer go four at a
+// time: with all at once the burst delays the others' gathers (n = 500 0.95 -> 1.03).
+template <int N, typename T>
+__device__ __forceinline__ void add_some(const T* pt, int NT, T& pri, T& dual, T& mx) {
+  T a[N], b[N], c[N];
+#pragma unroll
+  for (int w = 0; w < N; ++w) {
+    a[w] = pt[w * 64];
+    b[w] = pt[NT + w * 64];
+    c[w] = pt[2 * NT + w * 64];
+  }
+#pragma unroll
+  for (int w = 0; w < N; ++w) {
+    pri += a[w];
+    dual += b[w];
+    mx = __builtin_fmax(mx, c[w]);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void add_parts(const T* pt, int NW, int NT, T& pri, T& dual, T& mx) {
+  if (NW > 8) {
+    add_some<8>(pt, NT, pri, dual, mx);
+    pt += 8 * 64;
+  }
+  for (int w = (NW > 8 ? NW - 8 : NW) >> 2; w > 0; --w) {
+    add_some<4>(pt, NT, pri, dual, mx);
+    pt += 4 * 64;
+  }
+  if (NW & 2) {
+    add_some<2>(pt, NT, pri, dual, mx);
+    pt += 2 * 64;
+  }
+  if (NW & 1) add_some<1>(pt, NT, pri, dual, mx);
+}
+
 // Up to 1024 threads, so up to 128 VGPRs.
 // HELP: the workgroup has one wavefront more than its rows or columns fill, for the stop test.
 template <typename T, int W, int MODE, bool EARLY, bool HELP>
@@ -316,18 +354,11 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
       if (it > 0) {
         const T* pt = red + ((it - 1) & 1) * 3 * NT + lane;
         mx = zero;
-        for (int w = 0; w < NW; ++w) {
-          pri += pt[w * 64];
-          dual += pt[NT + w * 64];
-          mx = __builtin_fmax(mx, pt[2 * NT + w * 64]);
-        }
-        const T s2 = two_sums(pri, dual);
-        pri = read_lane(s2, 0);
-        dual = read_lane(s2, 32);
-        mx = wave_fmax(mx);
+        add_parts(pt, NW, NT, pri, dual, mx);
       }
       __syncthreads();
-      const bool ok = judge(pri, dual, mx);
+      const T s2 = two_sums(pri, dual);
+      const bool ok = judge(read_lane(s2, 0), read_lane(s2, 32), wave_fmax(mx));
       if (lane == 0) *flag = ok ? 1 : 0;
       __syncthreads();
     }
@@ -830,11 +861,7 @@ __global__ __launch_bounds__(MAXB) void k_solo_dense(SoloDense<T> A) {
       if (it > 0) {
         const T* pt = red + ((it - 1) & 1) * 3 * NT + lane;
         mx = zero;
-        for (int w = 0; w < NW; ++w) {
-          pri += pt[w * 64];
-          dual += pt[NT + w * 64];
-          mx = __builtin_fmax(mx, pt[2 * NT + w * 64]);
-        }
+        add_parts(pt, NW, NT, pri, dual, mx);
         const T s2 = two_sums(pri, dual);
         pri = read_lane(s2, 0);
         dual = read_lane(s2, 32);
