@@ -67,6 +67,24 @@ def test_solo_matches_streaming(n, me, mi, wmin, wmax, B, dtype, accelerated):
         np.testing.assert_array_equal(to_np(a.status)[same], to_np(s.status)[same])
 
 
+@pytest.mark.parametrize("waves", [1, 2, 3, 7, 9, 10, 11, 12, 13, 14, 15])
+def test_stop_test_wavefront_sums_every_wavefront(waves):
+    """The stop test's wavefront adds the others' terms in groups of eight, four, two and
+    one: counts as on the streaming passes for every remainder."""
+    require_gpu()
+    B, n = 4, 64 * waves - 1
+    w = workloads.ragged_rows(90 + waves, n=n, me=n // 20 + 1, mi=n // 8 + 1, wmin=2, wmax=5,
+                              batch=B)
+    plan = plan_for(canonical_from_workload(w), dtype=np.float64)
+    rhs = np.tile(w.rhs, (B, 1))
+    kw = dict(max_iterations=600, tolerance=1e-2)
+    a = plan.project(w.target, rhs, **kw)
+    s = plan.project(w.target, rhs, streaming=True, **kw)
+    np.testing.assert_array_equal(to_np(a.iterations), to_np(s.iterations))
+    np.testing.assert_array_equal(to_np(a.status), to_np(s.status))
+    assert rel_err(to_np(a.y), to_np(s.y)) <= 1e-10
+
+
 @pytest.mark.parametrize("iters", [1, 2, 3])
 def test_solo_short_runs(iters):
     """The stop test trails the loop: runs that end before its first verdicts, and samples
