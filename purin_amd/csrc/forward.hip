@@ -40,11 +40,18 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
   // diagnostics 20.6 -> 7.6 us, row diagnostics 17.5 -> 6.8, multiplier recovery 30.5 ->
   // 7.8 and 10.6 -> 4.6).  Not beyond 1024 columns: the per-sample folds walk the blocks'
   // partials one after the other.
-  const int64_t tiles = L.Bp / (es == 8 ? tile_samples<double>() : tile_samples<float>());
-  const bool fine = (extras & kLayoutFine) && n <= 1024 && m <= 1024 && L.ncb * tiles < 256;
-  L.cpw = fine ? 1 : kRowsPerWaveEarly;
+  const int64_t TS = es == 8 ? tile_samples<double>() : tile_samples<float>();
+  const bool may = (extras & kLayoutFine) && n <= 1024 && m <= 1024;
+  const int64_t fine_tiles = may ? 255 / std::max(L.ncb, 1) : 0;
+  L.cpw = may && L.Bp / TS <= fine_tiles ? 1 : kRowsPerWaveEarly;
   L.ncd = (int)((n + 4 * L.cpw - 1) / (4 * L.cpw));
   L.nrd = (int)((m + 4 * L.cpw - 1) / (4 * L.cpw));
+  // A workspace sized for a batch serves every smaller one: past the line the partials keep
+  // the size of the last batch before it, eight times the blocks.
+  auto partials = [&](size_t rows, int blocks) {
+    const size_t fine = (rows + 3) / 4 * (size_t)std::min(Bp, fine_tiles * TS);
+    return std::max((size_t)std::max(blocks, 1) * Bp, fine) * es;
+  };
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t r = o; o = al(o + bytes); return r; };
   L.hdr = take(kSavedHeader);
@@ -63,8 +70,8 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
   L.MF = (extras & kLayoutWarm) ? take(M * Bp * es) : 0;
   L.DF = take(M * Bp * es);
   L.SL = take(mi * Bp * es);
-  L.colpart = take((size_t)5 * std::max(L.ncd, 1) * Bp * es);
-  L.rowpart = take((size_t)3 * std::max(L.nrd, 1) * Bp * es);
+  L.colpart = take(5 * partials(n, L.ncd));
+  L.rowpart = take(3 * partials(m, L.nrd));
   L.decpart = take((size_t)8 * kDecideSplit * Bp * es);  // k_decide's split pre-pass
   L.done = take(Bp * 4);
   L.count = take(Bp * 4);
