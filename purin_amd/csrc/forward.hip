@@ -83,12 +83,11 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
     L.X = take(std::max(n, m) * Bp * es);
     L.Z = take(std::max(n, m) * Bp * es);
   }
-  L.WTG = L.WRR = L.WLO = L.WHI = 0;
-  if ((extras & kLayoutWide) && (solo_wide_fits(p, true) || solo_wide_fits(p, false))) {
-    L.WTG = take(n * batch * es);
-    L.WRR = take(m * batch * es);
-    L.WLO = take(n * batch * es);
-    L.WHI = take(n * batch * es);
+  L.WLO = L.WHI = 0;
+  if (extras & (kLayoutWide | kLayoutWideShared)) {
+    const size_t copies = (extras & kLayoutWide) ? batch : 1;
+    L.WLO = take(n * copies * es);
+    L.WHI = take(n * copies * es);
   }
   if (p->res_ok) {  // resident path: slot-ordered copies of the per-sample inputs
     const size_t Kr = (size_t)p->res_mr * kResThreads, Kc = (size_t)p->res_mc * kResThreads;
@@ -416,8 +415,9 @@ static int run_solo_wide(purin_cp_plan* p, hipStream_t st, const Layout& L, char
                         0, st>>>((const T*)src, ld, perm, count, copies, dst);
     return (const T*)dst;
   };
-  A.TG = sorted(sv + L.Tt, L.Bp, p->sl_cperm, n, batch, L.WTG);
-  A.RR = sorted(sv + L.R, L.Bp, p->sl_rperm, m, batch, L.WRR);
+  // in the passes' ybar and multiplier buffers, which the loop's end alone writes
+  A.TG = sorted(sv + L.Tt, L.Bp, p->sl_cperm, n, batch, L.YB);
+  A.RR = sorted(sv + L.R, L.Bp, p->sl_rperm, m, batch, L.DF);
   const bool shared = o.shared_bounds != 0;
   A.LO = sorted(sv + L.LO, shared ? 1 : L.Bp, p->sl_cperm, n, shared ? 1 : batch, L.WLO);
   A.HI = sorted(sv + L.HI, shared ? 1 : L.Bp, p->sl_cperm, n, shared ? 1 : batch, L.WHI);
@@ -734,9 +734,7 @@ int run_iterations(purin_cp_plan* p, hipStream_t st, int64_t batch, const Layout
   // per-sample coefficients: each tile streams its own
   const bool res_vals = !qp && ps && !ps->RVs;
   const bool solo_dense = qp && qp->dense && ps && !o.streaming && solo_dense_fits(p);
-  // (a longer call would extend the schedule, which the passes do not need)
-  const bool solo_wide = L.WTG && !ps && !qp && !o.streaming &&
-                         o.max_iterations <= p->res_sched_len && solo_wide_fits(p, early);
+  const bool solo_wide = L.WLO && !ps && !qp;  // (wide_extras)
   if (solo_dense || solo_wide || (lds && !o.streaming && !p->diag && ((!ps && !qp) || res_qp || res_vals))) {
     if (solo_dense) {
       if (int rc = run_solo_dense<T>(p, st, L, sv, ws, o, early, batch, done, count, ndone + 2,
@@ -1074,20 +1072,26 @@ static int check_capture(purin_cp_plan* p, hipStream_t st, const purin_cp_solve_
                               "iterations (early_stop = 0) or a problem the resident kernel takes");
 }
 
+// The layout's part for k_solo_wide, where the call takes it.  (A call longer than the step
+// schedule would extend it, which the passes do not need.)
+static int wide_extras(const purin_cp_plan* p, const purin_cp_solve_options& o) {
+  if (o.streaming || o.max_iterations > p->res_sched_len || !solo_wide_fits(p, o.early_stop != 0))
+    return 0;
+  return o.shared_bounds ? kLayoutWideShared : kLayoutWide;
+}
+
 // This call's buffers: the caller's workspace, the plan workspace (grown
 // stream-ordered) or, for the no-allocation entry, the device's scratch array.
+// Where the part for k_solo_wide does not fit, the call runs on the passes.
 template <typename T>
 static int prepare_buffers(purin_cp_plan* p, hipStream_t st, int64_t batch, void* saved,
                            Layout* L, char** sv, char** ws, bool values = false, int extras = 0,
                            bool noalloc = false, const purin_cp_solve_options* o = nullptr) {
   *L = make_layout(p, batch, values, extras);
   int err = PURIN_CP_OK;
-  const size_t need = L->ws_end + (saved ? 0 : L->saved_end);
+  size_t need = L->ws_end + (saved ? 0 : L->saved_end);
   char* base = nullptr;
-  if (o && o->workspace) {  // the caller's: nothing is allocated, nothing of the plan's changes
-    base = (char*)workspace(p, need, st, &err, false, o->workspace, o->workspace_bytes);
-    if (!base) return err;
-  } else if (noalloc) {
+  if (noalloc && !(o && o->workspace)) {
     int cur = -1;
     PURIN_HIP(hipGetDevice(&cur));
     if (cur != p->device)
@@ -1104,8 +1108,15 @@ static int prepare_buffers(purin_cp_plan* p, hipStream_t st, int64_t batch, void
       base = (char*)g_scratch_ptr[p->device];
     }
     if (!base) return set_error(PURIN_CP_ERR_HIP, "no scratch address for this device");
-  } else {
-    base = (char*)workspace(p, need, st, &err);
+  } else {  // with the caller's, nothing is allocated and nothing of the plan's changes
+    void* caller = o ? o->workspace : nullptr;
+    const int64_t bytes = caller ? o->workspace_bytes : 0;
+    base = (char*)workspace(p, need, st, &err, false, caller, bytes);
+    if (!base && L->WLO) {
+      *L = make_layout(p, batch, values, extras & ~(kLayoutWide | kLayoutWideShared));
+      need = L->ws_end + (saved ? 0 : L->saved_end);
+      base = (char*)workspace(p, need, st, &err, false, caller, bytes);
+    }
     if (!base) return err;
   }
   *ws = base;
@@ -1164,8 +1175,9 @@ static int solve_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T* 
   if ((rc = check_capture<T>(p, st, o, false))) return rc;
   Layout L;
   char *sv, *ws;
-  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false, kLayoutWide | kLayoutFine,
-                               false, &o))) return rc;
+  if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false,
+                               wide_extras(p, o) | kLayoutFine, false, &o)))
+    return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m;
   write_header<T>(st, sv, batch, Bp, 0, o.shared_bounds, p);
   to_minor<T>(st, target, batch, n, n, (T*)(sv + L.Tt), Bp, nullptr, 0);
@@ -1223,7 +1235,7 @@ static int project_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T
   if ((rc = check_capture<T>(p, st, o, per_sample))) return rc;
   if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, per_sample,
                                (mult0 ? kLayoutWarm : 0) |
-                                   (per_sample || noalloc ? 0 : kLayoutWide) |
+                                   (per_sample || noalloc ? 0 : wide_extras(p, o)) |
                                    (noalloc ? 0 : kLayoutFine),
                                noalloc, &o)))
     return rc;
@@ -1485,10 +1497,11 @@ int64_t purin_cp_workspace_bytes(const purin_cp_plan* p, int32_t entry, int64_t 
     const Layout L = make_layout(p, batch, values, extras);
     return (int64_t)(L.ws_end + L.saved_end);  // saved == NULL puts the state in the workspace
   };
+  const int wide = solo_wide_fits(p, true) || solo_wide_fits(p, false) ? kLayoutWide : 0;
   switch (entry) {
     case PURIN_CP_ENTRY_SPMM: return forward(false, kLayoutSpmm);
-    case PURIN_CP_ENTRY_SOLVE: return forward(false, kLayoutWide | kLayoutFine);
-    case PURIN_CP_ENTRY_PROJECT: return forward(false, kLayoutWarm | kLayoutWide | kLayoutFine);
+    case PURIN_CP_ENTRY_SOLVE: return forward(false, wide | kLayoutFine);
+    case PURIN_CP_ENTRY_PROJECT: return forward(false, kLayoutWarm | wide | kLayoutFine);
     case PURIN_CP_ENTRY_PROJECT_VALUES:
     case PURIN_CP_ENTRY_QP_SOLVE:
     case PURIN_CP_ENTRY_DENSE_SOLVE: return forward(true, kLayoutWarm | kLayoutFine);

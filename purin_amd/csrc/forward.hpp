@@ -24,7 +24,7 @@ struct Layout {
   // row-scaled (RV, CV), bound-row coefficients (BC), row scales (SC), steps
   size_t VF, RVo, CVo, RV, CV, BC, SC, SGR, ACB, DCB, STB, RPT, CPT, PX, PZ, PW, PD;
   size_t RVs, CVs;    // [nnz] the scaled CSR / CSC entries when every sample has the plan's
-  size_t WTG, WRR, WLO, WHI;  // sample-major targets, rhs and bounds (solo.hpp, SoloWide)
+  size_t WLO, WHI;    // bounds in slice order (solo.hpp, SoloWide)
   size_t QQ, QC, QS;  // general QP: q, c (n x Bp) and per-sample max q, min q
   size_t ws_end;
 };
@@ -33,7 +33,8 @@ struct Layout {
 constexpr int kLayoutSpmm = 1;  // X, Z: purin_cp_spmm's batch-minor staging
 constexpr int kLayoutWarm = 2;  // MF: warm-start multipliers / duals in batch-minor layout
 constexpr int kLayoutFine = 8;  // one row / column per wavefront in small diagnostic passes
-constexpr int kLayoutWide = 4;  // WTG..WHI where the plan takes k_solo_wide
+constexpr int kLayoutWide = 4;  // WLO, WHI per sample: the call takes k_solo_wide
+constexpr int kLayoutWideShared = 16;  // one copy of them
 
 Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values = false, int extras = 0);
 

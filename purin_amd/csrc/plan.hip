@@ -125,6 +125,7 @@ void* workspace(purin_cp_plan* p, size_t bytes, hipStream_t stream, int* err, bo
   void* nb = nullptr;
   hipError_t e = hipMallocAsync(&nb, bytes, stream);
   if (e != hipSuccess) {
+    (void)hipGetLastError();  // the call may go on with less
     *err = set_error(PURIN_CP_ERR_NOMEM, std::string("workspace hipMallocAsync: ") + hipGetErrorString(e));
     return nullptr;
   }

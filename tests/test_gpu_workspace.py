@@ -10,6 +10,7 @@ bit for bit, with the same calls made one after another on the plan's own
 workspace.  Every call goes through the C ABI.
 """
 
+import re
 import threading
 
 import numpy as np
@@ -111,6 +112,34 @@ def test_workspace_too_small_or_misaligned_is_an_argument_error():
     out = plan.project(w.target, rhs, max_iterations=10, workspace=ws[:need])
     torch.cuda.synchronize()
     assert np.all(np.isfinite(to_np(out.y)))
+
+
+@pytest.mark.parametrize("shared", [True, False])
+def test_wide_problem_runs_in_the_passes_workspace(shared):
+    """Beyond the tile kernels a call needs no more than the streaming passes: where the
+    per-sample loop's copies of the bounds do not fit, it runs on the passes (their bits), and
+    one shared copy of them is all that shared bounds take."""
+    torch = require_gpu()
+    B, n = 5, 4200
+    w = workloads.ragged_rows(31, n=n, me=200, mi=300, wmin=2, wmax=6, batch=B)
+    plan = plan_for(canonical_from_workload(w), dtype=np.float64)
+    rhs = np.tile(w.rhs, (B, 1))
+    kw = dict(max_iterations=60, early_stop=False, shared_bounds=shared)
+    def buffer(nbytes):
+        return torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+
+    with pytest.raises(PurinError, match="workspace too small") as err:
+        plan.project(w.target, rhs, streaming=True, workspace=buffer(256), **kw)
+    least = int(re.search(r"needs (\d+) bytes", str(err.value)).group(1))
+    copies = 2 * 8 * n * (1 if shared else B)
+    want = plan.project(w.target, rhs, streaming=True, workspace=buffer(least), **kw)
+    got = plan.project(w.target, rhs, workspace=buffer(least), timing=True, **kw)
+    assert plan.last_timing()["resident"] == 0
+    _same(got, want, PROJECT_FIELDS, "passes")
+    full = buffer(least + copies + 512)  # (each copy 256-byte aligned)
+    got = plan.project(w.target, rhs, workspace=full, timing=True, **kw)
+    assert plan.last_timing()["resident"] == 1
+    assert rel_err(to_np(got.y), to_np(want.y)) <= 1e-11
 
 
 def test_two_streams_on_one_plan():
