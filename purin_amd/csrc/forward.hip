@@ -1074,9 +1074,12 @@ static int check_capture(purin_cp_plan* p, hipStream_t st, const purin_cp_solve_
 
 // The layout's part for k_solo_wide, where the call takes it.  (A call longer than the step
 // schedule would extend it, which the passes do not need.)
-static int wide_extras(const purin_cp_plan* p, const purin_cp_solve_options& o) {
-  if (o.streaming || o.max_iterations > p->res_sched_len || !solo_wide_fits(p, o.early_stop != 0))
-    return 0;
+static int wide_extras(purin_cp_plan* p, const purin_cp_solve_options& o) {
+  if (o.streaming || !solo_wide_fits(p, o.early_stop != 0)) return 0;
+  {
+    std::lock_guard<std::mutex> lock(p->mu);  // another thread's call may extend it
+    if (o.max_iterations > p->res_sched_len) return 0;
+  }
   return o.shared_bounds ? kLayoutWideShared : kLayoutWide;
 }
 
