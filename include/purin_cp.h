@@ -349,12 +349,13 @@ int purin_cp_dense_solve(purin_cp_plan* plan, void* stream, int64_t batch, const
 /* Kernel times of the last solve()/project() call made with opts.timing = 1,
  * from HIP events recorded on that call's stream around each launch. */
 typedef struct {
-  int64_t iterations;   /* CP iterations timed */
-  double row_ms;        /* summed row-pass time */
+  int64_t iterations;   /* CP iterations timed (stop test: the longest sample's) */
+  double row_ms;        /* summed row-pass time (streaming passes, as the next two) */
   double col_ms;        /* summed column-pass time */
   double diag_ms;       /* summed residual + decide time (stop test) */
   double loop_ms;       /* first iteration kernel start to last end */
-  int32_t resident;     /* 1: the iterations ran in the resident kernel (one launch) */
+  int32_t resident;     /* 1: the iterations ran inside a kernel: the resident tiles or
+                           one workgroup per sample (dense stop test: two launches) */
   int32_t linear_kybar; /* 1: the streaming passes formed K ybar = (1 + theta) K y -
                            theta K y_prev instead of storing ybar (n > 2 m) */
   int32_t narrow_columns; /* 1: the fixed-iteration column pass took a quarter

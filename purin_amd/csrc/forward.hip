@@ -309,9 +309,10 @@ static size_t resident_lds(const purin_cp_plan* p, bool early = false) {
   return lds <= 160 * 1024 ? lds : 0;
 }
 
-// The launch check and, with timing, the launch's time (e0 was recorded before it).
+// The launch check and, with timing, the loop's time (e0 was recorded before it) and its
+// iterations: with the stop test the longest sample's, from ``count``.
 static int finish_resident(purin_cp_plan* p, hipStream_t st, const purin_cp_solve_options& o,
-                           hipEvent_t e0, hipEvent_t e1) {
+                           hipEvent_t e0, hipEvent_t e1, const int32_t* count, int64_t batch) {
   PURIN_HIP(hipGetLastError());
   if (!o.timing) return PURIN_CP_OK;
   PURIN_HIP(hipEventRecord(e1, st));
@@ -320,6 +321,13 @@ static int finish_resident(purin_cp_plan* p, hipStream_t st, const purin_cp_solv
   PURIN_HIP(hipEventElapsedTime(&ms, e0, e1));
   purin_cp_timing t{};
   t.iterations = o.max_iterations;
+  if (o.early_stop) {
+    std::vector<int32_t> counts((size_t)batch);
+    PURIN_HIP(hipMemcpyAsync(counts.data(), count, (size_t)batch * sizeof(int32_t),
+                             hipMemcpyDeviceToHost, st));
+    PURIN_HIP(hipStreamSynchronize(st));
+    t.iterations = *std::max_element(counts.begin(), counts.end());
+  }
   t.loop_ms = ms;
   t.resident = 1;
   record_timing(p, t);
@@ -436,7 +444,7 @@ static int run_solo_wide(purin_cp_plan* p, hipStream_t st, const Layout& L, char
     PURIN_HIP(hipEventRecord(e0, st));
   }
   if (int rc = solo_wide_launch<T>(st, p, A, early)) return rc;
-  return finish_resident(p, st, o, e0, e1);
+  return finish_resident(p, st, o, e0, e1, count, batch);
 }
 
 // The dense adapter's loop with one workgroup per sample (solo.hip).
@@ -484,7 +492,7 @@ static int run_solo_dense(purin_cp_plan* p, hipStream_t st, const Layout& L, cha
   if (!early)  // ybar0 = y0
     PURIN_HIP(hipMemcpyAsync(A.YB, A.Y, (size_t)p->n * L.Bp * sizeof(T), hipMemcpyDeviceToDevice, st));
   if (int rc = solo_dense_launch<T>(st, p, A, early)) return rc;
-  return finish_resident(p, st, o, e0, e1);
+  return finish_resident(p, st, o, e0, e1, count, batch);
 }
 
 // The CP loop on the resident kernel; fills Y and D like the passes (and, with
@@ -521,7 +529,7 @@ static int run_resident(purin_cp_plan* p, hipStream_t st, const Layout& L, char*
     }
     if (int rc = run_solo<T>(p, st, L, sv, o, early, batch, tol, tolv, done, count, sched, qp, ps))
       return rc;
-    return finish_resident(p, st, o, e0, e1);
+    return finish_resident(p, st, o, e0, e1, count, batch);
   }
   Res<T> R{};
   R.n = (int)p->n;
@@ -632,7 +640,7 @@ static int run_resident(purin_cp_plan* p, hipStream_t st, const Layout& L, char*
                                   o.shared_bounds != 0, early, BT,
                                   qp ? (ps->RVs ? 1 : 3) : (ps ? 2 : 0)))
     return rc;
-  return finish_resident(p, st, o, e0, e1);
+  return finish_resident(p, st, o, e0, e1, count, batch);
 }
 
 // The passes that leave partials, at the layout's rows / columns per wavefront.

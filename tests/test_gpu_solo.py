@@ -200,3 +200,26 @@ def test_final_passes_one_column_per_wavefront(n, me, mi, few, many, dtype):
         assert rel_err(to_np(getattr(s, f)), to_np(getattr(a, f))[:few]) <= bar, f
     for f in ("status", "finite", "eligible", "iterations"):
         np.testing.assert_array_equal(to_np(getattr(s, f)), to_np(getattr(a, f))[:few])
+
+
+@pytest.mark.parametrize("n,me,mi,dense", [(70, 12, 30, False), (1500, 100, 200, False),
+                                           (4200, 200, 300, False), (60, 12, 25, True)])
+def test_timing_counts_the_iterations_that_ran(n, me, mi, dense):
+    """With the stop test the timed iterations are the longest sample's, whichever kernel ran
+    them (one workgroup per sample, the tiles, several rows per thread, the dense adapter)."""
+    require_gpu()
+    B, limit = 6, 5000
+    w = workloads.ragged_rows(17, n=n, me=me, mi=mi, wmin=2, wmax=5, batch=B)
+    canon = canonical_from_workload(w)
+    kw = dict(tolerance=1e-2, max_iterations=limit, timing=True)
+    if dense:
+        plan = plan_for(canon, dtype=np.float64, bound_presolve=False, row_scaling=False,
+                        norm_bound=False)
+        one = np.ones((B, n))
+        rhs = np.tile(w.rhs, (B, 1))
+        counts = to_np(plan.dense_solve(one, -w.target, rhs, -one, one, **kw)[2])
+    else:
+        plan = plan_for(canon, dtype=np.float64)
+        counts = to_np(plan.project(w.target, np.tile(w.rhs, (B, 1)), **kw).iterations)
+    t = plan.last_timing()
+    assert t["resident"] == 1 and t["iterations"] == counts.max() < limit
