@@ -49,13 +49,32 @@ __device__ __forceinline__ T dot_regs(const T (&v)[W], const uint32_t (&ix)[W / 
 }
 
 // A slice's sum: groups of 4 entries in registers (the count is the wavefront's),
-// then the entries past W from LDS.
-template <typename T, int W>
+// then the entries past W from LDS.  FOUR: four of those in flight.  Most kernels' loops the
+// compiler unrolls by itself, by eight; the fp64 ones with the stop test that are short of
+// registers it leaves at one entry, 140 cycles each (us per iteration of the QP, a row of 200
+// entries, B = 256: 12.0, with FOUR 5.6; the others with FOUR 3.8 -> 5.1).
+template <bool FOUR, typename T, int W>
 __device__ __forceinline__ T slice_sum(const T (&v)[W], const uint32_t (&ix)[W / 2], int groups,
                                        const unsigned char* lds, const T* rv, const uint16_t* ri,
                                        int rest) {
   T acc = groups <= 1 ? dot_regs<4>(v, ix, lds) : dot_regs<8>(v, ix, lds);
-  for (int k = 0; k < rest; ++k)
+  int k = 0;
+  if constexpr (FOUR) {
+    for (; k + 4 <= rest; k += 4) {
+      T c[4], x[4];
+      uint32_t at[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        at[h] = ri[(k + h) * 64];
+        c[h] = rv[(k + h) * 64];
+      }
+#pragma unroll
+      for (int h = 0; h < 4; ++h) x[h] = *reinterpret_cast<const T*>(lds + at[h]);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) acc = __builtin_elementwise_fma(c[h], x[h], acc);
+    }
+  }
+  for (; k < rest; ++k)
     acc = __builtin_elementwise_fma(rv[k * 64], *reinterpret_cast<const T*>(lds + ri[k * 64]), acc);
   return acc;
 }
@@ -162,6 +181,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
     return;
   }
   constexpr bool QP = MODE == kSoloQP, PS = MODE != kSoloShared;
+  constexpr bool FOUR = sizeof(T) == 8 && EARLY && (PS || !HELP);
   const T zero = T(0), half = T(0.5), inf = T(__builtin_inf());
   // LDS: Gy [n] | zero | Gd [m] | zero | partials [16][4] or (HELP) [2][3][NT] | verdict |
   // rest values | rest offsets
@@ -308,7 +328,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
       const T sigma = PS ? sig : f_sig, a = PS ? pa : f_a, delta = PS ? pd : f_d,
               theta = PS ? th : f_th;
       if (has_r) {
-        const T acc = slice_sum<T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
+        const T acc = slice_sum<FOUR, T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
         T p = d + sigma * (acc - rr);
         if (ineq) p = res_pos(p);
         d = p;
@@ -316,7 +336,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
       }
       __syncthreads();
       if (has_c) {
-        const T tt = slice_sum<T, W>(cv, cx, cgr, lds, crv, cri, crest);
+        const T tt = slice_sum<FOUR, T, W>(cv, cx, cgr, lds, crv, cri, crest);
         const T s = primal_step(tt, a, delta);
         const T yn = odd ? clipp(s, lo, hi) : res_clip(s, lo, hi);
         if (t < n) Gy[t] = yn + theta * (yn - y);
@@ -334,7 +354,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
   // K y0 and the first d+
   T ky = zero;
   if (has_r) {
-    ky = slice_sum<T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
+    ky = slice_sum<FOUR, T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
     T p = d + (PS ? sig : sched[0]) * (ky - rr);
     if (ineq) p = res_pos(p);
     d = p;
@@ -393,7 +413,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
     q_pri = q_dual = q_max = zero;
     if (run && has_c) {
       const T a = PS ? pa : f_a, delta = PS ? pd : f_d;
-      const T tt = slice_sum<T, W>(cv, cx, cgr, lds, crv, cri, crest);
+      const T tt = slice_sum<FOUR, T, W>(cv, cx, cgr, lds, crv, cri, crest);
       const T s = primal_step(tt, a, delta);
       const T yn = odd ? clipp(s, lo, hi) : res_clip(s, lo, hi);
       y = yn;
@@ -444,7 +464,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
     if (PS && run) advance();
     if (run && has_r) {
       const T sigma_n = PS ? sig : f_sn;
-      const T acc = slice_sum<T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
+      const T acc = slice_sum<FOUR, T, W>(rv, rx, rgr, lds, rrv, rri, rrest);
       if (t < m) {  // kernels.py:158-166; d * 0 is NaN for a non-finite d
         const T e = acc - rr, w = ineq ? zero : T(-1);
         q_max = __builtin_fmax(q_max, __builtin_fmax(e, w * e));

@@ -141,6 +141,34 @@ def test_solo_values_and_qp_match_streaming(n, me, mi, B, early):
             assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= 1e-10
 
 
+@pytest.mark.parametrize("n,me,mi,wmax,B", [
+    (70, 12, 30, 41, 5),     # the wavefront of the stop test beside two of rows and columns
+    (250, 20, 40, 43, 515),  # four wavefronts without it
+])
+def test_solo_stop_test_with_long_rows(n, me, mi, wmax, B):
+    """Rows whose entries past the registers take the loop of four at a time and its
+    remainder, in the fp64 kernels with the stop test."""
+    require_gpu()
+    rng = np.random.default_rng(n)
+    w = workloads.ragged_rows(500 + n, n=n, me=me, mi=mi, wmin=2, wmax=wmax, batch=B)
+    canon = canonical_from_workload(w)
+    m = me + mi
+    rhs = np.tile(w.rhs, (B, 1))
+    values = np.tile(w.data, (B, 1))
+    kw = dict(max_iterations=300, tolerance=1e-2)
+    plan = plan_for(canon, dtype=np.float64)
+    rows = type(canon)(n=n, me=me, rows=canon.rows[:m], coef=canon.coef[:m])
+    qplan = plan_for(rows, dtype=np.float64, bound_presolve=False)
+    q, one = rng.uniform(0.5, 2.0, (B, n)), np.ones((B, n))
+    for call in (lambda **k: plan.project(w.target, rhs, **k, **kw),
+                 lambda **k: plan.project(w.target, rhs, values=values, **k, **kw),
+                 lambda **k: qplan.qp_solve(q, -w.target, rhs[:, :m], -one, one, **k, **kw)):
+        a, s = call(), call(streaming=True)
+        np.testing.assert_array_equal(to_np(a.iterations), to_np(s.iterations))
+        assert rel_err(to_np(a.y), to_np(s.y)) <= 1e-10
+        assert rel_err(to_np(a.multipliers), to_np(s.multipliers)) <= 1e-10
+
+
 @pytest.mark.parametrize("n,me,mi,B,dtype", [
     (4097, 60, 200, 3, np.float64),     # just beyond the tile kernels
     (4200, 500, 3596, 2, np.float64),   # 4096 rows: K y+ in registers, both loops
