@@ -14,7 +14,8 @@
 //     k's terms while the others run iteration k + 1, so the test is not on the path of
 //     the iterates.  The state of two iterations back is kept, and a sample accepted at
 //     k returns exactly that state and count.  (With all 16 wavefronts taken by rows or
-//     columns each reduces its own terms and the last one judges.)
+//     columns, or with four or eight where one more would cost a workgroup per CU
+//     (solo_block), each reduces its own terms and the last one judges.)
 // One iteration (kernels.py:91-150): the column pass gathers d+, forms y+ and its
 // diagnostics; the row pass gathers y+: K y+, the residual, and the next d+ from
 // K ybar = (1 + theta) K y+ - theta K y (resident.hpp, k_resident_early).  Without the
@@ -989,6 +990,8 @@ int rest_entries(const purin_cp_plan* p, int W) {
   return k;
 }
 
+constexpr size_t kLdsMax = 160 * 1024;
+
 int solo_waves(const purin_cp_plan* p) { return std::max(p->sl_nsr, p->sl_nsc); }
 
 int cu_count(const purin_cp_plan* p) {
@@ -1046,17 +1049,45 @@ int launch_mode(hipStream_t st, const Solo<T>& A, SoloBlock k, size_t lds, bool 
 //   fp32  n = 250, B = 8192: 6.5 / 2.5 (16.1 / 4.3); n = 500: 13.5 / 6.4 (16.4 / 4.6);
 //         n = 800: 32.3 / 15.5 (17.7 / 4.7), B = 512: 2.0 / 1.0 (4.2 / 1.2)
 // so a sample per workgroup while its wavefronts leave a CU at least two of them, and above
-// that for the batches of the first rounds.  Per-sample coefficients stay in registers
-// here and stream from HBM there, whatever the batch.
+// that for the batches of the first rounds.  Rows and columns past the registers (``chain``
+// entries of the widest) take LDS, and with it workgroups from a CU, and a workgroup's time
+// grows with them while the tiles' stream is shared by their samples (us per iteration, stop
+// test / without, here against the tiles):
+//   fp64  one workgroup per CU: n = 200, a dense row: B = 256 4.2 / 3.7 (5.6 / 4.3), B = 1024
+//         22.4 / 15.0 (11.2 / 8.7); n = 500, rows of 40: B = 512 4.8 / 3.5 (3.4 / 2.1)
+//         two: n = 250, rows of 40, B = 2048 9.3 / 7.1 (11.2 / 6.8); n = 120, a dense row,
+//         B = 8192 43.4 / 38.9 (63.1 / 44.8)
+//         n = 700, B = 2048: rows of 12 9.7 (9.9), of 24 11.3 (10.8), of 40 16.0 (13.2)
+//   fp32  n = 240, a dense row (one per CU): B = 256 4.3 / 4.2 (9.7 / 7.4), B = 1024 17.9 / 16.4
+//         (9.7 / 7.5); n = 300, five rows of 150 (two): B = 1024 6.5 / 6.1 (7.3 / 5.1),
+//         B = 8192 51.7 (28.9); n = 400, rows of 40 (three): B = 1024 3.8 / 3.4 (4.8 / 2.7),
+//         B = 2048 6.2 (4.9); n = 250, rows of 12: B = 1024 1.4 / 0.9 (4.0 / 1.3), B = 2048 2.6 /
+//         1.7 (4.0 / 1.2); n = 500, rows of 24, B = 2048: 5.2 (4.7)
+// A full round of the fp32 tiles is 2048 samples.  Per-sample coefficients stay in registers
+// and LDS here and stream from HBM there, whatever the batch (n = 200, a dense row, B = 8192:
+// fp64 186 / 118 against 202 / 151).
 bool solo_fits(const purin_cp_plan* p, int64_t batch, bool early, bool values) {
   if (!p->sl_ok || p->n > kSoloMax || p->m > kSoloMax) return false;
-  if (solo_lds(p, solo_block(p, batch, early)) > 160 * 1024) return false;
+  const size_t lds = solo_lds(p, solo_block(p, batch, early));
+  if (lds > kLdsMax) return false;
   const int w = solo_waves(p);
-  const int64_t cus = cu_count(p);
-  if (values || w <= 4) return true;
-  if (p->dtype == PURIN_CP_F64) return early ? (w <= 13 || batch <= cus) : (w <= 8 || batch <= cus);
-  if (early) return w <= 8 || batch <= 3 * cus;
-  return batch <= (w <= 8 ? 4 : 2) * cus;
+  const int64_t cus = cu_count(p), per_cu = (int64_t)(kLdsMax / lds);
+  auto past = [](const std::vector<int32_t>& v) { return v.empty() ? 0 : rest_of(v[0], kSoloW); };
+  const int chain = past(p->sl_rw) + past(p->sl_cw);
+  if (values) return true;
+  if (p->dtype == PURIN_CP_F64) {
+    if (batch <= cus) return true;
+    if (w > 8) return early && w <= 13 && chain <= 16;
+    return per_cu >= (early || w <= 2 ? 2 : 3);
+  }
+  if (early) {
+    if (w > 8) return batch <= 3 * cus;
+    if (per_cu >= 4 && (w < 8 || chain <= 8)) return true;
+    return batch <= 2 * std::min<int64_t>(per_cu, 2) * cus;
+  }
+  if (chain <= 3) return w <= 4 || batch <= (w <= 8 ? 4 : 2) * cus;
+  if (w <= 2 && per_cu >= 3) return true;
+  return batch <= (per_cu == 1 ? 1 : (w <= 4 ? 4 : 2)) * cus;
 }
 
 template <typename T>
@@ -1083,7 +1114,7 @@ static size_t wide_lds(const purin_cp_plan* p, bool early) {
 bool solo_wide_fits(const purin_cp_plan* p, bool early) {
   if (!p->sl_ok || p->res_ok || p->diag || p->m < 1) return false;
   if (!early && p->sl_nsr > 16 * kWideU) return false;
-  return wide_lds(p, early) <= 160 * 1024;
+  return wide_lds(p, early) <= kLdsMax;
 }
 
 template <typename T>

@@ -1,4 +1,5 @@
-"""Host rules of the library, on plans made up here (CPU only): workspace sizes.
+"""Host rules of the library, on plans made up here (CPU only): workspace sizes and which
+kernel runs a call.
 
 The rules read a plan's sizes and row and column widths alone, so a plan whose device arrays
 are empty serves.  A few lines of C++ against the library's own headers make one.
@@ -47,6 +48,9 @@ extern "C" purin_cp_plan* route_plan(int f64, int64_t n, int64_t m, int64_t M, c
   return p;
 }
 extern "C" void route_free(purin_cp_plan* p) { delete p; }
+extern "C" int route_solo(const purin_cp_plan* p, int64_t batch, int early, int values) {
+  return solo_fits(p, batch, early != 0, values != 0);
+}
 extern "C" int64_t route_workspace(const purin_cp_plan* p, int entry, int64_t batch) {
   return purin_cp_workspace_bytes(p, entry, batch, nullptr);
 }
@@ -68,6 +72,7 @@ def routes(tmp_path_factory):
     lib.route_plan.restype = vp
     lib.route_plan.argtypes = [C.c_int, i64, i64, i64, i32, i32]
     lib.route_free.argtypes = [vp]
+    lib.route_solo.argtypes = [vp, i64, C.c_int, C.c_int]
     lib.route_workspace.restype = i64
     lib.route_workspace.argtypes = [vp, C.c_int, i64]
     return lib
@@ -90,6 +95,9 @@ class _Plan:
     def __del__(self):
         self.lib.route_free(self.p)
 
+    def solo(self, batch, early, values=False):
+        return bool(self.lib.route_solo(self.p, batch, int(early), int(values)))
+
     def workspace(self, entry, batch):
         from purin_amd import _lib
 
@@ -106,3 +114,39 @@ def test_workspace_of_a_batch_serves_smaller_ones(routes, n, m, dtype, entry):
     sizes = [plan.workspace(entry, b) for b in range(1, 70000, 61)]
     assert min(sizes) > 0
     assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+
+
+def _rows(n, m, w, wide=0, wide_w=0):
+    return np.concatenate((np.full(wide, wide_w), np.full(m - wide, w))).astype(int)
+
+
+@pytest.mark.parametrize("n,m,w,wide,dtype,early,fixed", [
+    # the batches up to which one workgroup per sample pays (None: all), as measured
+    (250, 75, 5, (0, 0), np.float64, None, None),
+    (250, 75, 5, (0, 0), np.float32, None, None),
+    (500, 150, 5, (0, 0), np.float32, None, 1024),
+    (200, 21, 4, (1, 200), np.float64, 256, 256),   # one workgroup's entries fill the LDS
+    (240, 21, 4, (1, 240), np.float32, 512, 256),
+    (120, 21, 4, (1, 120), np.float64, None, None),  # two fit
+    (300, 65, 4, (5, 150), np.float64, 256, 256),
+    (300, 65, 4, (5, 150), np.float32, 1024, 512),
+    (250, 75, 40, (0, 0), np.float64, None, 256),
+    (250, 75, 12, (0, 0), np.float32, None, 1024),
+    (500, 150, 40, (0, 0), np.float64, 256, 256),
+    (500, 150, 24, (0, 0), np.float32, 1024, 512),
+    (700, 210, 12, (0, 0), np.float64, None, 256),
+    (700, 210, 40, (0, 0), np.float64, 256, 256),
+])
+def test_one_workgroup_per_sample_where_it_pays(routes, n, m, w, wide, dtype, early, fixed):
+    """Long rows take LDS from the workgroups that share a CU: past the batches where the tile
+    kernels are faster the calls go there.  Per-sample coefficients stay."""
+    widths = _rows(n, m, w, *wide)
+    # columns of a random matrix: a few stand out by up to ten entries
+    cols = np.full(n, widths.sum() // n)
+    if widths.max() > 8:
+        cols[:3] += 6
+    plan = _Plan(routes, n, widths, dtype, col_widths=cols)
+    for stop, last in ((True, early), (False, fixed)):
+        for batch in (1, 256, 257, 512, 513, 1024, 1025, 8192):
+            assert plan.solo(batch, stop) == (last is None or batch <= last), (batch, stop)
+            assert plan.solo(batch, stop, values=True)
