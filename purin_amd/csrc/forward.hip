@@ -1082,8 +1082,8 @@ static int check_capture(purin_cp_plan* p, hipStream_t st, const purin_cp_solve_
 
 // The layout's part for k_solo_wide, where the call takes it.  (A call longer than the step
 // schedule would extend it, which the passes do not need.)
-static int wide_extras(purin_cp_plan* p, const purin_cp_solve_options& o) {
-  if (o.streaming || !solo_wide_fits(p, o.early_stop != 0)) return 0;
+static int wide_extras(purin_cp_plan* p, int64_t batch, const purin_cp_solve_options& o) {
+  if (o.streaming || !solo_wide_fits(p, batch, o.early_stop != 0)) return 0;
   {
     std::lock_guard<std::mutex> lock(p->mu);  // another thread's call may extend it
     if (o.max_iterations > p->res_sched_len) return 0;
@@ -1187,7 +1187,7 @@ static int solve_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T* 
   Layout L;
   char *sv, *ws;
   if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, false,
-                               wide_extras(p, o) | kLayoutFine, false, &o)))
+                               wide_extras(p, batch, o) | kLayoutFine, false, &o)))
     return rc;
   const int64_t Bp = L.Bp, n = p->n, m = p->m;
   write_header<T>(st, sv, batch, Bp, 0, o.shared_bounds, p);
@@ -1246,7 +1246,7 @@ static int project_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const T
   if ((rc = check_capture<T>(p, st, o, per_sample))) return rc;
   if ((rc = prepare_buffers<T>(p, st, batch, saved, &L, &sv, &ws, per_sample,
                                (mult0 ? kLayoutWarm : 0) |
-                                   (per_sample || noalloc ? 0 : wide_extras(p, o)) |
+                                   (per_sample || noalloc ? 0 : wide_extras(p, batch, o)) |
                                    (noalloc ? 0 : kLayoutFine),
                                noalloc, &o)))
     return rc;
@@ -1508,7 +1508,8 @@ int64_t purin_cp_workspace_bytes(const purin_cp_plan* p, int32_t entry, int64_t 
     const Layout L = make_layout(p, batch, values, extras);
     return (int64_t)(L.ws_end + L.saved_end);  // saved == NULL puts the state in the workspace
   };
-  const int wide = solo_wide_fits(p, true) || solo_wide_fits(p, false) ? kLayoutWide : 0;
+  // (a smaller batch may take it where this one does not)
+  const int wide = solo_wide_can(p, true) || solo_wide_can(p, false) ? kLayoutWide : 0;
   switch (entry) {
     case PURIN_CP_ENTRY_SPMM: return forward(false, kLayoutSpmm);
     case PURIN_CP_ENTRY_SOLVE: return forward(false, wide | kLayoutFine);

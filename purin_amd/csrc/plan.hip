@@ -1174,7 +1174,7 @@ int purin_cp_plan_create(purin_cp_plan** out, int32_t dtype, int64_t n, int64_t 
     if (e != hipSuccess) rc = hip_check(e, "hipStreamCreateWithFlags");
   }
   // the resident kernel's step schedule, for calls of up to kSchedCapacity iterations
-  if (rc == PURIN_CP_OK && (p->res_ok || solo_wide_fits(p, true)))
+  if (rc == PURIN_CP_OK && (p->res_ok || solo_wide_can(p, true)))
     rc = ensure_schedule(p, kSchedCapacity, nullptr, true);
   // this device's address of the no-allocation entry's scratch array
   if (rc == PURIN_CP_OK) rc = scratch_init_device(p->device);

@@ -518,6 +518,7 @@ __global__ __launch_bounds__(1024) void k_solo(Solo<T> A) {
 // four slices in flight.
 // ---------------------------------------------------------------------------
 constexpr int kWideU = 4;  // slices of a wavefront in flight
+constexpr int kWideThreads = 1024;
 
 // sums of slices s0, s0 + 16, ... (kWideU of them): acc[u] = entries times x
 template <typename T>
@@ -1111,10 +1112,31 @@ static size_t wide_lds(const purin_cp_plan* p, bool early) {
 // 55.9 / 40.1 at B = 1024 (162 / 59.8); n = 6000, m = 2100 fp64 12.6 / 10.1 (85.6 / 17.9) and
 // 51.4 / 40.5 (140 / 59.1).  Fixed iterations of more than 4096 rows stay on the passes,
 // whose narrow column tiles serve them.
-bool solo_wide_fits(const purin_cp_plan* p, bool early) {
+bool solo_wide_can(const purin_cp_plan* p, bool early) {
   if (!p->sl_ok || p->res_ok || p->diag || p->m < 1) return false;
   if (!early && p->sl_nsr > 16 * kWideU) return false;
   return wide_lds(p, early) <= kLdsMax;
+}
+
+// Every workgroup streams the matrix, and a CU holds one; the passes read it once per 128
+// (fp64) or 256 (fp32) samples.  us per iteration here against the passes, n = 8000:
+//   a row or column far longer than a wavefront's share of the entries is one wavefront's
+//   chain, in every round of the launch: fp64 a dense row fixed B = 256 949 (1526), B = 512
+//   1897 (1606), stop test B = 512 1953 (2932), B = 1024 3900 (3183); a column of 3000 fixed
+//   B = 512 694 (932), B = 1024 1412 (1041); four rows of 2000 fixed B = 512 465 (579), B =
+//   1024 933 (614), stop test B = 4096 4071 (4488)
+//   even rows, fixed: fp64 up to 400 wide (800,000 entries) even or better from B = 256 on,
+//   but B = 64 rows of 200 135 (119), n = 12000 rows of 75 107 (81); fp32 rows of 50 324 (392)
+//   at B = 4096, of 100 162 (136) at B = 1024, n = 6000 rows of 300 1116 (668) at B = 4096;
+//   up to B = 512 better at any width.  With the stop test better at any width and batch.
+bool solo_wide_fits(const purin_cp_plan* p, int64_t batch, bool early) {
+  if (!solo_wide_can(p, early)) return false;
+  const int64_t cus = cu_count(p), chain = (int64_t)p->sl_rw[0] + p->sl_cw[0];
+  const bool uneven = chain > 4 * ((p->sl_rn + p->sl_cn) / kWideThreads);
+  if (early) return !uneven || chain <= 2048 || batch <= 2 * cus;
+  if (uneven) return batch <= (chain <= 4096 ? 2 : 1) * cus;
+  if (p->dtype == PURIN_CP_F64) return p->nnz <= 160000 || batch > 128;
+  return batch <= 2 * cus || p->nnz <= 13 * (p->n + p->m);
 }
 
 template <typename T>
@@ -1122,7 +1144,7 @@ int solo_wide_launch(hipStream_t st, const purin_cp_plan* p, const SoloWide<T>& 
   const size_t lds = wide_lds(p, early);
   auto kern = early ? k_solo_wide<T, true> : k_solo_wide<T, false>;
   if (int rc = raise_lds_cap((const void*)kern, lds)) return rc;
-  kern<<<(unsigned)A.Bp, 1024, lds, st>>>(A);
+  kern<<<(unsigned)A.Bp, kWideThreads, lds, st>>>(A);
   return PURIN_CP_OK;
 }
 template int solo_wide_launch<double>(hipStream_t, const purin_cp_plan*, const SoloWide<double>&, bool);

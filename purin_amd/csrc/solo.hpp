@@ -88,7 +88,9 @@ struct SoloWide {
   T* Y;
   T* D;
 };
-bool solo_wide_fits(const purin_cp_plan* p, bool early);
+// Whether the kernel takes this plan, and whether it pays for this batch.
+bool solo_wide_can(const purin_cp_plan* p, bool early);
+bool solo_wide_fits(const purin_cp_plan* p, int64_t batch, bool early);
 template <typename T>
 int solo_wide_launch(hipStream_t st, const purin_cp_plan* p, const SoloWide<T>& A, bool early);
 

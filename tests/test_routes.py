@@ -51,6 +51,9 @@ extern "C" void route_free(purin_cp_plan* p) { delete p; }
 extern "C" int route_solo(const purin_cp_plan* p, int64_t batch, int early, int values) {
   return solo_fits(p, batch, early != 0, values != 0);
 }
+extern "C" int route_wide(const purin_cp_plan* p, int64_t batch, int early) {
+  return solo_wide_fits(p, batch, early != 0);
+}
 extern "C" int64_t route_workspace(const purin_cp_plan* p, int entry, int64_t batch) {
   return purin_cp_workspace_bytes(p, entry, batch, nullptr);
 }
@@ -73,6 +76,7 @@ def routes(tmp_path_factory):
     lib.route_plan.argtypes = [C.c_int, i64, i64, i64, i32, i32]
     lib.route_free.argtypes = [vp]
     lib.route_solo.argtypes = [vp, i64, C.c_int, C.c_int]
+    lib.route_wide.argtypes = [vp, i64, C.c_int]
     lib.route_workspace.restype = i64
     lib.route_workspace.argtypes = [vp, C.c_int, i64]
     return lib
@@ -97,6 +101,9 @@ class _Plan:
 
     def solo(self, batch, early, values=False):
         return bool(self.lib.route_solo(self.p, batch, int(early), int(values)))
+
+    def wide(self, batch, early):
+        return bool(self.lib.route_wide(self.p, batch, int(early)))
 
     def workspace(self, entry, batch):
         from purin_amd import _lib
@@ -150,3 +157,28 @@ def test_one_workgroup_per_sample_where_it_pays(routes, n, m, w, wide, dtype, ea
         for batch in (1, 256, 257, 512, 513, 1024, 1025, 8192):
             assert plan.solo(batch, stop) == (last is None or batch <= last), (batch, stop)
             assert plan.solo(batch, stop, values=True)
+
+
+@pytest.mark.parametrize("n,m,w,wide,dtype,early,fixed", [
+    # (smallest, largest) batch of the workgroup per sample, as measured
+    (8000, 2000, 4, (0, 0), np.float64, (1, None), (1, None)),
+    (8000, 2000, 75, (0, 0), np.float64, (1, None), (1, None)),
+    (8000, 2000, 200, (0, 0), np.float64, (1, None), (129, None)),
+    (8000, 2000, 50, (0, 0), np.float32, (1, None), (1, None)),
+    (8000, 2000, 100, (0, 0), np.float32, (1, None), (1, 512)),
+    (12000, 4000, 10, (0, 0), np.float64, (1, None), (1, None)),
+    (8000, 3000, 4, (1, 8000), np.float64, (1, 512), (1, 256)),
+    (8000, 3000, 4, (4, 2000), np.float64, (1, None), (1, 512)),
+    (8000, 3000, 4, (64, 500), np.float64, (1, None), (1, 512)),
+    (8000, 3000, 4, (4, 100), np.float64, (1, None), (1, None)),
+    (8000, 4100, 4, (0, 0), np.float64, (1, None), None),  # rows beyond one group
+])
+def test_wide_loop_where_it_pays(routes, n, m, w, wide, dtype, early, fixed):
+    """A workgroup streams the whole matrix: wide rows, one long chain and many rounds go to
+    the passes."""
+    widths = _rows(n, m, w, *wide)
+    plan = _Plan(routes, n, widths, dtype)
+    for stop, line in ((True, early), (False, fixed)):
+        for batch in (1, 64, 128, 129, 256, 257, 512, 513, 1024, 4096):
+            pays = line is not None and line[0] <= batch and (line[1] is None or batch <= line[1])
+            assert plan.wide(batch, stop) == pays, (batch, stop)
