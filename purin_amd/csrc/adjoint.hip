@@ -1371,6 +1371,13 @@ struct QPAdjArgs {
                       // no convergence masking
 };
 
+// The restart length a call runs with.  The dense layer's BiCGSTAB keeps its five work
+// vectors in the basis slots.
+static int64_t adjoint_restart(const purin_cp_plan* p, const purin_cp_adjoint_options& o,
+                               bool dense) {
+  return dense ? 5 : std::min<int64_t>({(int64_t)o.restart, (int64_t)o.max_iterations, 2 * p->n + p->m});
+}
+
 // ``size_only``: compute the workspace bytes of this call into *size_only and
 // return, touching neither the device nor the plan (purin_cp_workspace_bytes).
 template <typename T>
@@ -1392,17 +1399,13 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   const Layout L = make_layout(p, batch);
   const int64_t Bp = L.Bp, n = p->n, m = p->m, M = p->M;
   const int64_t W = 2 * n + m;
-  // the dense layer's BiCGSTAB keeps its five work vectors in the basis slots
-  const int restart = (qa && qa->dense)
-                          ? 5
-                          : (int)std::min<int64_t>({(int64_t)o.restart, (int64_t)o.max_iterations, W});
-  if (restart > kMaxRestart) return set_error(PURIN_CP_ERR_UNSUPPORTED, "restart above 128");
   const bool dense = qa && qa->dense;
+  const int restart = (int)adjoint_restart(p, o, dense);
+  if (restart > kMaxRestart) return set_error(PURIN_CP_ERR_UNSUPPORTED, "restart above 128");
   static_assert((kMaxRestart + 2) * 4 <= kPinnedBytes, "per-step counts must fit the pinned buffer");
-  // The solver runs one workgroup per sample where its vectors u and w fit LDS and the
-  // restart length its one-lane-per-vector algebra; otherwise on batch-minor passes
-  // (very large problems, long restarts)
-  const bool wg = gmr_fits(p, restart);
+  // The solver runs one workgroup per sample up to gmr_batch samples; otherwise on
+  // batch-minor passes (very large problems, long restarts, many samples)
+  const bool wg = batch <= gmr_batch(p, restart, dense);
   // workspace
   const int nchunk = (int)((W + kChunk - 1) / kChunk);
   // Gram--Schmidt passes: about 1024 blocks of 4 wavefronts over the batch tiles
@@ -2035,9 +2038,20 @@ static int adjoint_bytes_t(const purin_cp_plan* cp, int32_t entry, int64_t batch
   const QPAdjArgs<T> qa{&dummy, &dummy, &dummy, nullptr, entry == PURIN_CP_ENTRY_DENSE_ADJOINT};
   const bool per_sample = entry != PURIN_CP_ENTRY_ADJOINT;
   const bool qp = entry == PURIN_CP_ENTRY_QP_ADJOINT || entry == PURIN_CP_ENTRY_DENSE_ADJOINT;
-  return adjoint_impl<T>(p, nullptr, batch, nullptr, nullptr, o, nullptr, nullptr, nullptr,
-                         nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, per_sample,
-                         qp ? &qa : nullptr, bytes);
+  auto size = [&](int64_t samples, int64_t* out) {
+    return adjoint_impl<T>(p, nullptr, samples, nullptr, nullptr, o, nullptr, nullptr, nullptr,
+                           nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, per_sample,
+                           qp ? &qa : nullptr, out);
+  };
+  if (int rc = size(batch, bytes)) return rc;
+  // a batch's workspace serves every smaller one: the largest on the other route too
+  const bool dense = entry == PURIN_CP_ENTRY_DENSE_ADJOINT;
+  const int64_t last = gmr_batch(p, adjoint_restart(p, o, dense), dense);
+  int64_t less = 0;
+  if (last >= 1 && last < batch)
+    if (int rc = size(last, &less)) return rc;
+  *bytes = std::max(*bytes, less);
+  return PURIN_CP_OK;
 }
 
 int adjoint_workspace_bytes(const purin_cp_plan* p, int32_t entry, int64_t batch,

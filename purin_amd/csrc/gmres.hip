@@ -804,9 +804,15 @@ int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base
 
 }  // namespace
 
-bool gmr_fits(const purin_cp_plan* p, int64_t restart) {
-  return p->sl_ok && restart <= kGmrRestart &&
-         lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 <= kLdsMax;
+// BiCGSTAB's sums over the batch go through one counter and the last workgroup: ms per call
+// here against the passes, n = 60: B = 1024 5.3 (6.3), B = 2048 8.7 (6.9), B = 4096 18.0 (8.0).
+int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
+  if (!p->sl_ok || restart > kGmrRestart) return 0;
+  if (lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 > kLdsMax) return 0;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess)
+    cus = 256;
+  return dense ? 4 * (int64_t)cus : INT64_MAX;
 }
 
 template <typename T>

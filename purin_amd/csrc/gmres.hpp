@@ -46,8 +46,9 @@ struct Gmr {
   int32_t* ctrl;               // [kGmrGroup] steps of the group's cycles (largest over the batch)
 };
 
-// Whether the cycle kernel takes this plan and restart length.
-bool gmr_fits(const purin_cp_plan* p, int64_t restart);
+// The largest batch that runs one workgroup per sample (0: none), for GMRES of this restart
+// length or the dense layer's BiCGSTAB.
+int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense);
 
 // One restart cycle for every unconverged sample: cycle ``c`` of a group whose
 // earlier groups completed ``base`` steps of ``max_iterations``.

@@ -182,6 +182,7 @@ def test_dense_adjoint_matches_oracle_at_the_same_state(with_dual_cotangent, tol
     (60, 12, 25, 5),    # four wavefronts sharing a slice of rows and of columns
     (100, 30, 70, 66),  # two slices each
     (230, 20, 40, 3),   # eight wavefronts
+    (8, 2, 3, 1030),    # more samples than take a workgroup each: the batch-minor passes
 ])
 def test_dense_adjoint_wide_rows(n, me, mi, B):
     """The per-sample BiCGSTAB kernels where wavefronts share a slice's entries, at the

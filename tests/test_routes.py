@@ -17,6 +17,7 @@ from purin_amd import build as B
 HARNESS = r"""
 #include <algorithm>
 #include "forward.hpp"
+#include "gmres.hpp"
 #include "solo.hpp"
 
 using namespace purin;
@@ -54,6 +55,9 @@ extern "C" int route_solo(const purin_cp_plan* p, int64_t batch, int early, int 
 extern "C" int route_wide(const purin_cp_plan* p, int64_t batch, int early) {
   return solo_wide_fits(p, batch, early != 0);
 }
+extern "C" int64_t route_gmr(const purin_cp_plan* p, int64_t restart, int dense) {
+  return gmr_batch(p, restart, dense != 0);
+}
 extern "C" int64_t route_workspace(const purin_cp_plan* p, int entry, int64_t batch) {
   return purin_cp_workspace_bytes(p, entry, batch, nullptr);
 }
@@ -77,6 +81,8 @@ def routes(tmp_path_factory):
     lib.route_free.argtypes = [vp]
     lib.route_solo.argtypes = [vp, i64, C.c_int, C.c_int]
     lib.route_wide.argtypes = [vp, i64, C.c_int]
+    lib.route_gmr.restype = i64
+    lib.route_gmr.argtypes = [vp, i64, C.c_int]
     lib.route_workspace.restype = i64
     lib.route_workspace.argtypes = [vp, C.c_int, i64]
     return lib
@@ -104,6 +110,9 @@ class _Plan:
 
     def wide(self, batch, early):
         return bool(self.lib.route_wide(self.p, batch, int(early)))
+
+    def gmr(self, restart, dense=False):
+        return self.lib.route_gmr(self.p, restart, int(dense))
 
     def workspace(self, entry, batch):
         from purin_amd import _lib
@@ -182,3 +191,17 @@ def test_wide_loop_where_it_pays(routes, n, m, w, wide, dtype, early, fixed):
         for batch in (1, 64, 128, 129, 256, 257, 512, 513, 1024, 4096):
             pays = line is not None and line[0] <= batch and (line[1] is None or batch <= line[1])
             assert plan.wide(batch, stop) == pays, (batch, stop)
+
+
+ALL = 2**63 - 1
+
+
+@pytest.mark.parametrize("n,m,w,wide,dtype,restart,dense,batch", [
+    (60, 30, 60, (0, 0), np.float64, 5, True, 1024),  # sums over the batch through one counter
+    (20000, 50, 4, (0, 0), np.float64, 5, True, 0),   # beyond the LDS
+    (300, 90, 5, (0, 0), np.float64, 30, False, ALL),
+    (300, 90, 5, (0, 0), np.float64, 33, False, 0),
+])
+def test_adjoint_workgroups_where_they_pay(routes, n, m, w, wide, dtype, restart, dense, batch):
+    """The largest batch whose implicit VJP runs one workgroup per sample."""
+    assert _Plan(routes, n, _rows(n, m, w, *wide), dtype).gmr(restart, dense) == batch
