@@ -806,13 +806,28 @@ int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base
 
 // BiCGSTAB's sums over the batch go through one counter and the last workgroup: ms per call
 // here against the passes, n = 60: B = 1024 5.3 (6.3), B = 2048 8.7 (6.9), B = 4096 18.0 (8.0).
+//
+// GMRES: each sample stops by itself here, so whole calls are faster at any batch (ms, fp64:
+// n = 64 B = 16384 5.9 (11.7); n = 300 43 (71), with rows of 24 37.6 (39.5)), except where a
+// long row or column is one wavefront's chain, ``chain`` entries, in every round of the launch:
+// fp64 chain 1000 B = 1024 29.6 (35.4), B = 4096 106 (73); 2000 B = 512 66 (78), B = 1024 123
+// (99); 8000 B = 512 194 (225), B = 1024 366 (269).  fp32 1000 B = 4096 37 (47), B = 16384 153
+// (129); 2000 B = 1024 55 (79), B = 4096 189 (148); 8000 B = 1024 168 (221).
 int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
   if (!p->sl_ok || restart > kGmrRestart) return 0;
   if (lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 > kLdsMax) return 0;
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess)
     cus = 256;
-  return dense ? 4 * (int64_t)cus : INT64_MAX;
+  if (dense) return 4 * (int64_t)cus;
+  const int64_t W = 2 * p->n + p->m;
+  auto longest = [&](const std::vector<int32_t>& w) -> int64_t {
+    return w.empty() ? 0 : w[0] / gmr_parts(W, (int)w.size(), w[0]);
+  };
+  const int64_t chain = longest(p->sl_rw) + longest(p->sl_cw);
+  if (chain <= 256) return INT64_MAX;
+  const bool f64 = p->dtype == PURIN_CP_F64;
+  return std::max<int64_t>(f64 ? 2 : 4, (f64 ? 6000 : 18000) / chain) * cus;
 }
 
 template <typename T>

@@ -201,6 +201,12 @@ ALL = 2**63 - 1
     (20000, 50, 4, (0, 0), np.float64, 5, True, 0),   # beyond the LDS
     (300, 90, 5, (0, 0), np.float64, 30, False, ALL),
     (300, 90, 5, (0, 0), np.float64, 33, False, 0),
+    (300, 50, 4, (1, 300), np.float64, 30, False, ALL),  # eight wavefronts share the row
+    (1000, 300, 4, (1, 1000), np.float64, 30, False, 5 * 256),
+    (1000, 300, 4, (1, 1000), np.float32, 30, False, 17 * 256),
+    (4000, 600, 4, (20, 2000), np.float64, 30, False, 512),
+    (8000, 500, 4, (1, 8000), np.float64, 30, False, 512),
+    (8000, 500, 4, (1, 8000), np.float32, 30, False, 1024),
 ])
 def test_adjoint_workgroups_where_they_pay(routes, n, m, w, wide, dtype, restart, dense, batch):
     """The largest batch whose implicit VJP runs one workgroup per sample."""
