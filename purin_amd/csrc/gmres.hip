@@ -809,10 +809,13 @@ int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base
 //
 // GMRES: each sample stops by itself here, so whole calls are faster at any batch (ms, fp64:
 // n = 64 B = 16384 5.9 (11.7); n = 300 43 (71), with rows of 24 37.6 (39.5)), except where a
-// long row or column is one wavefront's chain, ``chain`` entries, in every round of the launch:
-// fp64 chain 1000 B = 1024 29.6 (35.4), B = 4096 106 (73); 2000 B = 512 66 (78), B = 1024 123
-// (99); 8000 B = 512 194 (225), B = 1024 366 (269).  fp32 1000 B = 4096 37 (47), B = 16384 153
-// (129); 2000 B = 1024 55 (79), B = 4096 189 (148); 8000 B = 1024 168 (221).
+// long row or column is one wavefront's chain, ``chain`` entries, in every round of the launch
+// and not small beside the vectors: fp64, n = 600, chain 400 B = 1024 18.2 (20.8), B = 2048
+// 34.6 (27.9); n = 1000, chain 1000 B = 1024 29.6 (35.4), B = 2048 56.7 (46.8); n = 4000, chain
+// 2000 B = 512 66 (78), B = 1024 123 (99); n = 8000, chain 8000 B = 512 194 (225), B = 1024 366
+// (269); but n = 2000, chain 600 B = 8192 193 (216).  fp32, n = 600, chain 400 B = 4096 21.9
+// (28.6); chain 600 with per-sample coefficients B = 2048 29.5 (32.3), B = 4096 51.4 (42.6);
+// n = 4000, chain 2000 B = 1024 55 (79), B = 4096 189 (148).
 int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
   if (!p->sl_ok || restart > kGmrRestart) return 0;
   if (lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 > kLdsMax) return 0;
@@ -825,9 +828,9 @@ int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
     return w.empty() ? 0 : w[0] / gmr_parts(W, (int)w.size(), w[0]);
   };
   const int64_t chain = longest(p->sl_rw) + longest(p->sl_cw);
-  if (chain <= 256) return INT64_MAX;
-  const bool f64 = p->dtype == PURIN_CP_F64;
-  return std::max<int64_t>(f64 ? 2 : 4, (f64 ? 6000 : 18000) / chain) * cus;
+  if (chain <= std::max<int64_t>(128, W / 7)) return INT64_MAX;
+  if (p->dtype == PURIN_CP_F64) return (chain <= 256 ? 8 : (chain <= 1024 ? 4 : 2)) * (int64_t)cus;
+  return (chain <= 512 ? 16 : (chain <= 1024 ? 8 : 4)) * (int64_t)cus;
 }
 
 template <typename T>

@@ -202,8 +202,11 @@ ALL = 2**63 - 1
     (300, 90, 5, (0, 0), np.float64, 30, False, ALL),
     (300, 90, 5, (0, 0), np.float64, 33, False, 0),
     (300, 50, 4, (1, 300), np.float64, 30, False, ALL),  # eight wavefronts share the row
-    (1000, 300, 4, (1, 1000), np.float64, 30, False, 5 * 256),
-    (1000, 300, 4, (1, 1000), np.float32, 30, False, 17 * 256),
+    (800, 300, 4, (2, 300), np.float64, 30, False, 1024),
+    (600, 300, 4, (4, 400), np.float32, 30, False, 4096),
+    (1000, 300, 4, (1, 1000), np.float64, 30, False, 1024),
+    (1000, 300, 4, (1, 1000), np.float32, 30, False, 2048),
+    (2000, 400, 4, (8, 600), np.float64, 30, False, ALL),  # small beside the vectors
     (4000, 600, 4, (20, 2000), np.float64, 30, False, 512),
     (8000, 500, 4, (1, 8000), np.float64, 30, False, 512),
     (8000, 500, 4, (1, 8000), np.float32, 30, False, 1024),
