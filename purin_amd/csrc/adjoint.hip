@@ -1380,13 +1380,14 @@ static int64_t adjoint_restart(const purin_cp_plan* p, const purin_cp_adjoint_op
 
 // ``size_only``: compute the workspace bytes of this call into *size_only and
 // return, touching neither the device nor the plan (purin_cp_workspace_bytes).
+// ``passes``: on the batch-minor passes, whatever the route would be.
 template <typename T>
 static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const void* saved,
                         const T* cot_y, const purin_cp_adjoint_options& o, T* g_target, T* g_rhs,
                         T* g_lower, T* g_upper, uint8_t* valid, int32_t* info, T* gres,
                         const T* values = nullptr, T* g_values = nullptr,
                         bool per_sample = false, const QPAdjArgs<T>* qa = nullptr,
-                        int64_t* size_only = nullptr) {
+                        int64_t* size_only = nullptr, bool passes = false) {
   if (!size_only && (!saved || !cot_y))
     return set_error(PURIN_CP_ERR_ARG, "NULL saved state or cotangent");
   if (!size_only && per_sample && !qa && p->nnz_full && !values)
@@ -1405,7 +1406,7 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   static_assert((kMaxRestart + 2) * 4 <= kPinnedBytes, "per-step counts must fit the pinned buffer");
   // The solver runs one workgroup per sample up to gmr_batch samples; otherwise on
   // batch-minor passes (very large problems, long restarts, many samples)
-  const bool wg = batch <= gmr_batch(p, restart, dense);
+  const bool wg = !passes && batch <= gmr_batch(p, restart, dense);
   // workspace
   const int nchunk = (int)((W + kChunk - 1) / kChunk);
   // Gram--Schmidt passes: about 1024 blocks of 4 wavefronts over the batch tiles
@@ -1421,7 +1422,7 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   const size_t vec = (size_t)W * Bp * es;
   size_t o_ = 0;
   auto take = [&](size_t bytes) { size_t r = o_; o_ = al(o_ + bytes); return r; };
-  const size_t oX = take(vec), oCm = take(n * Bp * es), oClo = take(n * Bp * es),
+  const size_t oCm = take(n * Bp * es), oClo = take(n * Bp * es),
                oChi = take(n * Bp * es), oDm = take(m * Bp * es), oDp = take(m * Bp * es),
                oU = take(n * Bp * es), oThr = take(Bp * es), oRinf = take(Bp * es),
                oS2 = take(Bp * es), oLw = take(Bp * es), oGt = take(n * Bp * es),
@@ -1448,11 +1449,14 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
   const int64_t Wp = round_up(W, 16);
   const bool dg = per_sample || p->diag;
   const size_t smp = wg ? (size_t)batch * es : 0;
-  const size_t zZ = take(smp * (restart + 1) * Wp), zX = take(smp * Wp), zR = take(smp * Wp),
-               zG = take(smp * Wp), zM = take(smp * (n + m)), zA = take(dg ? smp * n : 0),
-               zD = take(dg ? smp * n : 0), zS = take(dg ? smp * m : 0),
-               zRv = take(per_sample ? smp * p->sl_rn : 0),
-               zCv = take(per_sample ? smp * p->sl_cn : 0);
+  // (the plan's own coefficients, values == nullptr: one copy)
+  const size_t ent = !per_sample ? 0 : (size_only || values ? smp : (wg ? es : 0));
+  const size_t zZ = take(wg ? std::max(smp * (restart + 1) * Wp, vec) : 0), zX = take(smp * Wp),
+               zR = take(smp * Wp), zG = take(smp * Wp), zM = take(smp * (n + m)),
+               zA = take(dg ? smp * n : 0), zD = take(dg ? smp * n : 0), zS = take(dg ? smp * m : 0),
+               zRv = take(ent * p->sl_rn), zCv = take(ent * p->sl_cn);
+  // the solution for the final pullback: in the basis, which is free by then
+  const size_t oX = wg ? zZ : take(vec);
   // per-sample coefficients: the forward's per-sample arrays are rebuilt from
   // values in a region laid out like the forward workspace, plus sigma . w and
   // the coefficient gradient in entry order
@@ -1518,6 +1522,9 @@ static int adjoint_impl(purin_cp_plan* p, hipStream_t st, int64_t batch, const v
 
   int err = PURIN_CP_OK;
   char* ws = (char*)workspace(p, o_, st, &err, true, o.workspace, o.workspace_bytes);
+  if (!ws && wg)  // the passes may need less
+    return adjoint_impl<T>(p, st, batch, saved, cot_y, o, g_target, g_rhs, g_lower, g_upper, valid,
+                           info, gres, values, g_values, per_sample, qa, nullptr, true);
   if (!ws) return err;
   HostWords hw(p);  // this call's host words for the counter reads
   T* Vb = (T*)(ws + oV);

@@ -18,6 +18,7 @@ import pytest
 
 from purin_amd import workloads
 from purin_amd._lib import ERR_ARG, PurinError
+from purin_amd.plan import Plan
 from tests._gpu import canonical_from_workload, plan_for, rel_err, require_gpu, to_np
 
 pytestmark = pytest.mark.gpu
@@ -140,6 +141,50 @@ def test_wide_problem_runs_in_the_passes_workspace(shared):
     got = plan.project(w.target, rhs, workspace=full, timing=True, **kw)
     assert plan.last_timing()["resident"] == 1
     assert rel_err(to_np(got.y), to_np(want.y)) <= 1e-11
+
+
+def test_adjoint_of_a_dense_row_runs_in_the_passes_workspace():
+    """A dense row pads 63 others in the per-sample entries of the backward with per-sample
+    coefficients (131 MB here): a call that the passes' workspace holds runs in it, and the
+    plan's own coefficients take one copy."""
+    torch = require_gpu()
+    B, n = 128, 2000
+    rng = np.random.default_rng(3)
+    ptr, idx = np.array([0, n, n + 4]), np.concatenate((np.arange(n), [3, 70, 800, 1999]))
+    val = rng.normal(size=n + 4) / np.sqrt(n)
+    box = np.arange(2 * n)
+    plan = Plan(n, 1, 1 + 2 * n, np.concatenate((ptr, n + 5 + box)),
+                np.concatenate((idx, box % n)),
+                np.concatenate((val, np.ones(n), -np.ones(n))), dtype=torch.float64)
+    values = np.tile(np.concatenate((val, np.ones(n), -np.ones(n))), (B, 1))
+    values[:, :n] *= rng.uniform(0.9, 1.1, (B, 1))
+    rhs = np.concatenate((np.zeros((B, 1)), np.full((B, 1), 0.3), np.ones((B, 2 * n))), axis=1)
+    fwd = plan.project(rng.normal(size=(B, n)), rhs, values=values, max_iterations=60,
+                       early_stop=False, save=True)
+    cot = rng.normal(size=(B, n))
+    kw = dict(values=values, force_eligible=True, tolerance=1e-13, max_iterations=200)
+
+    def adjoint(nbytes):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+        return plan.adjoint(fwd.saved, None, None, cot, workspace=ws, **kw)
+
+    with pytest.raises(PurinError, match="workspace too small") as err:
+        adjoint(256)
+    least = int(re.search(r"needs (\d+) bytes", str(err.value)).group(1))
+    full = plan.workspace_bytes("adjoint_values", B)
+    assert full - least > 100e6
+    a, b = adjoint(least), adjoint(full)
+    np.testing.assert_array_equal(to_np(a.info), 0)
+    np.testing.assert_array_equal(to_np(b.info), 0)
+    for f in ("g_target", "g_rhs", "g_values"):  # GMRES residuals of 1e-13, condition below 1e3
+        assert rel_err(to_np(getattr(a, f)), to_np(getattr(b, f))) <= 1e-9, f
+    # the QP's backward with the plan's own coefficients
+    qp = Plan(n, 1, 1, ptr, idx, val, dtype=torch.float64, bound_presolve=False)
+    q = np.ones((B, n))
+    state = qp.qp_solve(q, q, rhs[:, :2], -q, q, max_iterations=20, early_stop=False, save=True)
+    qp.qp_adjoint(state.saved, q, q, cot, force_eligible=True)
+    assert (qp.workspace_bytes("qp_adjoint", B) - qp.current_info().adjoint_workspace_bytes
+            > 100e6)
 
 
 def test_two_streams_on_one_plan():
