@@ -101,6 +101,38 @@ def test_dense_one_workgroup_loop(n, me, mi, B, accelerated, dtype):
             assert it[0] < iters
 
 
+@pytest.mark.parametrize("n,me,mi", [(13, 2, 3), (60, 12, 25), (200, 20, 44)])
+@pytest.mark.parametrize("early", [False, True])
+def test_dense_nonfinite_inputs(n, me, mi, early):
+    """A NaN bound, a NaN and an infinite cost and infinite bounds, each in one sample: non-finite
+    entries in the oracle's places, the other samples at the parity bar.  A sample with a
+    non-finite iterate is never accepted, so every sample runs to the limit."""
+    require_gpu()
+    q, c, A, b, C, d, lo, hi = _problem(62, B=6, n=n, me=me, mi=mi)
+    lo[1, 2] = np.nan
+    c[2, 3] = np.nan
+    c[3, 1] = -np.inf
+    lo[4], hi[4] = -np.inf, np.inf
+    iters = 40
+    with np.errstate(invalid="ignore", over="ignore"):
+        y, lam, mu, it, _ = od.solve_dense(q, c, A, b, C, d, lo, hi, max_iterations=iters,
+                                           tolerance=1e-3 if early else 1e-300)
+    want, wm = y, np.concatenate((lam, mu), axis=1)
+    assert np.all(it == iters) and not np.isfinite(y[[1, 2]]).all(axis=1).any()
+    got, gm, git, _ = _dense_plan(n, me, mi, np.float64).dense_solve(
+        q, c, np.concatenate((b, d), axis=1), lo, hi,
+        values=np.concatenate((A, C), axis=1).reshape(6, -1), max_iterations=iters,
+        tolerance=1e-3 if early else 1e-30, early_stop=early)
+    np.testing.assert_array_equal(to_np(git), it)
+    for g, w in ((to_np(got), want), (to_np(gm), wm)):
+        np.testing.assert_array_equal(np.isnan(g), np.isnan(w))
+        inf = np.isinf(w)
+        np.testing.assert_array_equal(np.isinf(g), inf)
+        np.testing.assert_array_equal(g[inf], w[inf])
+        fin = np.isfinite(w)
+        assert rel_err(g[fin], w[fin]) <= TOL[np.float64]
+
+
 def test_dense_packed_inequality_support():
     """A packed inequality support (sparse_layer.py:44-122): the inequality rows
     keep only their listed columns; the same iteration otherwise."""

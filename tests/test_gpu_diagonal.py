@@ -82,7 +82,8 @@ def test_diagonal_project_matches_oracle(dtype):
     assert rel_err(mult, want_mult) <= TOL[dtype]
 
 
-def test_diagonal_vjp_matches_oracle_at_the_same_state():
+@pytest.mark.parametrize("restart", [30, 45])  # one workgroup per sample, batch-minor passes
+def test_diagonal_vjp_matches_oracle_at_the_same_state(restart):
     """The adjoint linearises the preconditioned cp_step (per-row sigma, per-variable
     tau) at the GPU's converged state; converged GMRES at 1e-14."""
     from oracle import adjoint as oadj
@@ -96,7 +97,7 @@ def test_diagonal_vjp_matches_oracle_at_the_same_state():
     target = w.target
     cot = np.random.default_rng(3).normal(size=(B, canon.n))
     cfg = op.Config(max_iterations=20000, tolerance=1e-9, diagonal_preconditioning=True,
-                    gmres_tolerance=1e-14, gmres_max_iterations=300)
+                    gmres_tolerance=1e-14, gmres_restart=restart, gmres_max_iterations=300)
     pre = op.presolve(canon, rhs, cfg, dtype)
     plan = plan_for(canon, dtype=dtype, diagonal_preconditioning=True)
     o, saved = plan.solve(pre.kept_rhs, target, pre.lower, pre.upper, tol=pre.tolerance,
@@ -108,7 +109,7 @@ def test_diagonal_vjp_matches_oracle_at_the_same_state():
     want = oadj.adjoint(pre.kept_values[0], ksup, kmask, canon.me, to_np(o.y), to_np(o.dual),
                         conv, target, pre.kept_rhs, pre.lower, pre.upper, cot, cfg)
     adj = plan.adjoint(saved, target, pre.kept_rhs, cot, bounds_grad=True, rhs_rows=plan.m,
-                       tolerance=cfg.gmres_tolerance, max_iterations=cfg.gmres_max_iterations)
+                       restart=restart, tolerance=cfg.gmres_tolerance, max_iterations=cfg.gmres_max_iterations)
     np.testing.assert_array_equal(to_np(adj.valid), want.valid)
     np.testing.assert_array_equal(to_np(adj.info), want.info)
     assert rel_err(to_np(adj.g_target), want.g_target) <= 1e-10

@@ -190,7 +190,7 @@ def test_crossed_bounds_keep_running_under_early_stop(dtype):
     infeasible; the reference's stop test sees their bound violation
     (kernels.py:158-175) and never accepts them, so they run to
     max_iterations with status 1, beside feasible samples of the same batch
-    (y0 in [-1, 1]) that stop on their own.  The resident early-stop kernel
+    (y0 in [-1, 1]) that stop on their own.  The loop of one workgroup per sample
     (which drops the violation term on lanes whose bounds cannot be violated)
     and the streaming passes against the oracle."""
     require_gpu()
@@ -215,6 +215,31 @@ def test_crossed_bounds_keep_running_under_early_stop(dtype):
         np.testing.assert_array_equal(to_np(got.status), want.status)
         if dtype == np.float64:
             np.testing.assert_array_equal(it, want.iterations)
+
+
+@pytest.mark.parametrize("n,me,mi", [(1100, 80, 160), (4200, 200, 300)])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_crossed_bounds_in_large_problems(n, me, mi, dtype):
+    """The same on the resident early-stop tiles and the loop beyond them: samples with one
+    crossed pair of bounds run to the limit with status 1, their neighbours stop."""
+    require_gpu()
+    B, limit = 6, 3000
+    w = workloads.ragged_rows(77, n=n, me=me, mi=mi, wmin=2, wmax=5, batch=B)
+    plan = plan_for(canonical_from_workload(w), dtype=dtype)
+    rhs = np.tile(w.rhs, (B, 1)).astype(dtype)
+    crossed = np.arange(B) % 2 == 0
+    # each variable's two bound rows are among the last 2 n: y <= u, -y <= -l
+    rows = [k for k in range(me + mi, w.rows_total) if w.indices[w.indptr[k]] == 0]
+    assert len(rows) == 2
+    rhs[np.ix_(crossed, rows)] = [[0.0 if w.data[w.indptr[k]] > 0 else -1.0 for k in rows]]
+    for streaming in (False, True):
+        got = plan.project(w.target.astype(dtype), rhs, max_iterations=limit, tolerance=1e-2,
+                           streaming=streaming, timing=True)
+        assert plan.last_timing()["resident"] == (0 if streaming else 1)
+        it, status = to_np(got.iterations), to_np(got.status)
+        np.testing.assert_array_equal(it[crossed], limit)
+        assert np.all(it[~crossed] < limit)
+        np.testing.assert_array_equal(status, crossed.astype(status.dtype))
 
 
 def test_known_answer_no_constraints_identity():
@@ -266,19 +291,24 @@ def _same_nonfinite(got, want, bar, what):
     assert rel_err(got[fin], want[fin]) <= bar, what
 
 
+@pytest.mark.parametrize("n,me,mi", [
+    (48, 8, 20),       # one workgroup per sample
+    (1100, 80, 160),   # the resident tiles
+    (4200, 200, 300),  # beyond them
+])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("early_stop", [False, True])
-def test_nonfinite_bounds_and_targets(dtype, early_stop):
+def test_nonfinite_bounds_and_targets(dtype, early_stop, n, me, mi):
     """Per-sample bounds with NaN entries (the lanes whose clip propagates NaN,
     kernels.py:133-147's jnp.clip), infinite bounds, a tied box, and NaN and
-    infinite targets, in some samples of a batch: the resident kernel (fixed
+    infinite targets, in some samples of a batch: the on-chip loops (fixed
     and early stop) and the streaming passes each against the oracle.  NaN
     and infinity land in the same places; the other samples keep the parity
     bar and, in fp64, the oracle's iteration counts (a sample with a
     non-finite iterate never passes the stop test)."""
     torch = require_gpu()
     B = 40
-    w = workloads.small_random(13, n=48, me=8, mi=20, width=4, batch=B)
+    w = workloads.small_random(13, n=n, me=me, mi=mi, width=4, batch=B)
     canon = canonical_from_workload(w)
     rhs = np.tile(w.rhs, (B, 1)).astype(dtype)
     target = w.target.astype(dtype).copy()

@@ -315,15 +315,16 @@ def test_qp_shared_values_and_warm_start(early_stop):
     np.testing.assert_array_equal(to_np(got2.iterations), to_np(got_s.iterations))
 
 
+@pytest.mark.parametrize("restart", [30, 39])  # one workgroup per sample, batch-minor passes
 @pytest.mark.parametrize("mode", ["scalar", "diagonal"])
-def test_qp_vjp_matches_oracle_at_the_same_state(mode):
+def test_qp_vjp_matches_oracle_at_the_same_state(mode, restart):
     """All six gradients and the dual cotangent's path at the GPU's converged
     state; converged GMRES at 1e-14."""
     require_gpu()
     rows, me, mi, n, support, mask, data = _problem(44, n=16, me=2, mi=5, width=3, B=20)
     kw = dict(diagonal_preconditioning=True) if mode == "diagonal" else {}
     cfg = Config(max_iterations=30000, tolerance=1e-9, gmres_tolerance=1e-14,
-                 gmres_max_iterations=300, **kw)
+                 gmres_restart=restart, gmres_max_iterations=300, **kw)
     plan = _plan(rows, me, mi, n, np.float64, **kw)
     vals = data.values[:, mask]
     fwd = plan.qp_solve(data.q, data.c, data.rhs, data.lower, data.upper, values=vals,
@@ -339,7 +340,8 @@ def test_qp_vjp_matches_oracle_at_the_same_state(mode):
                           state=(to_np(fwd.y), dual))
     np.testing.assert_array_equal(status, res.status)
     adj = plan.qp_adjoint(fwd.saved, data.q, data.c, cot, values=vals, cot_dual=cot_dual,
-                          tolerance=cfg.gmres_tolerance, max_iterations=cfg.gmres_max_iterations)
+                          restart=restart, tolerance=cfg.gmres_tolerance,
+                          max_iterations=cfg.gmres_max_iterations)
     np.testing.assert_array_equal(to_np(adj.valid), oadj.valid)
     np.testing.assert_array_equal(to_np(adj.info), oadj.info)
     for name, want in (("g_q", g.q), ("g_c", g.c), ("g_rhs", g.rhs), ("g_lower", g.lower),

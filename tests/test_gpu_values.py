@@ -229,7 +229,8 @@ def test_shared_values_match_the_shared_path():
     assert torch.equal(b.iterations, a.iterations)
 
 
-def test_values_vjp_matches_oracle_at_the_same_state():
+@pytest.mark.parametrize("restart", [30, 40])  # one workgroup per sample, batch-minor passes
+def test_values_vjp_matches_oracle_at_the_same_state(restart):
     """g_target, g_rhs and g_values (the VJP of cp_step w.r.t. the scaled
     coefficients, chained through row scaling and the bound thresholds) at the
     GPU's converged state; converged GMRES at 1e-14."""
@@ -241,7 +242,7 @@ def test_values_vjp_matches_oracle_at_the_same_state():
     target = w.target
     cot = np.random.default_rng(9).normal(size=(B, canon.n))
     cfg = op.Config(max_iterations=20000, tolerance=1e-9, gmres_tolerance=1e-14,
-                    gmres_max_iterations=300)
+                    gmres_restart=restart, gmres_max_iterations=300)
     plan = plan_for(canon, dtype=dtype)
     vcsr = _csr(values, mask)
     fwd = plan.project(target, rhs, values=vcsr, tolerance=cfg.tolerance,
@@ -253,7 +254,7 @@ def test_values_vjp_matches_oracle_at_the_same_state():
     res, g_t, g_r, oadj, g_v = op.vjp(canon, target, rhs, cfg, cot, values=values,
                                       return_values=True, state=(to_np(fwd.y), dual))
     np.testing.assert_array_equal(status, res.status)
-    adj = plan.adjoint(fwd.saved, None, None, cot, values=vcsr,
+    adj = plan.adjoint(fwd.saved, None, None, cot, values=vcsr, restart=restart,
                        tolerance=cfg.gmres_tolerance, max_iterations=cfg.gmres_max_iterations)
     np.testing.assert_array_equal(to_np(adj.valid), oadj.valid)
     np.testing.assert_array_equal(to_np(adj.info), oadj.info)
