@@ -804,6 +804,10 @@ int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base
 
 }  // namespace
 
+bool gmr_holds(const purin_cp_plan* p) {
+  return lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 <= kLdsMax;
+}
+
 // BiCGSTAB's sums over the batch go through one counter and the last workgroup: ms per call
 // here against the passes, n = 60: B = 1024 5.3 (6.3), B = 2048 8.7 (6.9), B = 4096 18.0 (8.0).
 //
@@ -817,8 +821,7 @@ int dispatch(hipStream_t st, const Gmr<T>& A, int64_t batch, int c, int64_t base
 // (28.6); chain 600 with per-sample coefficients B = 2048 29.5 (32.3), B = 4096 51.4 (42.6);
 // n = 4000, chain 2000 B = 1024 55 (79), B = 4096 189 (148).
 int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
-  if (!p->sl_ok || restart > kGmrRestart) return 0;
-  if (lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p) + 64 > kLdsMax) return 0;
+  if (!p->sl_ok || restart > kGmrRestart || !gmr_holds(p)) return 0;
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device) != hipSuccess)
     cus = 256;

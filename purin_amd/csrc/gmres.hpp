@@ -46,6 +46,9 @@ struct Gmr {
   int32_t* ctrl;               // [kGmrGroup] steps of the group's cycles (largest over the batch)
 };
 
+// Whether a workgroup's LDS holds the products' vectors (n + m up to 16,130 in fp64, 36,600 in
+// fp32).
+bool gmr_holds(const purin_cp_plan* p);
 // The largest batch that runs one workgroup per sample (0: none), for GMRES of this restart
 // length or the dense layer's BiCGSTAB.
 int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense);

@@ -1112,8 +1112,11 @@ static size_t wide_lds(const purin_cp_plan* p, bool early) {
 // 55.9 / 40.1 at B = 1024 (162 / 59.8); n = 6000, m = 2100 fp64 12.6 / 10.1 (85.6 / 17.9) and
 // 51.4 / 40.5 (140 / 59.1).  Fixed iterations of more than 4096 rows stay on the passes,
 // whose narrow column tiles serve them.
+bool solo_wide_holds(const purin_cp_plan* p) {
+  return !p->res_ok && !p->diag && p->m >= 1 && wide_lds(p, false) <= kLdsMax;
+}
 bool solo_wide_can(const purin_cp_plan* p, bool early) {
-  if (!p->sl_ok || p->res_ok || p->diag || p->m < 1) return false;
+  if (!p->sl_ok || !solo_wide_holds(p)) return false;
   if (!early && p->sl_nsr > 16 * kWideU) return false;
   return wide_lds(p, early) <= kLdsMax;
 }

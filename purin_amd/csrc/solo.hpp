@@ -88,7 +88,9 @@ struct SoloWide {
   T* Y;
   T* D;
 };
-// Whether the kernel takes this plan, and whether it pays for this batch.
+// Whether a workgroup's LDS holds the plan's vectors, whether the kernel takes it, and whether
+// it pays for this batch.
+bool solo_wide_holds(const purin_cp_plan* p);
 bool solo_wide_can(const purin_cp_plan* p, bool early);
 bool solo_wide_fits(const purin_cp_plan* p, int64_t batch, bool early);
 template <typename T>

@@ -251,3 +251,21 @@ def test_timing_counts_the_iterations_that_ran(n, me, mi, dense):
         counts = to_np(plan.project(w.target, np.tile(w.rhs, (B, 1)), **kw).iterations)
     t = plan.last_timing()
     assert t["resident"] == 1 and t["iterations"] == counts.max() < limit
+
+
+def test_plan_keeps_slices_only_where_a_kernel_reads_them():
+    """Two dense rows of 60,000 columns pad 62 others in the sliced rows, 60 MB; no kernel
+    that reads the slices holds such vectors."""
+    torch = require_gpu()
+    from purin_amd.plan import Plan
+
+    n = 60000
+    ptr, idx = np.array([0, n, 2 * n]), np.tile(np.arange(n), 2)
+    val = np.random.default_rng(1).normal(size=2 * n)
+    Plan(8, 1, 1, np.array([0, 2, 4]), np.array([0, 1, 2, 3]), np.ones(4))  # the library's own
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan = Plan(n, 2, 0, ptr, idx, val)
+    assert free - torch.cuda.mem_get_info()[0] < 32e6
+    y = plan.project(np.zeros((1, n)), np.array([[1.0, -2.0]]), max_iterations=400).y
+    np.testing.assert_allclose(to_np(y)[0] @ val.reshape(2, n).T, [1.0, -2.0], atol=1e-6)
