@@ -38,8 +38,10 @@ Layout make_layout(const purin_cp_plan* p, int64_t batch, bool values, int extra
   // The passes that leave partials take 8 rows or columns per wavefront, one after the
   // other; small problems, where that leaves CUs idle, take one (n = 24, batch 1: column
   // diagnostics 20.6 -> 7.6 us, row diagnostics 17.5 -> 6.8, multiplier recovery 30.5 ->
-  // 7.8 and 10.6 -> 4.6).  Not beyond 1024 columns: the per-sample folds walk the blocks'
-  // partials one after the other.
+  // 7.8 and 10.6 -> 4.6), and so the streaming loops with the stop test, which run two of
+  // them each iteration (us per iteration, n = 24 batch 1 54 -> 34, n = 300 batch 1024 53 ->
+  // 31, n = 1000 batch 256 72 -> 37).  Not beyond 1024 columns: the per-sample folds walk the
+  // blocks' partials one after the other.
   const int64_t TS = es == 8 ? tile_samples<double>() : tile_samples<float>();
   const bool may = (extras & kLayoutFine) && n <= 1024 && m <= 1024;
   const int64_t fine_tiles = may ? 255 / std::max(L.ncb, 1) : 0;

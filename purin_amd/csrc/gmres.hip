@@ -605,7 +605,9 @@ __global__ __launch_bounds__(BS) void k_gmr_cycle(Gmr<T> A, int c, int64_t base,
 // --- BiCGSTAB over the batch --------------------------------------------------------
 
 // The batch's sums of the workgroups' N values: each leaves its own in ``part``, and the
-// last to arrive adds them in sample order and hands them to ``then`` (one thread).
+// last to arrive adds them and hands them to ``then`` (one thread).  The order is fixed,
+// whichever arrives last: samples tid, tid + BS, ... in each thread, the lanes' tree, then the
+// wavefronts in order.
 template <typename T, int BS, int N, typename Then>
 __device__ __forceinline__ void batch_sums(const GmrBi<T>& B, T (&v)[N], T* red, Then then) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
