@@ -821,7 +821,8 @@ bool gmr_holds(const purin_cp_plan* p) {
 // 2000 B = 512 66 (78), B = 1024 123 (99); n = 8000, chain 8000 B = 512 194 (225), B = 1024 366
 // (269); but n = 2000, chain 600 B = 8192 193 (216).  fp32, n = 600, chain 400 B = 4096 21.9
 // (28.6); chain 600 with per-sample coefficients B = 2048 29.5 (32.3), B = 4096 51.4 (42.6);
-// n = 4000, chain 2000 B = 1024 55 (79), B = 4096 189 (148).
+// n = 4000, chain 2000 B = 1024 55 (79), B = 4096 189 (148); n = 8000, chain 8000 B = 1024 256
+// (223).
 int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
   if (!p->sl_ok || restart > kGmrRestart || !gmr_holds(p)) return 0;
   int cus = 0;
@@ -835,7 +836,7 @@ int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
   const int64_t chain = longest(p->sl_rw) + longest(p->sl_cw);
   if (chain <= std::max<int64_t>(128, W / 7)) return INT64_MAX;
   if (p->dtype == PURIN_CP_F64) return (chain <= 256 ? 8 : (chain <= 1024 ? 4 : 2)) * (int64_t)cus;
-  return (chain <= 512 ? 16 : (chain <= 1024 ? 8 : 4)) * (int64_t)cus;
+  return (chain <= 512 ? 16 : (chain <= 1024 ? 8 : (chain <= 4096 ? 4 : 2))) * (int64_t)cus;
 }
 
 template <typename T>

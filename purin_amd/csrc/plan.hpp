@@ -107,9 +107,10 @@ struct purin_cp_plan {
   hipStream_t upload = nullptr;      // the plan's own stream for schedule uploads
   std::mutex mu;                     // guards the schedule, timing, adjoint stats and steps
 
-  // sliced rows and columns of the scaled kept matrix (the adjoint's per-sample
-  // kernels): positions in decreasing degree, 64 to a slice, each slice's entries
-  // in [entry][lane] order padded to its widest row / column (index n / m, value 0)
+  // sliced rows and columns of the scaled kept matrix (the kernels of one workgroup per
+  // sample, solo.hip and gmres.hip; sl_ok false where no such kernel takes the plan):
+  // positions in decreasing degree, 64 to a slice, each slice's entries in [entry][lane]
+  // order padded to its widest row / column (index n / m, value 0)
   bool sl_ok = false;
   int32_t sl_nsr = 0, sl_nsc = 0;    // slices
   std::vector<int32_t> sl_rw, sl_cw; // entries per lane of each slice (decreasing)

@@ -209,7 +209,8 @@ ALL = 2**63 - 1
     (2000, 400, 4, (8, 600), np.float64, 30, False, ALL),  # small beside the vectors
     (4000, 600, 4, (20, 2000), np.float64, 30, False, 512),
     (8000, 500, 4, (1, 8000), np.float64, 30, False, 512),
-    (8000, 500, 4, (1, 8000), np.float32, 30, False, 1024),
+    (4000, 600, 4, (20, 2000), np.float32, 30, False, 1024),
+    (8000, 500, 4, (1, 8000), np.float32, 30, False, 512),
 ])
 def test_adjoint_workgroups_where_they_pay(routes, n, m, w, wide, dtype, restart, dense, batch):
     """The largest batch whose implicit VJP runs one workgroup per sample."""
