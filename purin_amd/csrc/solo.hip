@@ -1132,13 +1132,16 @@ bool solo_wide_can(const purin_cp_plan* p, bool early) {
 //   but B = 64 rows of 200 135 (119), n = 12000 rows of 75 107 (81); fp32 rows of 50 324 (392)
 //   at B = 4096, of 100 162 (136) at B = 1024, n = 6000 rows of 300 1116 (668) at B = 4096;
 //   up to B = 512 better at any width.  With the stop test better at any width and batch.
+//   fp32, few rows and columns, fixed: a round is latency, n = 4200, m = 200 B = 1024 14.8
+//   (18.5), B = 4096 58.9 (47.3); n = 5000, m = 400 B = 4096 70 (60); m = 1500 80 (93).
 bool solo_wide_fits(const purin_cp_plan* p, int64_t batch, bool early) {
   if (!solo_wide_can(p, early)) return false;
   const int64_t cus = cu_count(p), chain = (int64_t)p->sl_rw[0] + p->sl_cw[0];
-  const bool uneven = chain > 4 * ((p->sl_rn + p->sl_cn) / kWideThreads);
+  const bool uneven = chain > std::max<int64_t>(128, 4 * ((p->sl_rn + p->sl_cn) / kWideThreads));
   if (early) return !uneven || chain <= 2048 || batch <= 2 * cus;
   if (uneven) return batch <= (chain <= 4096 ? 2 : 1) * cus;
   if (p->dtype == PURIN_CP_F64) return p->nnz <= 160000 || batch > 128;
+  if (batch > 4 * cus && p->n + p->m < 5500) return false;
   return batch <= 2 * cus || p->nnz <= 13 * (p->n + p->m);
 }
 

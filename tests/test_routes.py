@@ -181,6 +181,8 @@ def test_one_workgroup_per_sample_where_it_pays(routes, n, m, w, wide, dtype, ea
     (8000, 3000, 4, (64, 500), np.float64, (1, None), (1, 512)),
     (8000, 3000, 4, (4, 100), np.float64, (1, None), (1, None)),
     (8000, 4100, 4, (0, 0), np.float64, (1, None), None),  # rows beyond one group
+    (4200, 200, 4, (0, 0), np.float64, (1, None), (1, None)),  # nearly empty
+    (4200, 200, 12, (0, 0), np.float32, (1, None), (1, 1024)),
 ])
 def test_wide_loop_where_it_pays(routes, n, m, w, wide, dtype, early, fixed):
     """A workgroup streams the whole matrix: wide rows, one long chain and many rounds go to
