@@ -400,7 +400,7 @@ enum purin_cp_entry {
 };
 
 /*
- * Bytes of caller workspace an entry point needs for ``batch`` samples: the
+ * Bytes of caller workspace an entry point needs for ``batch`` samples or fewer: the
  * largest over its optional arguments (a NULL ``saved``, whose state then
  * lives in the workspace; warm-start multipliers or duals; a dual cotangent).
  * For the adjoints ``adjoint_opts`` gives the GMRES restart length (NULL: the
