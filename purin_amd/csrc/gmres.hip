@@ -816,10 +816,12 @@ bool gmr_holds(const purin_cp_plan* p) {
 // GMRES: each sample stops by itself here, so whole calls are faster at any batch (ms, fp64:
 // n = 64 B = 16384 5.9 (11.7); n = 300 43 (71), with rows of 24 37.6 (39.5)), except where a
 // long row or column is one wavefront's chain, ``chain`` entries, in every round of the launch
-// and not small beside the vectors: fp64, n = 600, chain 400 B = 1024 18.2 (20.8), B = 2048
+// and not small beside the vectors, whose streams it hides behind where two workgroups share
+// a CU: fp64, n = 600, chain 400 B = 1024 18.2 (20.8), B = 2048
 // 34.6 (27.9); n = 1000, chain 1000 B = 1024 29.6 (35.4), B = 2048 56.7 (46.8); n = 4000, chain
 // 2000 B = 512 66 (78), B = 1024 123 (99); n = 8000, chain 8000 B = 512 194 (225), B = 1024 366
-// (269); but n = 2000, chain 600 B = 8192 193 (216).  fp32, n = 600, chain 400 B = 4096 21.9
+// (269); but n = 2000, chain 600 B = 8192 193 (216), n = 4000, chain 1150 B = 4096 202 (217);
+// one workgroup per CU, n = 8000, m = 2500, chain 1500 B = 512 89 (102), B = 2048 343 (248).  fp32, n = 600, chain 400 B = 4096 21.9
 // (28.6); chain 600 with per-sample coefficients B = 2048 29.5 (32.3), B = 4096 51.4 (42.6);
 // n = 4000, chain 2000 B = 1024 55 (79), B = 4096 189 (148); n = 8000, chain 8000 B = 1024 256
 // (223).
@@ -834,7 +836,8 @@ int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
     return w.empty() ? 0 : w[0] / gmr_parts(W, (int)w.size(), w[0]);
   };
   const int64_t chain = longest(p->sl_rw) + longest(p->sl_cw);
-  if (chain <= std::max<int64_t>(128, W / 7)) return INT64_MAX;
+  const size_t lds = lds_elems(p->n, p->m, 0, 0, 512, false) * elem_size(p);
+  if (chain <= std::max<int64_t>(128, lds <= kLdsMax / 2 ? W / 7 : W / 50)) return INT64_MAX;
   if (p->dtype == PURIN_CP_F64) return (chain <= 256 ? 8 : (chain <= 1024 ? 4 : 2)) * (int64_t)cus;
   return (chain <= 512 ? 16 : (chain <= 1024 ? 8 : (chain <= 4096 ? 4 : 2))) * (int64_t)cus;
 }

@@ -209,6 +209,9 @@ ALL = 2**63 - 1
     (1000, 300, 4, (1, 1000), np.float64, 30, False, 1024),
     (1000, 300, 4, (1, 1000), np.float32, 30, False, 2048),
     (2000, 400, 4, (8, 600), np.float64, 30, False, ALL),  # small beside the vectors
+    (8000, 2500, 4, (4, 1500), np.float64, 30, False, 512),  # but one workgroup per CU
+    (8000, 2500, 4, (4, 1500), np.float32, 30, False, ALL),
+    (8000, 2000, 50, (0, 0), np.float64, 30, False, ALL),
     (4000, 600, 4, (20, 2000), np.float64, 30, False, 512),
     (8000, 500, 4, (1, 8000), np.float64, 30, False, 512),
     (4000, 600, 4, (20, 2000), np.float32, 30, False, 1024),
