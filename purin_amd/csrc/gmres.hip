@@ -816,15 +816,17 @@ bool gmr_holds(const purin_cp_plan* p) {
 // GMRES: each sample stops by itself here, so whole calls are faster at any batch (ms, fp64:
 // n = 64 B = 16384 5.9 (11.7); n = 300 43 (71), with rows of 24 37.6 (39.5)), except where a
 // long row or column is one wavefront's chain, ``chain`` entries, in every round of the launch
-// and not small beside the vectors, whose streams it hides behind where two workgroups share
-// a CU: fp64, n = 600, chain 400 B = 1024 18.2 (20.8), B = 2048
-// 34.6 (27.9); n = 1000, chain 1000 B = 1024 29.6 (35.4), B = 2048 56.7 (46.8); n = 4000, chain
-// 2000 B = 512 66 (78), B = 1024 123 (99); n = 8000, chain 8000 B = 512 194 (225), B = 1024 366
-// (269); but n = 2000, chain 600 B = 8192 193 (216), n = 4000, chain 1150 B = 4096 202 (217);
-// one workgroup per CU, n = 8000, m = 2500, chain 1500 B = 512 89 (102), B = 2048 343 (248).  fp32, n = 600, chain 400 B = 4096 21.9
-// (28.6); chain 600 with per-sample coefficients B = 2048 29.5 (32.3), B = 4096 51.4 (42.6);
-// n = 4000, chain 2000 B = 1024 55 (79), B = 4096 189 (148); n = 8000, chain 8000 B = 1024 256
-// (223).
+// and not small beside the vectors, whose streams hide it where two workgroups share a CU:
+//   fp64  n = 600, chain 400: B = 1024 18.2 (20.8), B = 2048 34.6 (27.9)
+//         n = 1000, chain 1000: B = 1024 29.6 (35.4), B = 2048 56.7 (46.8)
+//         n = 4000, chain 2000: B = 512 66 (78), B = 1024 123 (99)
+//         n = 8000, chain 8000: B = 512 194 (225), B = 1024 366 (269)
+//         but n = 2000, chain 600, B = 8192 193 (216); n = 4000, chain 1150, B = 4096 202 (217)
+//         one workgroup per CU, n = 8000, m = 2500, chain 1500: B = 512 89 (102), B = 2048 343 (248)
+//   fp32  n = 600, chain 400: B = 4096 21.9 (28.6)
+//         chain 600, coefficients per sample: B = 2048 29.5 (32.3), B = 4096 51.4 (42.6)
+//         n = 4000, chain 2000: B = 1024 55 (79), B = 4096 189 (148)
+//         n = 8000, chain 8000: B = 1024 256 (223)
 int64_t gmr_batch(const purin_cp_plan* p, int64_t restart, bool dense) {
   if (!p->sl_ok || restart > kGmrRestart || !gmr_holds(p)) return 0;
   int cus = 0;
